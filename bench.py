@@ -50,6 +50,7 @@ def kernel_bytes(mesh, name, precision_bytes=8, ns=2):
     C, F, E = mesh.n_cells, mesh.n_faces, mesh.n_edges
     nc2f, nf2e, nec = 4 * C, 3 * F, int(mesh.array("ec_ptr")[-1])
     b = precision_bytes
+    rs = -(-(5 * ns + 6) // 8) * 8
     table = {
         # x (E) read, phi (F) write, f2e ptr+idx
         "d1": E * b + F * b + 4 * (F + 1) + 4 * nf2e,
@@ -62,14 +63,14 @@ def kernel_bytes(mesh, name, precision_bytes=8, ns=2):
                       + 2 * E * b + 8 * E + E + E * b,
         # one fused MGS step: w read + write, two basis vectors
         "mgs": 4 * E * b,
-        "prepare": ns * 5 * C * 8 * 2 + F * 8 + 3 * C * 8 * 5 + C * 8 + 4 * F * 8 + 4 * nc2f + 4 * (C + 1) + C * 8 + C,
-        "grad_current": ns * (5 * C * 8 + 15 * C * 8) + 3 * C * 8 * 2 + 6 * C * 8 + nc2f * (4 + 8 + 24) + 3 * F * 8 * 2 + 3 * C * 8
-                        + 8 * F + C * 8 + C + 4 * (C + 1),
-        "face": ns * (5 * C * 8 + 15 * C * 8) + 5 * ns * F * 8 + 3 * F * 8 + 3 * C * 8 * 3 + F * 8 * 2 + 3 * F * 8 * 2 + F * 8 + 8 * F
-                + 3 * C * 8 + F,
-        "cell_update": 5 * ns * F * 8 + ns * 5 * C * 8 * 3 + 3 * C * 8 * 2 + C * 8 + C + 4 * nc2f + 4 * (C + 1),
-        "edge_emf": 3 * F * 8 + 3 * C * 8 + F * 8 + 4 * (E + 1) + 4 * nf2e + 8 * nf2e + 4 * (E + 1) + 4 * nec + 3 * F * 8 * 2 + F * 8
-                    + 3 * E * 8 * 2 + E * 8 + E * 8 + E,
+        # the explicit stage (csrc/kernels/explicit_step.h): cell records of rs doubles, a state per ion at every (cell, face)
+        # entry, a flux per ion and a 32-byte EMF row at every face
+        "prepare": ns * 5 * C * 8 + rs * C * 8 + F * 8 + 3 * C * 8 * 4 + C * 8 * 2 + 4 * F * 8 + 4 * nc2f + C,
+        "states": rs * C * 8 + 3 * F * 8 * 2 + 6 * C * 8 + 12 * nc2f + C * 8 + C + 3 * C * 8 + 5 * ns * nc2f * 8
+                  + 4 * F * 8 * 2 + 8 * F + 2 * F * 8 + 6 * C * 8,
+        "fluxes": 5 * ns * nc2f * 8 + 4 * F * 8 + 8 * F + F + 5 * ns * F * 8
+                  + 4 * F * 8 * 2 + 3 * F * 8 + 3 * C * 8 + 8 * (E + 1) + 12 * nf2e + 4 * nec + 3 * E * 8 * 2 + E * 8 * 2 + E,
+        "update": 5 * ns * F * 8 + rs * C * 8 + ns * 5 * C * 8 * 2 + 3 * C * 8 * 2 + C * 8 + C + 4 * nc2f,
         "faraday": E * 8 + F * 8 * 2 + 4 * (F + 1) + 4 * nf2e + 8 * F,
         # FP32 operator of the mixed solve (int32 incidence, FP32 values)
         "d1_f32": 4 * (F + 1) + 4 * nf2e + 4 * E + 4 * E + E + 4 * F,
@@ -90,8 +91,7 @@ def kernel_bytes(mesh, name, precision_bytes=8, ns=2):
 
 
 KERNEL_CLASSES = {
-    "explicit": ("prepare", "dt_final", "grad_current", "face", "face_emf", "cell_update", "edge_emf", "edge_emf_heavy", "faraday",
-                 "gyrate"),
+    "explicit": ("prepare", "dt_final", "states", "fluxes", "update", "faraday", "gyrate"),
     "operator": ("d1", "bcell", "hall_g", "edge_apply", "edge_apply_heavy", "d1_f32", "bcell_f32", "hall_g_f32", "edge_apply_f32",
                  "mg_apply_f32"),
     "orthogonalisation": ("mgs", "finish", "dot", "multidot", "multidot_final", "multiaxpy", "scale", "multidot64", "multidot64_final",

@@ -1157,7 +1157,7 @@ void mhdg_ctx::vjp_alloc(int n_steps)
             aw.sF[s] = D(20 * K); aw.sG[s] = D(5 * K); aw.sFA[s] = D(5 * K);
         }
         aw.Phi = D(F); aw.Bind = D(3 * C); aw.Btot = D(3 * C); aw.up = D(3 * C); aw.J = D(3 * C); aw.alpha = D(C);
-        aw.FA = D(10 * F); aw.Ef = D(3 * F); aw.E = D(E); aw.dt_part = D(size_t(nbk(nc)) + 1); aw.dt_dev = D(1);
+        aw.FA = D(10 * F); aw.Ef = D(4 * F); aw.E = D(E); aw.dt_part = D(size_t(nbk(nc)) + 1); aw.dt_dev = D(1);
         aw.Phib = D(F); aw.PhiAddb = D(F); aw.Baddb = D(3 * C); aw.Eb = D(E); aw.Efb = D(3 * F); aw.FAb = D(10 * F);
         aw.upb = D(3 * C); aw.Btb = D(3 * C); aw.Bib = D(3 * C); aw.Jb = D(3 * C);
         aw.sE = D(9 * K); aw.sPhi = D(K);
@@ -1206,7 +1206,7 @@ double mhdg_ctx::vjp_stage(double dt_max, bool update)
     }
     LAUNCH("face", k_face<double>, dim3(nbk(nf)), dim3(256), 0, stream, d, P, 2, 0, Wc, Gc, none, aw.FA,
            static_cast<const double *>(aw.up), static_cast<const double *>(aw.Btot), static_cast<const double *>(aw.Bind),
-           static_cast<const double *>(aw.Phi), static_cast<const double *>(PhiAdd), aw.Ef);
+           static_cast<const double *>(aw.Phi), static_cast<const double *>(PhiAdd), static_cast<const double *>(aw.Phi), aw.Ef);
     double dt = 0;
     d2h(&dt, aw.dt_dev, 8);
     if (!std::isfinite(dt) || dt <= 0) throw std::runtime_error("invalid time step");
@@ -1214,7 +1214,7 @@ double mhdg_ctx::vjp_stage(double dt_max, bool update)
         LAUNCH("cell_update", k_cell_update<double>, dim3(nb), dim3(256), 0, stream, d, P, 2, 0, static_cast<const double *>(aw.FA), none, Wc,
                static_cast<const double *>(aw.Btot), static_cast<const double *>(aw.J), static_cast<const double *>(aw.dt_dev), 0.0, 1, 1,
                Uw, noneW);
-    launch_edge_emf(aw.Ef, aw.up, aw.Phi, P.cuct, nullptr, aw.E, 1);
+    launch_edge_emf(aw.Ef, aw.up, P.cuct, nullptr, aw.E, 1);
     if (update)
         LAUNCH("faraday", k_faraday<double>, dim3(nbk(nf)), dim3(256), 0, stream, d, static_cast<const double *>(aw.E),
                static_cast<const double *>(nullptr), static_cast<const double *>(aw.dt_dev), 0.0, aw.Phi);

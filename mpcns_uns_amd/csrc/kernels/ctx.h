@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "../../../include/mhdg.h"
+#include "explicit_step.h"
 #include "induction.h"
 #include "mixed.h"
 
@@ -21,7 +22,7 @@ struct mhdg_ctx
     mhdg_config cfg{};
     mhdg::Params P{};
     mhdg::DevMesh d{};
-    int32_t nc = 0, nf = 0, ne = 0, n_heavy = 0;
+    int32_t nc = 0, nf = 0, ne = 0, n_heavy = 0, max_valence = 0;
     size_t c2f_nnz = 0, ec_nnz = 0, e2f_nnz = 0;
     int32_t cdeg = 0, fdeg = 0; // uniform faces per cell / edges per face (0: mixed shapes)
     void *heavy = nullptr;
@@ -29,8 +30,9 @@ struct mhdg_ctx
     int8_t *dir_mercury = nullptr;
     // resident state and derived fields
     double *U[mhdg::kMaxSpecies]{}, *Phi = nullptr, *PhiAdd = nullptr, *Badd = nullptr;
-    double *W[mhdg::kMaxSpecies]{}, *grad[mhdg::kMaxSpecies]{}, *Bind = nullptr, *Btot = nullptr, *uplus = nullptr, *J = nullptr, *alpha = nullptr, *B0 = nullptr;
-    double *FA = nullptr, *Ef = nullptr, *E_expl = nullptr, *E_last = nullptr, *dt_part = nullptr, *dt_dev = nullptr;
+    double *Btot = nullptr, *uplus = nullptr, *J = nullptr, *alpha = nullptr, *B0 = nullptr;
+    mhdg::StepFields sf{}; // the explicit stage's layouts: primitives and field per cell, face states, fluxes, EMF candidates
+    double *E_expl = nullptr, *E_last = nullptr, *dt_part = nullptr, *dt_dev = nullptr;
     // implicit induction work
     double *phi_w = nullptr, *bcell = nullptr, *gcell = nullptr, *corr = nullptr;
     bool have_corr = false;
@@ -106,7 +108,14 @@ struct mhdg_ctx
     double *stage_in(int slot, const void *host, size_t n_doubles);
     void d2h(void *host, const void *dev, size_t bytes);
     void check_launch(const char *what);
-    void launch_edge_emf(const double *Ef, const double *u, const double *phi_ind, double cuct, const double *Ein, double *Eout, int bc);
+    void launch_edge_emf(const double *Ef, const double *u, double cuct, const double *Ein, double *Eout, int bc);
+    // explicit_step.hip
+    void step_build();
+    void launch_prepare();
+    void launch_states(int32_t n_face, double *dt_out, double dt_max); // n_face face-EMF blocks and (dt_out) the CFL minimum with them
+    // the explicit stage, with_ct: and the CT update with its EMF; the state is untouched when it throws
+    double explicit_stage(double dt_max, bool with_ct);
+    void get_record(int32_t first, int32_t n, double *host);
     double dot(const double *a, const double *b, int op, int slot);
     void apply_op(const double *phi, const double *v, const double *inv, const int8_t *dir, double dt, int mode, int mask, const double *b,
                   double *out);

@@ -195,6 +195,7 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     if (t.max_valence > kHeavyMax) throw std::runtime_error("edge valence exceeds the supported maximum");
     nc = t.nc; nf = t.nf; ne = t.ne;
     n_heavy = static_cast<int32_t>(t.heavy.size());
+    max_valence = t.max_valence;
     c2f_nnz = t.c2f.size();
     ec_nnz = t.ec_cell.size();
     e2f_nnz = t.e2f.size();
@@ -232,6 +233,12 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     d.evec = upload(m.edge_vec, 3 * E); d.emid = upload(m.edge_mid, 3 * E); d.elen = upload(m.edge_len, E);
     d.ecw = upload(m.ec_weight, size_t(m.ec_ptr[E])); d.efw = upload(m.ef_weight, t.e2f.size());
     d.star2 = upload(m.star2, F);
+    {
+        double *geo = static_cast<double *>(alloc(4 * F * sizeof(double)));
+        hipLaunchKernelGGL(k_face_geo, dim3(nblk(nf)), dim3(256), 0, stream, d, geo);
+        check_launch("face geometry");
+        d.geo = geo;
+    }
     d.snb = upload(t.snb); d.sw = upload(t.sw); d.sd = upload(t.sd); d.sinv = upload(t.sinv); d.svalid = upload(t.svalid);
     d.recon = upload(t.recon); d.m_e = upload(t.m_e); d.d2 = upload(t.d2); d.taper = upload(t.taper);
     heavy = upload(t.heavy);
@@ -272,13 +279,14 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     hip_check(hipMemset(Phi, 0, F * 8), "memset");
     for (int s = 0; s < P.ns; ++s)
     {
-        U[s] = D(5 * C); W[s] = D(5 * C); grad[s] = D(15 * C);
+        U[s] = D(5 * C);
         hip_check(hipMemset(U[s], 0, 5 * C * 8), "memset");
     }
-    Bind = D(3 * C); Btot = D(3 * C); uplus = D(3 * C); J = D(3 * C); alpha = D(C); B0 = D(3 * C);
+    Btot = D(3 * C); uplus = D(3 * C); J = D(3 * C); alpha = D(C); B0 = D(3 * C);
     hip_check(hipMemset(alpha, 0, C * 8), "memset"); hip_check(hipMemset(B0, 0, 3 * C * 8), "memset");
-    FA = D(5 * size_t(P.ns) * F); Ef = D(3 * F); E_expl = D(E); E_last = D(E);
-    dt_part = D(size_t(nblk(nc)) + 1); dt_dev = D(1);
+    step_build(); // the layouts of the explicit stage
+    E_expl = D(E); E_last = D(E);
+    dt_part = D(size_t(nblk(nc, 256 / P.ns)) + 1); dt_dev = D(1);
     // induction work
     phi_w = D(F); bcell = D(3 * C); gcell = D(3 * C); corr = D(E); have_corr = false;
     x0 = D(E); bvec = D(E); rvec = D(E); wvec = D(E); invdiag = D(E); delta = D(E); tmp = D(E);
@@ -298,13 +306,11 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
 }
 
 // ------------------------------------------------------------------------------------ pieces
-void mhdg_ctx::launch_edge_emf(const double *Efp, const double *u, const double *phi_ind, double cuct, const double *Ein, double *Eout,
-                               int bc)
+void mhdg_ctx::launch_edge_emf(const double *Efp, const double *u, double cuct, const double *Ein, double *Eout, int bc)
 {
-    LAUNCH("edge_emf", k_edge_emf<double>, dim3(nblk(ne)), dim3(256), 0, stream, d, P, Efp, u, phi_ind, cuct, kLightMax, Ein, Eout, bc);
-    if (n_heavy)
-        LAUNCH("edge_emf_heavy", k_edge_emf_heavy<double>, dim3(n_heavy), dim3(256), 0, stream, d, P, Efp, u, phi_ind, cuct,
-                           static_cast<const int32_t *>(heavy), Ein, Eout, bc);
+    const size_t lds = n_heavy ? 6 * size_t(max_valence) * sizeof(double) : 0;
+    LAUNCH("edge_emf", k_edge_emf<double>, dim3(n_heavy + nblk(ne)), dim3(256), lds, stream, d, P, Efp, u, cuct, kLightMax, Ein, Eout, bc,
+           static_cast<const int32_t *>(heavy), n_heavy, max_valence);
     check_launch("edge emf");
 }
 
@@ -340,8 +346,8 @@ void mhdg_ctx::apply_op(const double *phi_in, const double *v, const double *inv
         // add_ideal_emf of (u, b, phi) with b as total and induced field (ImplicitInduction.cpp:150-157)
         SpC none{};
         LAUNCH("face", k_face<double>, dim3(nblk(nf)), dim3(256), 0, stream, d, P, 0, 0, none, none, none, static_cast<double *>(nullptr), u_ideal,
-               bcell, bcell, phi, static_cast<const double *>(nullptr), Ef_i);
-        launch_edge_emf(Ef_i, u_ideal, phi, P.cuct, nullptr, ide, 0);
+               bcell, bcell, phi, static_cast<const double *>(nullptr), phi, Ef_i);
+        launch_edge_emf(Ef_i, u_ideal, P.cuct, nullptr, ide, 0);
     }
     const double *idp = ideal_part ? ide : nullptr;
     LAUNCH("edge_apply", k_edge_apply, dim3(nblk(ne)), dim3(256), 0, stream, d, int32_t(op_res), int32_t(op_hall), phi, gcell, idp,
@@ -463,94 +469,22 @@ double mhdg_ctx::step(double dt_max, int precision, int *iters, double *res)
     if (precision == 2 && mgh.n_nodes <= 0) throw std::runtime_error("multigrid preconditioner: the mesh descriptor carried no e2n incidence");
     if ((precision == 1 || precision == 2) && ideal_cfg && u_ideal)
         throw std::runtime_error("mixed-precision solve: the implicit ideal part has no FP32 operator; use precision 0");
-    const int nb = nblk(nc);
-    SpC Uc{}, Wc{};
-    SpW Ww{};
-    for (int s = 0; s < P.ns; ++s) { Uc.p[s] = U[s]; Wc.p[s] = W[s]; Ww.p[s] = W[s]; }
-    LAUNCH("prepare", k_prepare<double>, dim3(nb), dim3(256), 0, stream, d, P, Uc, static_cast<const double *>(Phi),
-           static_cast<const double *>(Badd), Ww, Bind, Btot, uplus, alpha,
-                       dt_part);
-    LAUNCH("dt_final", k_dt_final<double>, dim3(1), dim3(256), 0, stream, dt_part, nb, dt_max, dt_dev);
-    double *dth = static_cast<double *>(host_pin);
-    hip_check(hipMemcpyAsync(dth, dt_dev, 8, hipMemcpyDeviceToHost, stream), "D2H");
-    hipEvent_t ev;
-    hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
-    hip_check(hipEventRecord(ev, stream), "event");
-    // Strang split of the ions' gyration (Solver.cpp:237-241): half a step, then prepare again.  The rotation changes
-    // U, so the time step is checked first, as the reference throws before it touches the state (Solver.cpp:236).
-    const bool split = P.induce_coeff > 0 && P.lorentz;
-    if (split)
-    {
-        hip_check(hipEventSynchronize(ev), "event sync");
-        if (!std::isfinite(dth[0]) || dth[0] <= 0)
-        {
-            (void)hipEventDestroy(ev);
-            throw std::runtime_error("invalid time step");
-        }
-        LAUNCH("gyrate", k_gyrate, dim3(nb), dim3(256), 0, stream, d, P, U[0], U[1], static_cast<const double *>(Btot),
-               static_cast<const double *>(dt_dev), 0.5);
-        LAUNCH("prepare", k_prepare<double>, dim3(nb), dim3(256), 0, stream, d, P, Uc, static_cast<const double *>(Phi),
-               static_cast<const double *>(Badd), Ww, Bind, Btot, uplus, alpha, dt_part);
-    }
-    SpC Ws{}, none{}, gradsC{};
-    SpW grads{}, Us{}, noneW{};
-    for (int s = 0; s < P.ns; ++s)
-    {
-        Ws.p[s] = W[s];
-        grads.p[s] = grad[s];
-        gradsC.p[s] = grad[s];
-        Us.p[s] = U[s];
-    }
-    if (P.second_order)
-    {
-        // many species: the stencil rows loaded once for all of them
-        auto kgrad = P.ns > 2 ? k_grad_current<double, true> : k_grad_current<double, false>;
-        LAUNCH("grad_current", kgrad, dim3(nb), dim3(256), 0, stream, d, P, P.ns, 0, Ws, none, grads, 1, Bind, J);
-    }
-    else
-    {
-        for (int s = 0; s < P.ns; ++s) hip_check(hipMemsetAsync(grad[s], 0, 15 * size_t(nc) * 8, stream), "memset");
-        LAUNCH("grad_current", k_grad_current<double>, dim3(nb), dim3(256), 0, stream, d, P, 0, 0, Ws, none, grads, 1, Bind, J);
-    }
-    if (P.ns > 2)
-    {
-        // many species (for two, one thread per face with LDS-staged rows measured faster: 2.03 against 2.28 ms at 8M): one thread per (face, species) for the fluxes, then the face EMF candidates alone
-        const int per = 256 / P.ns;
-        LAUNCH("face", k_face_species<double>, dim3(nblk(nf, per)), dim3(256), 0, stream, d, P, P.ns, Ws, gradsC, FA);
-        LAUNCH("face_emf", k_face<double>, dim3(nblk(nf)), dim3(256), 0, stream, d, P, 0, 0, Ws, gradsC, none, static_cast<double *>(nullptr),
-               uplus, Btot, Bind, Phi, PhiAdd, Ef);
-    }
-    else
-        LAUNCH("face", k_face<double>, dim3(nblk(nf)), dim3(256), 0, stream, d, P, P.ns, 0, Ws, gradsC, none, FA, uplus, Btot, Bind, Phi, PhiAdd, Ef);
-    check_launch("explicit stage");
-    hip_check(hipEventSynchronize(ev), "event sync");
-    (void)hipEventDestroy(ev);
-    const double gdt = dth[0];
-    // nothing above wrote U or Phi (only derived fields), so the state is unchanged when this throws
-    if (!std::isfinite(gdt) || gdt <= 0) throw std::runtime_error("invalid time step");
-    if (P.ns > 2)
-        LAUNCH("cell_update", k_cell_update_many<double>, dim3(nb), dim3(256), 0, stream, d, P, P.ns, static_cast<const double *>(FA), Wc,
-               static_cast<const double *>(Btot), static_cast<const double *>(J), static_cast<const double *>(dt_dev), Us);
-    else
-        LAUNCH("cell_update", k_cell_update<double>, dim3(nb), dim3(256), 0, stream, d, P, P.ns, 0, static_cast<const double *>(FA), none, Wc,
-               static_cast<const double *>(Btot), static_cast<const double *>(J), static_cast<const double *>(dt_dev), 0.0, 1, 1, Us, noneW);
-    launch_edge_emf(Ef, uplus, Phi, P.cuct, nullptr, E_expl, 1);
+    const bool implicit = (op_hall || op_res || ideal_cfg) && !skip_implicit; // ImplicitInduction::active()
+    const double gdt = explicit_stage(dt_max, !implicit);
     *iters = 0;
     *res = 0.0;
-    const double *Euse = E_expl;
-    if ((op_hall || op_res || ideal_cfg) && !skip_implicit) // ImplicitInduction::active()
+    if (implicit)
     {
         hip_check(hipMemcpyAsync(B0, Btot, 3 * size_t(nc) * 8, hipMemcpyDeviceToDevice, stream), "copy");
         if (precision == 0) *iters = solve64(Phi, E_expl, dir_mercury, gdt, E_last, res);
         else if (precision == 3) *iters = solve64_cgs(Phi, E_expl, dir_mercury, gdt, E_last, res);
         else *iters = solve_mixed(Phi, E_expl, dir_mercury, gdt, E_last, res, precision == 2, dir_mercury_h.data());
-        Euse = E_last;
+        LAUNCH("faraday", k_faraday<double>, dim3(nblk(nf)), dim3(256), 0, stream, d, E_last, nullptr, dt_dev, 0.0, Phi);
     }
     else
-        hip_check(hipMemcpyAsync(E_last, E_expl, size_t(ne) * 8, hipMemcpyDeviceToDevice, stream), "copy");
-    LAUNCH("faraday", k_faraday<double>, dim3(nblk(nf)), dim3(256), 0, stream, d, Euse, nullptr, dt_dev, 0.0, Phi);
-    if (split) // the second half of the gyration, with the field of the step's prepare (Solver.cpp:272)
-        LAUNCH("gyrate", k_gyrate, dim3(nb), dim3(256), 0, stream, d, P, U[0], U[1], static_cast<const double *>(Btot),
+        std::swap(E_last, E_expl); // the explicit EMF is the step's
+    if (P.induce_coeff > 0 && P.lorentz) // the second half of the gyration, with the field of the step's prepare (Solver.cpp:272)
+        LAUNCH("gyrate", k_gyrate, dim3(nblk(nc)), dim3(256), 0, stream, d, P, U[0], U[1], static_cast<const double *>(Btot),
                static_cast<const double *>(dt_dev), 0.5);
     check_launch("faraday");
     if (prof_on) prof_flush();
@@ -702,7 +636,8 @@ int mhdg_flux_rhs(mhdg_ctx *c, int species, const double fs[5], const double *W,
         ro.p[0] = c->stage(4, 5 * size_t(c->nc));
         hipLaunchKernelGGL(k_face<double>, dim3(nblk(c->nf)), dim3(256), 0, c->stream, c->d, P, 1, species, Ws, Gs, gh, fa,
                            static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), static_cast<const double *>(nullptr),
-                           static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), static_cast<double *>(nullptr));
+                           static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), static_cast<const double *>(nullptr),
+                           static_cast<double *>(nullptr));
         hipLaunchKernelGGL(k_cell_update<double>, dim3(nblk(c->nc)), dim3(256), 0, c->stream, c->d, P, 1, species, static_cast<const double *>(fa),
                            none, none, static_cast<const double *>(nullptr), static_cast<const double *>(nullptr),
                            static_cast<const double *>(nullptr), 0.0, 0, 0, nw, ro);
@@ -717,11 +652,11 @@ int mhdg_ideal_emf(mhdg_ctx *c, const double *u, const double *Bt, const double 
         const double *du = c->stage_in(0, u, C3), *dbt = c->stage_in(1, Bt, C3), *dbi = c->stage_in(2, Bi, C3);
         const double *dpt = c->stage_in(3, pt, c->nf), *dpi = c->stage_in(4, pi, c->nf);
         double *dE = c->stage_in(5, E, c->ne);
-        double *ef = c->stage(6, 3 * size_t(c->nf));
+        double *ef = c->stage(6, 4 * size_t(c->nf));
         SpC none{};
         hipLaunchKernelGGL(k_face<double>, dim3(nblk(c->nf)), dim3(256), 0, c->stream, c->d, c->P, 0, 0, none, none, none,
-                           static_cast<double *>(nullptr), du, dbt, dbi, dpt, static_cast<const double *>(nullptr), ef);
-        c->launch_edge_emf(ef, du, dpi, cuct, dE, dE, 0);
+                           static_cast<double *>(nullptr), du, dbt, dbi, dpt, static_cast<const double *>(nullptr), dpi, ef);
+        c->launch_edge_emf(ef, du, cuct, dE, dE, 0);
         c->d2h(E, dE, size_t(c->ne) * 8);
     })
 }
@@ -848,7 +783,7 @@ int mhdg_ind_set_ideal_state(mhdg_ctx *c, const double *u, const int8_t *mask)
         {
             c->u_ideal = static_cast<double *>(c->alloc(3 * size_t(c->nc) * 8));
             c->ide = static_cast<double *>(c->alloc(size_t(c->ne) * 8));
-            c->Ef_i = static_cast<double *>(c->alloc(3 * size_t(c->nf) * 8));
+            c->Ef_i = static_cast<double *>(c->alloc(4 * size_t(c->nf) * 8));
             c->imask = static_cast<int8_t *>(c->alloc(size_t(c->ne)));
         }
         hip_check(hipMemcpyAsync(c->u_ideal, u, 3 * size_t(c->nc) * 8, hipMemcpyHostToDevice, c->stream), "H2D");
@@ -1033,8 +968,7 @@ int mhdg_get_species_prim(mhdg_ctx *c, int species, double *W)
 {
     MHDG_TRY(c, {
         if (species < 0 || species >= c->P.ns) throw std::runtime_error("species out of range for this context's n_species");
-        hip_check(hipStreamSynchronize(c->stream), "sync");
-        hip_check(hipMemcpy(W, c->W[species], 5 * size_t(c->nc) * 8, hipMemcpyDeviceToHost), "D2H");
+        c->get_record(5 * species, 5, W);
     })
 }
 int mhdg_set_background(mhdg_ctx *c, const double *PA, const double *BA)
@@ -1104,14 +1038,8 @@ int mhdg_state_restore(mhdg_ctx *c)
 int mhdg_prepare(mhdg_ctx *c)
 {
     MHDG_TRY(c, {
-        const int nb = nblk(c->nc);
-        SpC Uc{}, none{};
-        SpW Ww{}, noneW{};
-        for (int s = 0; s < c->P.ns; ++s) { Uc.p[s] = c->U[s]; Ww.p[s] = c->W[s]; }
-        hipLaunchKernelGGL(k_prepare<double>, dim3(nb), dim3(256), 0, c->stream, c->d, c->P, Uc, static_cast<const double *>(c->Phi),
-                           static_cast<const double *>(c->Badd), Ww, c->Bind, c->Btot, c->uplus, c->alpha, c->dt_part);
-        hipLaunchKernelGGL(k_grad_current<double>, dim3(nb), dim3(256), 0, c->stream, c->d, c->P, 0, 0, none, none, noneW, 1,
-                           static_cast<const double *>(c->Bind), c->J);
+        c->launch_prepare();
+        c->launch_states(0, nullptr, 0);
         c->check_launch("prepare");
         hip_check(hipStreamSynchronize(c->stream), "sync");
     })
@@ -1124,9 +1052,9 @@ int mhdg_get_derived(mhdg_ctx *c, int which, double *out)
         size_t n = 0;
         switch (which)
         {
-        case 0: src = c->W[0]; n = 5 * C; break;
-        case 1: src = c->W[1]; n = 5 * C; break;
-        case 2: src = c->Bind; n = 3 * C; break;
+        case 0: c->get_record(0, 5, out); return 0;
+        case 1: c->get_record(5, 5, out); return 0;
+        case 2: c->get_record(5 * c->P.ns, 3, out); return 0;
         case 3: src = c->Btot; n = 3 * C; break;
         case 4: src = c->J; n = 3 * C; break;
         case 5: src = c->uplus; n = 3 * C; break;

@@ -38,6 +38,7 @@ struct DevMesh
     const int32_t *ec_ptr, *ec_cell;
     const int8_t *mat, *kind, *emode;
     const double *farea, *fcen, *famag, *ccen, *cvol, *evec, *emid, *elen, *ecw, *efw, *star2;
+    const double *geo;              // 4 per face: unit normal, |A| (32-byte rows for the gathers)
     // Stencil (reference Reconstruction.h:34-41), aligned with c2f entries
     const int32_t *snb;             // neighbour cell, -(f+1) virtual, kNoStencil for a Skip face
     const double *sw, *sd, *sinv;   // weight, offset (3), symmetric inverse (6 per cell: 0 1 2 4 5 8)

@@ -93,34 +93,6 @@ template <class R> __global__ void __launch_bounds__(256) k_dt_final(const R *pa
     if (threadIdx.x == 0) out[0] = mn(v, dt_max);
 }
 
-// Stencil neighbour state of a boundary entry (nb < 0, face f = -(nb + 1), c2f entry v): the ghost table row, or
-// ghost_state (Common/fluid/Reconstruction.cpp:9-24) with the cell value wc inside.
-template <class R>
-__device__ __forceinline__ void stencil_ghost(const DevMesh &d, int32_t sp, const R *gh, const R *wc, const R *fs, int32_t v, int32_t nb,
-                                              R *wn)
-{
-    const int32_t f = -(nb + 1);
-    if (gh)
-    {
-        for (int m = 0; m < 5; ++m) wn[m] = gh[5 * size_t(f) + m];
-        return;
-    }
-    const int8_t kind = d.kind[f];
-    for (int m = 0; m < 5; ++m) wn[m] = wc[m];
-    if (kind == kWall)
-    {
-        if (sp == 1) { wn[0] = 1e-12; wn[1] = 0; wn[2] = 0; wn[3] = 0; wn[4] = 1e-12; }
-        else
-        {
-            const V3T<R> n = (psg(v) / d.famag[f]) * L3(d.farea, f);
-            const R un = wc[1] * n.x + wc[2] * n.y + wc[3] * n.z;
-            wn[1] -= 2 * un * n.x; wn[2] -= 2 * un * n.y; wn[3] -= 2 * un * n.z;
-        }
-    }
-    else if (kind == kInflow)
-        for (int m = 0; m < 5; ++m) wn[m] = fs[m];
-}
-
 // Stencil::limited_gradients (Common/fluid/Reconstruction.cpp:80-142) for `ns` species and cell_current
 // (Common/induction/Current.cpp:9-31, by the blocks of grid row 0).  ghost: optional per-face table of 5
 // primitives per species.
@@ -129,7 +101,7 @@ __device__ __forceinline__ void stencil_ghost(const DevMesh &d, int32_t sp, cons
 // Cells of at most kGradFast faces load their face and stencil rows once, together, before the gathers, and
 // the limiter's face offsets once for every species; the operations and their order are those of the general
 // path.
-template <class R, bool HOIST> __global__ void __launch_bounds__(256, 3) k_grad_current(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<R> Ws, SpCT<R> ghosts, SpWT<R> grads,
+template <class R> __global__ void __launch_bounds__(256, 3) k_grad_current(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<R> Ws, SpCT<R> ghosts, SpWT<R> grads,
                                                       int32_t limit, const R *Bind, R *J)
 {
     __shared__ R stage[256 * 15];
@@ -191,14 +163,6 @@ template <class R, bool HOIST> __global__ void __launch_bounds__(256, 3) k_grad_
 #pragma unroll
         for (int i = 0; i < kGradFast; ++i)
             if (i < nk) dxk[i] = L3(d.fcen, pid(vk[i])) - xc;
-    // HOIST (many species): the stencil rows too are loaded once for every species
-    int32_t nbh[kGradFast];
-    double swh[kGradFast];
-    V3 sdh[kGradFast];
-    if (HOIST && fast)
-#pragma unroll
-        for (int i = 0; i < kGradFast; ++i)
-            if (i < nk) { nbh[i] = d.snb[k0 + i]; swh[i] = d.sw[k0 + i]; sdh[i] = L3(d.sd, k0 + i); }
     // species s of the block: blockIdx.y, blockIdx.y + gridDim.y, ... (one grid row, every species, measured
     // faster than one row per species)
     for (int32_t s = int32_t(blockIdx.y); s < ns; s += int32_t(gridDim.y))
@@ -216,8 +180,8 @@ template <class R, bool HOIST> __global__ void __launch_bounds__(256, 3) k_grad_
         R wc[5], r[5][3], lo[5], hi[5];
         for (int m = 0; m < 5; ++m) { wc[m] = W[5 * size_t(c) + m]; lo[m] = hi[m] = wc[m]; r[m][0] = r[m][1] = r[m][2] = 0.0; }
         auto accumulate = [&](int32_t k, const R *wn) {
-            const R w = HOIST && fast ? R(swh[k - k0]) : R(d.sw[k]);
-            const V3T<R> dd = HOIST && fast ? V3T<R>(sdh[k - k0]) : V3T<R>(L3(d.sd, k));
+            const R w = d.sw[k];
+            const V3T<R> dd = L3(d.sd, k);
             for (int m = 0; m < 5; ++m)
             {
                 const R dq = wn[m] - wc[m];
@@ -231,7 +195,7 @@ template <class R, bool HOIST> __global__ void __launch_bounds__(256, 3) k_grad_
             int32_t nbk[kGradFast];
 #pragma unroll
             for (int i = 0; i < kGradFast; ++i)
-                if (i < nk) nbk[i] = HOIST ? nbh[i] : d.snb[k0 + i];
+                if (i < nk) nbk[i] = d.snb[k0 + i];
 #pragma unroll
             for (int i = 0; i < kGradFast; ++i)
                 if (i < nk && nbk[i] != kNoStencil)
@@ -403,36 +367,13 @@ __device__ __forceinline__ void face_species_flux(const DevMesh &d, const Params
 }
 } // namespace
 
-// Face fluxes of many species, one thread per (face, species) with the species fastest: a block's threads
-// write its faces' 5*ns flux values as one contiguous range (FA layout of k_face).  The face EMF candidate
-// is left to k_face.
-template <class R> __global__ void __launch_bounds__(256) k_face_species(DevMesh d, Params P, int32_t ns, SpCT<R> Ws, SpCT<R> grads, R *FA)
-{
-    const int32_t per = int32_t(blockDim.x) / ns;
-    const int32_t t = int32_t(threadIdx.x);
-    const int32_t f = int32_t(blockIdx.x) * per + t / ns, s = t % ns;
-    if (t >= per * ns || f >= d.nf) return;
-    const int32_t l = d.fL[f], r = d.fR[f];
-    const int8_t kind = d.kind[f];
-    const bool any = (l >= 0 && d.mat[l] == 0) || (r >= 0 && d.mat[r] == 0);
-    R *out = FA + size_t(5 * ns) * f + 5 * s;
-    if (kind == kSkip || !any)
-    {
-        for (int m = 0; m < 5; ++m) out[m] = 0.0;
-        return;
-    }
-    const R A = d.famag[f];
-    const V3T<R> n = (1.0 / A) * L3(d.farea, f);
-    SpCT<R> none{};
-    face_species_flux(d, P, f, l, r, kind, A, n, s, s, Ws, grads, none, out);
-}
-
 // Face kernel: fluid_flux_rhs's face body (Common/fluid/FluxRHS.cpp:36-73) for `ns` species, storing
 // F*|A| per face and species (FA, 5*ns per face, zero for skipped faces), and optionally the ideal EMF
-// face candidate E_f (Common/induction/IdealEMF.cpp:32-55, 3 per face).
+// face candidate E_f (Common/induction/IdealEMF.cpp:32-55) with phi_ind / |A|: four values per face, what the edge sum
+// reads of it.
 template <class R> __global__ void __launch_bounds__(256) k_face(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<R> Ws, SpCT<R> grads, SpCT<R> ghosts, R *FA,
                                               const R *uplus, const R *Btot, const R *Bind, const R *Phi,
-                                              const R *PhiAdd, R *Ef)
+                                              const R *PhiAdd, const R *phi_ind, R *Ef)
 {
     // up to two species the block's flux rows are staged in LDS and written as one contiguous range
     __shared__ R stage[256 * 10];
@@ -461,7 +402,9 @@ template <class R> __global__ void __launch_bounds__(256) k_face(DevMesh d, Para
             const V3T<R> u = L3(uplus, c);
             F = dot(u, n) * L3(Btot, c) - Bn_tot * u;
         }
-        st3(Ef, f, -1.0 * cross(n, F));
+        const V3T<R> E = -1.0 * cross(n, F);
+        R *out = Ef + 4 * size_t(f);
+        out[0] = E.x; out[1] = E.y; out[2] = E.z; out[3] = phi_ind[f] / A;
     }
     if (FA && act)
     {
@@ -578,344 +521,25 @@ template <class R> __global__ void __launch_bounds__(256) k_cell_update(DevMesh 
 }
 
 
-// k_cell_update of the fused step for more than two ions (rhs_in, rhs_out none, s0 = 0, sources and update on):
-// every species' flux sum is gathered in one pass over the cell's faces, so each face row (5 ns values) is read
-// once; with one pass per species the rows' lines were fetched again for every species (3x the algorithmic bytes
-// for ten ions).  Each species' sum runs over the faces in the same ascending order, so the results are those of
-// k_cell_update bit for bit.
-template <class R> __global__ void __launch_bounds__(256) k_cell_update_many(DevMesh d, Params P, int32_t ns, const R *FA, SpCT<R> Wall,
-                                                                            const R *Btot, const R *J, const R *dt_dev, SpWT<R> Us)
+// add_ideal_emf edge loop (Common/induction/IdealEMF.cpp:59-128).  The first n_heavy blocks take one high-valence edge
+// each (they last longest: 30 to 70 us alone behind this kernel before), the others one edge per thread with valence at
+// most `vmax`.  E_out[e] = E_in[e] + E_ideal (E_in nullable = 0); apply_bc additionally applies the boundary EMF of
+// Solver::rhs.  Dynamic LDS: six rows of hv values when there are heavy edges.
+template <class R> __global__ void __launch_bounds__(256) k_edge_emf(DevMesh d, Params P, const R *Ef, const R *u_cell, double cuct,
+                                                  int32_t vmax, const R *E_in, R *E_out, int32_t apply_bc, const int32_t *heavy,
+                                                  int32_t n_heavy, int32_t hv)
 {
-    const int32_t c = gid();
-    if (c >= d.nc) return;
-    const bool fluid = d.mat[c] == 0;
-    const R dt = dt_dev[0];
-    const R V = d.cvol[c];
-    const R ne_c = fluid ? electron_density(P, Wall.p, c) : R(0.0);
-    R rhs[kMaxSpecies][5];
-#pragma unroll
-    for (int s = 0; s < kMaxSpecies; ++s)
-        for (int m = 0; m < 5; ++m) rhs[s][m] = 0;
-    if (fluid)
-        for (int32_t k = d.c2f_ptr[c]; k < d.c2f_ptr[c + 1]; ++k)
-        {
-            const int32_t v = d.cfs[k];
-            const R *fa = FA + size_t(5 * ns) * pid(v);
-#pragma unroll
-            for (int s = 0; s < kMaxSpecies; ++s)
-                if (s < ns)
-                {
-                    if (v >= 0) for (int m = 0; m < 5; ++m) rhs[s][m] -= fa[5 * s + m] / V;
-                    else for (int m = 0; m < 5; ++m) rhs[s][m] += fa[5 * s + m] / V;
-                }
-        }
-#pragma unroll
-    for (int s = 0; s < kMaxSpecies; ++s)
-        if (s < ns && fluid)
-        {
-            R *r = rhs[s];
-            // mercury::add_sources for ion s (MercurySources.cpp:20-63), as in k_cell_update
-            const R *W = Wall.p[s];
-            const R ws = ion_density(P, s, W[5 * size_t(c)]) / sqrt(ne_c * ne_c + P.ne_floor * P.ne_floor);
-            const R rho = mx(W[5 * size_t(c)], 0.0);
-            const V3T<R> u(W[5 * size_t(c) + 1], W[5 * size_t(c) + 2], W[5 * size_t(c) + 3]);
-            V3T<R> S;
-            if (P.lorentz) S += (P.inver_MA2 * ws) * cross(L3(J, c), L3(Btot, c));
-            r[1] += S.x; r[2] += S.y; r[3] += S.z;
-            r[4] += dot(u, S) + (rho > 1e-30 ? 0.5 * dt * dot(S, S) / rho : 0.0);
-            if (P.src_rate[s] != 0.0 && d.atm)
-            {
-                const double q = P.src_rate[s] * d.atm[c];
-                r[0] += q;
-                r[4] += q * P.src_T / (P.gamma - 1.0);
-            }
-            // forward Euler with floors (Solver.cpp:246-252, 171-191), as in k_cell_update
-            R *u0 = Us.p[s] + 5 * size_t(c);
-            R q[5];
-            for (int m = 0; m < 5; ++m) q[m] = u0[m] + dt * r[m];
-            const R ke = q[0] > 0 ? 0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0] : 0.0;
-            if (!(q[0] >= P.rho_floor)) to_cons(PrimT<R>{P.rho_floor, 0, 0, 0, P.p_floor}, P.gamma, q);
-            else if ((P.gamma - 1.0) * (q[4] - ke) < P.p_floor)
-            {
-                const PrimT<R> w = to_prim(q, P.gamma, P.rho_floor, P.p_floor);
-                to_cons(w, P.gamma, q);
-            }
-            for (int m = 0; m < 5; ++m) u0[m] = q[m];
-        }
-}
-template __global__ void k_cell_update_many<double>(DevMesh d, Params P, int32_t ns, const double *FA, SpCT<double> Wall, const double *Btot,
-                                                    const double *J, const double *dt_dev, SpWT<double> Us);
-
-// add_ideal_emf edge loop (Common/induction/IdealEMF.cpp:59-128), one thread per edge with valence at most
-// `vmax`; larger edges are left to k_edge_emf_heavy.  E_out[e] = E_in[e] + E_ideal (E_in nullable = 0);
-// apply_bc additionally applies the boundary EMF of Solver::rhs.
-template <class R> __global__ void __launch_bounds__(256) k_edge_emf(DevMesh d, Params P, const R *Ef, const R *u_cell, const R *phi_ind,
-                                                  double cuct, int32_t vmax, const R *E_in, R *E_out, int32_t apply_bc)
-{
-    const int32_t e = gid();
-    if (e >= d.ne) return;
-    const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1];
-    const int32_t nf = f1 - f0;
-    if (nf > vmax) return;
-    R out = E_in ? E_in[e] : 0.0;
-    const int32_t c0 = d.ec_ptr[e], c1 = d.ec_ptr[e + 1];
-    const int32_t nc = c1 - c0;
-    const bool fast = nf <= kEmfFast && nc <= kEmfFast;
-    // common valence: the row indices are loaded once, together, before their gathers
-    int32_t fid[kEmfFast], cid[kEmfFast];
-    bool any_fluid = false;
-    if (fast)
-    {
-#pragma unroll
-        for (int i = 0; i < kEmfFast; ++i)
-        {
-            if (i < nf) fid[i] = pid(d.e2f[f0 + i]);
-            if (i < nc) cid[i] = d.ec_cell[c0 + i];
-        }
-#pragma unroll
-        for (int k = 0; k < kEmfFast; ++k)
-            if (k < nc) any_fluid |= d.mat[cid[k]] == 0;
-    }
-    else
-        for (int32_t k = c0; k < c1 && !any_fluid; ++k) any_fluid = d.mat[d.ec_cell[k]] == 0;
-    if (nf > 0 && d.elen[e] > 0 && any_fluid)
-    {
-        const V3 t = L3(d.evec, e);
-        const double L = d.elen[e];
-        const V3 th = (1.0 / L) * t;
-        R Ec = 0;
-        if (fast)
-        {
-            V3T<R> ef[kEmfFast];
-#pragma unroll
-            for (int i = 0; i < kEmfFast; ++i)
-                if (i < nf) ef[i] = L3(Ef, fid[i]);
-#pragma unroll
-            for (int i = 0; i < kEmfFast; ++i)
-                if (i < nf) Ec += d.efw[f0 + i] * dot(ef[i], t);
-        }
-        else
-            for (int32_t i = f0; i < f1; ++i) Ec += d.efw[i] * dot(L3(Ef, pid(d.e2f[i])), t);
-        V3 e1, e2;
-        plane_basis(th, e1, e2);
-        R M11 = 0, M12 = 0, M22 = 0, g1 = 0, g2 = 0, Eu = 0;
-        if (fast)
-        {
-            // the edge's cell velocities and the per-face terms stay in registers, so the second pass re-reads
-            // nothing (same operations in the same order as the general path)
-            V3T<R> uc[kEmfFast];
-#pragma unroll
-            for (int k = 0; k < kEmfFast; ++k)
-                if (k < nc) uc[k] = L3(u_cell, cid[k]);
-            R fqa[kEmfFast], fqb[kEmfFast], faef[kEmfFast], fsig[kEmfFast];
-#pragma unroll
-            for (int i = 0; i < kEmfFast; ++i)
-                if (i < nf)
-                {
-                    const int32_t f = fid[i];
-                    V3 m, nrm;
-                    face_dirs(d, f, e, th, m, nrm);
-                    R aef = 0.0;
-#pragma unroll
-                    for (int k = 0; k < kEmfFast; ++k)
-                        if (k < nc) aef = mx(aef, fabs(dot(uc[k], m)));
-                    const R sig = dot(th, cross(m, nrm));
-                    const V3T<R> qv = (aef * sig) * nrm;
-                    const R qa = dot(qv, e1), qb = dot(qv, e2), w = d.efw[f0 + i];
-                    M11 += w * qa * qa;
-                    M12 += w * qa * qb;
-                    M22 += w * qb * qb;
-                    g1 += w * qa;
-                    g2 += w * qb;
-                    fqa[i] = qa; fqb[i] = qb; faef[i] = aef; fsig[i] = sig;
-                }
-            R l1, l2;
-            uct_solve(M11, M12, M22, g1, g2, l1, l2);
-            // the face weight and flux are loaded again (cache hits) rather than held across the solve
-#pragma unroll
-            for (int i = 0; i < kEmfFast; ++i)
-                if (i < nf)
-                {
-                    const R omega = d.efw[f0 + i] * (1.0 - (fqa[i] * l1 + fqb[i] * l2));
-                    Eu += omega * faef[i] * fsig[i] * (phi_ind[fid[i]] / d.famag[fid[i]]);
-                }
-        }
-        else
-        {
-            for (int32_t i = f0; i < f1; ++i)
-            {
-                const int32_t f = pid(d.e2f[i]);
-                V3 m, nrm;
-                face_dirs(d, f, e, th, m, nrm);
-                const R aef = edge_amax(d, u_cell, c0, c1, m);
-                const V3T<R> qv = (aef * dot(th, cross(m, nrm))) * nrm;
-                const R qa = dot(qv, e1), qb = dot(qv, e2), w = d.efw[i];
-                M11 += w * qa * qa;
-                M12 += w * qa * qb;
-                M22 += w * qb * qb;
-                g1 += w * qa;
-                g2 += w * qb;
-            }
-            R l1, l2;
-            uct_solve(M11, M12, M22, g1, g2, l1, l2);
-            for (int32_t i = f0; i < f1; ++i)
-            {
-                const int32_t f = pid(d.e2f[i]);
-                V3 m, nrm;
-                face_dirs(d, f, e, th, m, nrm);
-                const R aef = edge_amax(d, u_cell, c0, c1, m);
-                const V3T<R> qv = (aef * dot(th, cross(m, nrm))) * nrm;
-                const R qa = dot(qv, e1), qb = dot(qv, e2), w = d.efw[i];
-                const R omega = w * (1.0 - (qa * l1 + qb * l2));
-                const R sig = dot(th, cross(m, nrm));
-                Eu += omega * aef * sig * (phi_ind[f] / d.famag[f]);
-            }
-        }
-        out += Ec + 2.0 * cuct * L * Eu;
-    }
-    E_out[e] = apply_bc ? edge_bc(d, P, e, out) : out;
-}
-
-// The same for one high-valence edge per block (pole axes of a lat-lon net): per-face terms in parallel,
-// every sum sequential in the reference's order.
-template <class R> __global__ void __launch_bounds__(256) k_edge_emf_heavy(DevMesh d, Params P, const R *Ef, const R *u_cell,
-                                                        const R *phi_ind, double cuct, const int32_t *heavy,
-                                                        const R *E_in, R *E_out, int32_t apply_bc)
-{
-    constexpr int kHS = kHeavyShared<R>();
-    __shared__ R s_w[kHS], s_ec[kHS], s_qa[kHS], s_qb[kHS], s_sig[kHS], s_aef[kHS];
-    __shared__ R s_l[2];
-    const int32_t e = heavy[blockIdx.x];
-    const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1], nf = f1 - f0;
-    const int32_t c0 = d.ec_ptr[e], c1 = d.ec_ptr[e + 1];
-    bool any_fluid = false;
-    for (int32_t k = c0; k < c1 && !any_fluid; ++k) any_fluid = d.mat[d.ec_cell[k]] == 0;
-    const bool active = nf > 0 && d.elen[e] > 0 && any_fluid;
-    const V3 t = L3(d.evec, e);
-    const double L = d.elen[e];
-    const V3 th = (1.0 / L) * t;
-    V3 e1, e2;
-    plane_basis(th, e1, e2);
-    // The edge's cell velocities are staged in LDS (in s_qa, s_qb, s_sig, before those take the per-face terms):
-    // every face's max over the cells then reads LDS, where a dependent global gather per (face, cell) pair made
-    // this kernel latency-bound (n_lon^2 pairs per pole-axis edge).  Same values, same order.
-    const int32_t nc = c1 - c0;
-    const bool staged = active && nc <= kHS;
-    if (staged)
-        for (int32_t k = threadIdx.x; k < nc; k += blockDim.x)
-        {
-            const V3T<R> u = L3(u_cell, d.ec_cell[c0 + k]);
-            s_qa[k] = u.x; s_qb[k] = u.y; s_sig[k] = u.z;
-        }
-    __syncthreads();
-    constexpr int kPer = (kHS + 255) / 256; // faces per thread (nf <= kHS, 256 threads)
-    R qa_r[kPer], qb_r[kPer], sig_r[kPer];
-    if (active)
-#pragma unroll
-        for (int j = 0; j < kPer; ++j)
-        {
-            const int32_t i = int32_t(threadIdx.x) + j * int32_t(blockDim.x);
-            if (i >= nf) break;
-            const int32_t f = pid(d.e2f[f0 + i]);
-            s_w[i] = d.efw[f0 + i];
-            s_ec[i] = dot(L3(Ef, f), t);
-            V3 m, nrm;
-            face_dirs(d, f, e, th, m, nrm);
-            R aef = 0.0;
-            if (staged)
-                for (int32_t k = 0; k < nc; ++k) aef = mx(aef, fabs(dot(V3T<R>(s_qa[k], s_qb[k], s_sig[k]), m)));
-            else
-                aef = edge_amax(d, u_cell, c0, c1, m);
-            const R sig = dot(th, cross(m, nrm));
-            const V3T<R> qv = (aef * sig) * nrm;
-            qa_r[j] = dot(qv, e1);
-            qb_r[j] = dot(qv, e2);
-            sig_r[j] = sig;
-            s_aef[i] = aef;
-        }
-    __syncthreads(); // every read of the staged velocities is done
-    if (active)
-#pragma unroll
-        for (int j = 0; j < kPer; ++j)
-        {
-            const int32_t i = int32_t(threadIdx.x) + j * int32_t(blockDim.x);
-            if (i >= nf) break;
-            s_qa[i] = qa_r[j]; s_qb[i] = qb_r[j]; s_sig[i] = sig_r[j];
-        }
-    __syncthreads();
-    R Ec = 0;
-    if (threadIdx.x == 0 && active)
-    {
-        R M11 = 0, M12 = 0, M22 = 0, g1 = 0, g2 = 0;
-        for (int32_t i = 0; i < nf; ++i)
-        {
-            Ec += s_w[i] * s_ec[i];
-            M11 += s_w[i] * s_qa[i] * s_qa[i];
-            M12 += s_w[i] * s_qa[i] * s_qb[i];
-            M22 += s_w[i] * s_qb[i] * s_qb[i];
-            g1 += s_w[i] * s_qa[i];
-            g2 += s_w[i] * s_qb[i];
-        }
-        const R tr = M11 + M22;
-        const R eps = 1e-14 * tr;
-        const R det = (M11 + eps) * (M22 + eps) - M12 * M12;
-        R l1 = 0, l2 = 0;
-        if (tr > 0 && det > 0)
-        {
-            l1 = ((M22 + eps) * g1 - M12 * g2) / det;
-            l2 = ((M11 + eps) * g2 - M12 * g1) / det;
-        }
-        s_l[0] = l1; s_l[1] = l2;
-    }
-    __syncthreads();
-    if (active)
-        for (int32_t i = threadIdx.x; i < nf; i += blockDim.x)
-        {
-            const int32_t f = pid(d.e2f[f0 + i]);
-            const R omega = s_w[i] * (1.0 - (s_qa[i] * s_l[0] + s_qb[i] * s_l[1]));
-            s_ec[i] = omega * s_aef[i] * s_sig[i] * (phi_ind[f] / d.famag[f]);
-        }
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        R out = E_in ? E_in[e] : 0.0;
-        if (active)
-        {
-            R Eu = 0;
-            for (int32_t i = 0; i < nf; ++i) Eu += s_ec[i];
-            out += Ec + 2.0 * cuct * L * Eu;
-        }
-        E_out[e] = apply_bc ? edge_bc(d, P, e, out) : out;
-    }
+    extern __shared__ double heavy_shared[];
+    const int32_t b = blockIdx.x;
+    if (b < n_heavy) edge_emf_heavy<R>(d, P, Ef, u_cell, cuct, heavy[b], E_in, E_out, apply_bc, reinterpret_cast<R *>(heavy_shared), hv);
+    else edge_emf_light<R>(d, P, Ef, u_cell, cuct, vmax, (b - n_heavy) * int32_t(blockDim.x) + int32_t(threadIdx.x), E_in, E_out, apply_bc);
 }
 
 // faraday_update / faraday_update_edge_dt (Common/induction/Faraday.cpp:15-36): B -= dt d1 E.
 template <class R> __global__ void __launch_bounds__(256) k_faraday(DevMesh d, const R *E, const double *dte, const R *dt_dev, double dt_val,
                                                  R *B)
 {
-    const int32_t f = gid();
-    if (f >= d.nf) return;
-    if (d.fL[f] < 0 && d.fR[f] < 0) return;
-    R circ = 0.0;
-    if (dte)
-    {
-        for (int32_t k = d.f2e_ptr[f]; k < d.f2e_ptr[f + 1]; ++k)
-        {
-            const int32_t v = d.f2e[k], e = pid(v);
-            circ += psg(v) * dte[e] * E[e];
-        }
-        B[f] -= circ;
-    }
-    else
-    {
-        for (int32_t k = d.f2e_ptr[f]; k < d.f2e_ptr[f + 1]; ++k)
-        {
-            const int32_t v = d.f2e[k];
-            circ += psg(v) * E[pid(v)];
-        }
-        const R dt = dt_dev ? dt_dev[0] : dt_val;
-        B[f] -= dt * circ;
-    }
+    faraday_face(d, E, dte, dt_dev, dt_val, B, gid());
 }
 
 // div_b (Common/diagnostics/DivB.cpp:8-24): per-block (max |s|, first cell attaining it, max rel).
@@ -1005,20 +629,16 @@ template __global__ void k_shell_energy<double>(DevMesh, const double *, const d
 template __global__ void k_shell_energy<Dual>(DevMesh, const Dual *, const Dual *, double, double, Dual *);
 template __global__ void k_prepare<double>(DevMesh d, Params P, SpCT<double> Us, const double *Phi, const double *Badd, SpWT<double> Ws, double *Bind, double *Btot, double *uplus, double *alpha, double *dt_part);
 template __global__ void k_dt_final<double>(const double *part, int32_t n, double dt_max, double *out);
-template __global__ void k_grad_current<double, false>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<double> Ws, SpCT<double> ghosts, SpWT<double> grads, int32_t limit, const double *Bind, double *J);
-template __global__ void k_grad_current<double, true>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<double> Ws, SpCT<double> ghosts, SpWT<double> grads, int32_t limit, const double *Bind, double *J);
-template __global__ void k_face_species<double>(DevMesh d, Params P, int32_t ns, SpCT<double> Ws, SpCT<double> grads, double *FA);
-template __global__ void k_face<double>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<double> Ws, SpCT<double> grads, SpCT<double> ghosts, double *FA, const double *uplus, const double *Btot, const double *Bind, const double *Phi, const double *PhiAdd, double *Ef);
+template __global__ void k_grad_current<double>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<double> Ws, SpCT<double> ghosts, SpWT<double> grads, int32_t limit, const double *Bind, double *J);
+template __global__ void k_face<double>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<double> Ws, SpCT<double> grads, SpCT<double> ghosts, double *FA, const double *uplus, const double *Btot, const double *Bind, const double *Phi, const double *PhiAdd, const double *phi_ind, double *Ef);
 template __global__ void k_cell_update<double>(DevMesh d, Params P, int32_t ns, int32_t s0, const double *FA, SpCT<double> rhs_in, SpCT<double> Wall, const double *Btot, const double *J, const double *dt_dev, double dt_val, int32_t sources, int32_t update, SpWT<double> Us, SpWT<double> rhs_out);
-template __global__ void k_edge_emf<double>(DevMesh d, Params P, const double *Ef, const double *u_cell, const double *phi_ind, double cuct, int32_t vmax, const double *E_in, double *E_out, int32_t apply_bc);
-template __global__ void k_edge_emf_heavy<double>(DevMesh d, Params P, const double *Ef, const double *u_cell, const double *phi_ind, double cuct, const int32_t *heavy, const double *E_in, double *E_out, int32_t apply_bc);
+template __global__ void k_edge_emf<double>(DevMesh d, Params P, const double *Ef, const double *u_cell, double cuct, int32_t vmax, const double *E_in, double *E_out, int32_t apply_bc, const int32_t *heavy, int32_t n_heavy, int32_t hv);
 template __global__ void k_faraday<double>(DevMesh d, const double *E, const double *dte, const double *dt_dev, double dt_val, double *B);
 template __global__ void k_prepare<Dual>(DevMesh d, Params P, SpCT<Dual> Us, const Dual *Phi, const Dual *Badd, SpWT<Dual> Ws, Dual *Bind, Dual *Btot, Dual *uplus, Dual *alpha, Dual *dt_part);
 template __global__ void k_dt_final<Dual>(const Dual *part, int32_t n, double dt_max, Dual *out);
-template __global__ void k_grad_current<Dual, false>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<Dual> Ws, SpCT<Dual> ghosts, SpWT<Dual> grads, int32_t limit, const Dual *Bind, Dual *J);
-template __global__ void k_face<Dual>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<Dual> Ws, SpCT<Dual> grads, SpCT<Dual> ghosts, Dual *FA, const Dual *uplus, const Dual *Btot, const Dual *Bind, const Dual *Phi, const Dual *PhiAdd, Dual *Ef);
+template __global__ void k_grad_current<Dual>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<Dual> Ws, SpCT<Dual> ghosts, SpWT<Dual> grads, int32_t limit, const Dual *Bind, Dual *J);
+template __global__ void k_face<Dual>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<Dual> Ws, SpCT<Dual> grads, SpCT<Dual> ghosts, Dual *FA, const Dual *uplus, const Dual *Btot, const Dual *Bind, const Dual *Phi, const Dual *PhiAdd, const Dual *phi_ind, Dual *Ef);
 template __global__ void k_cell_update<Dual>(DevMesh d, Params P, int32_t ns, int32_t s0, const Dual *FA, SpCT<Dual> rhs_in, SpCT<Dual> Wall, const Dual *Btot, const Dual *J, const Dual *dt_dev, double dt_val, int32_t sources, int32_t update, SpWT<Dual> Us, SpWT<Dual> rhs_out);
-template __global__ void k_edge_emf<Dual>(DevMesh d, Params P, const Dual *Ef, const Dual *u_cell, const Dual *phi_ind, double cuct, int32_t vmax, const Dual *E_in, Dual *E_out, int32_t apply_bc);
-template __global__ void k_edge_emf_heavy<Dual>(DevMesh d, Params P, const Dual *Ef, const Dual *u_cell, const Dual *phi_ind, double cuct, const int32_t *heavy, const Dual *E_in, Dual *E_out, int32_t apply_bc);
+template __global__ void k_edge_emf<Dual>(DevMesh d, Params P, const Dual *Ef, const Dual *u_cell, double cuct, int32_t vmax, const Dual *E_in, Dual *E_out, int32_t apply_bc, const int32_t *heavy, int32_t n_heavy, int32_t hv);
 template __global__ void k_faraday<Dual>(DevMesh d, const Dual *E, const double *dte, const Dual *dt_dev, double dt_val, Dual *B);
 } // namespace mhdg

@@ -2,7 +2,7 @@
 // Finite-volume device helpers shared by the explicit-stage kernels and their adjoints: cell vector
 // reconstruction, CFL time step, face states, Rusanov flux, ghost states, the UCT edge quantities and the
 // boundary EMF.  Templates on the real type R (double, or Dual for forward-mode derivatives).
-#include "dev.h"
+#include "kernels.h"
 
 namespace mhdg
 {
@@ -172,6 +172,34 @@ template <class R> __device__ void rusanov(const PrimT<R> &L, const PrimT<R> &Rt
     for (int m = 0; m < 5; ++m) F[m] = 0.5 * (FL[m] + FR[m]) - 0.5 * s * (UR[m] - UL[m]);
 }
 
+// Stencil neighbour state of a boundary entry (nb < 0, face f = -(nb + 1), c2f entry v): the ghost table row, or
+// ghost_state (Common/fluid/Reconstruction.cpp:9-24) with the cell value wc inside.
+template <class R>
+__device__ __forceinline__ void stencil_ghost(const DevMesh &d, int32_t sp, const R *gh, const R *wc, const R *fs, int32_t v, int32_t nb,
+                                              R *wn)
+{
+    const int32_t f = -(nb + 1);
+    if (gh)
+    {
+        for (int m = 0; m < 5; ++m) wn[m] = gh[5 * size_t(f) + m];
+        return;
+    }
+    const int8_t kind = d.kind[f];
+    for (int m = 0; m < 5; ++m) wn[m] = wc[m];
+    if (kind == kWall)
+    {
+        if (sp == 1) { wn[0] = 1e-12; wn[1] = 0; wn[2] = 0; wn[3] = 0; wn[4] = 1e-12; }
+        else
+        {
+            const V3T<R> n = (psg(v) / d.famag[f]) * L3(d.farea, f);
+            const R un = wc[1] * n.x + wc[2] * n.y + wc[3] * n.z;
+            wn[1] -= 2 * un * n.x; wn[2] -= 2 * un * n.y; wn[3] -= 2 * un * n.z;
+        }
+    }
+    else if (kind == kInflow)
+        for (int m = 0; m < 5; ++m) wn[m] = fs[m];
+}
+
 // ghost_state (Common/fluid/Reconstruction.cpp:9-24)
 template <class R> __device__ __forceinline__ PrimT<R> ghost_state(int8_t kind, int species, const PrimT<R> &in, const V3T<R> &n, const R *fs)
 {
@@ -194,7 +222,8 @@ __device__ __forceinline__ void face_dirs(const DevMesh &d, int32_t f, int32_t e
     v -= dot(v, th) * th;
     const double nv = norm(v);
     m = nv > 0 ? (1.0 / nv) * v : V3();
-    nrm = (1.0 / d.famag[f]) * L3(d.farea, f);
+    const double *g = d.geo + 4 * size_t(f);
+    nrm = V3(g[0], g[1], g[2]);
 }
 template <class R> __device__ __forceinline__ R edge_amax(const DevMesh &d, const R *u_cell, int32_t c0, int32_t c1, const V3T<R> &m)
 {
@@ -233,6 +262,288 @@ template <class R> __device__ __forceinline__ R edge_bc(const DevMesh &d, const 
         return dot(V3T<R>(seeded<R>(P.E_inf[0], P.dE_inf[0]), seeded<R>(P.E_inf[1], P.dE_inf[1]), seeded<R>(P.E_inf[2], P.dE_inf[2])),
                    L3(d.evec, e));
     return v;
+}
+} // namespace
+namespace
+{
+template <class R> __device__ __forceinline__ V3T<R> emf_of(const R *Ef, int32_t f)
+{
+    const R *q = Ef + 4 * size_t(f);
+    return V3T<R>(q[0], q[1], q[2]);
+}
+
+// One high-valence edge per block (pole axes of a lat-lon net): per-face terms in parallel, every sum sequential in the
+// reference's order.  sh holds eight rows of hv values (hv the largest valence of the mesh).
+template <class R>
+__device__ __forceinline__ void edge_emf_heavy(const DevMesh &d, const Params &P, const R *Ef, const R *u_cell, double cuct, int32_t e,
+                                               const R *E_in, R *E_out, int32_t apply_bc, R *sh, int32_t hv)
+{
+    constexpr int kHS = kHeavyShared<R>();
+    R *s_w = sh, *s_ec = sh + hv, *s_qa = sh + 2 * hv, *s_qb = sh + 3 * hv, *s_sig = sh + 4 * hv, *s_aef = sh + 5 * hv;
+    __shared__ R s_l[3];
+    const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1], nf = f1 - f0;
+    const int32_t c0 = d.ec_ptr[e], c1 = d.ec_ptr[e + 1];
+    bool any_fluid = false;
+    for (int32_t k = c0; k < c1 && !any_fluid; ++k) any_fluid = d.mat[d.ec_cell[k]] == 0;
+    const bool active = nf > 0 && d.elen[e] > 0 && any_fluid;
+    const V3 t = L3(d.evec, e);
+    const double L = d.elen[e];
+    const V3 th = (1.0 / L) * t;
+    V3 e1, e2;
+    plane_basis(th, e1, e2);
+    // The edge's cell velocities are staged in LDS (in s_qa, s_qb, s_sig, before those take the per-face terms):
+    // every face's max over the cells then reads LDS, where a dependent global gather per (face, cell) pair made
+    // this kernel latency-bound (n_lon^2 pairs per pole-axis edge).  Same values, same order.
+    const int32_t nc = c1 - c0;
+    const bool staged = active && nc <= hv;
+    if (staged)
+        for (int32_t k = threadIdx.x; k < nc; k += blockDim.x)
+        {
+            const V3T<R> u = L3(u_cell, d.ec_cell[c0 + k]);
+            s_qa[k] = u.x; s_qb[k] = u.y; s_sig[k] = u.z;
+        }
+    __syncthreads();
+    constexpr int kPer = (kHS + 255) / 256; // faces per thread (nf <= kHS, 256 threads)
+    R qa_r[kPer], qb_r[kPer], sig_r[kPer];
+    if (active)
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+        {
+            const int32_t i = int32_t(threadIdx.x) + j * int32_t(blockDim.x);
+            if (i >= nf) break;
+            const int32_t f = pid(d.e2f[f0 + i]);
+            s_w[i] = d.efw[f0 + i];
+            s_ec[i] = dot(emf_of(Ef, f), t);
+            V3 m, nrm;
+            face_dirs(d, f, e, th, m, nrm);
+            R aef = 0.0;
+            if (staged)
+                for (int32_t k = 0; k < nc; ++k) aef = mx(aef, fabs(dot(V3T<R>(s_qa[k], s_qb[k], s_sig[k]), m)));
+            else
+                aef = edge_amax(d, u_cell, c0, c1, m);
+            const R sig = dot(th, cross(m, nrm));
+            const V3T<R> qv = (aef * sig) * nrm;
+            qa_r[j] = dot(qv, e1);
+            qb_r[j] = dot(qv, e2);
+            sig_r[j] = sig;
+            s_aef[i] = aef;
+        }
+    __syncthreads(); // every read of the staged velocities is done
+    if (active)
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+        {
+            const int32_t i = int32_t(threadIdx.x) + j * int32_t(blockDim.x);
+            if (i >= nf) break;
+            s_qa[i] = qa_r[j]; s_qb[i] = qb_r[j]; s_sig[i] = sig_r[j];
+        }
+    __syncthreads();
+    // the sequential sums side by side: M11, M12, M22, g1, g2 and Ec on a wave each would be idle most of the time, so
+    // the first lanes of one wave take one sum each
+    __shared__ R s_sum[6];
+    if (threadIdx.x < 6 && active)
+    {
+        const int32_t w = threadIdx.x;
+        const R *x = w == 5 ? s_ec : w == 2 || w == 4 ? s_qb : s_qa;
+        const R *y = w == 0 ? s_qa : s_qb;
+        R acc = 0;
+        if (w < 3)
+            for (int32_t i = 0; i < nf; ++i) acc += s_w[i] * x[i] * y[i];
+        else
+            for (int32_t i = 0; i < nf; ++i) acc += s_w[i] * x[i];
+        s_sum[w] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && active)
+    {
+        R l1, l2;
+        uct_solve(s_sum[0], s_sum[1], s_sum[2], s_sum[3], s_sum[4], l1, l2);
+        s_l[0] = l1; s_l[1] = l2;
+    }
+    __syncthreads();
+    if (active)
+        for (int32_t i = threadIdx.x; i < nf; i += blockDim.x)
+        {
+            const int32_t f = pid(d.e2f[f0 + i]);
+            const R omega = s_w[i] * (1.0 - (s_qa[i] * s_l[0] + s_qb[i] * s_l[1]));
+            s_ec[i] = omega * s_aef[i] * s_sig[i] * Ef[4 * size_t(f) + 3];
+        }
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        R out = E_in ? E_in[e] : 0.0;
+        if (active)
+        {
+            R Eu = 0;
+            for (int32_t i = 0; i < nf; ++i) Eu += s_ec[i];
+            out += s_sum[5] + 2.0 * cuct * L * Eu;
+        }
+        E_out[e] = apply_bc ? edge_bc(d, P, e, out) : out;
+    }
+}
+
+// B -= dt d1 E of one face (Common/induction/Faraday.cpp:15-36), or with a per-edge step dte B -= d1 (dte E)
+template <class R>
+__device__ __forceinline__ void faraday_face(const DevMesh &d, const R *E, const double *dte, const R *dt_dev, double dt_val, R *B, int32_t f)
+{
+    if (f >= d.nf) return;
+    if (d.fL[f] < 0 && d.fR[f] < 0) return;
+    R circ = 0.0;
+    if (dte)
+    {
+        for (int32_t k = d.f2e_ptr[f]; k < d.f2e_ptr[f + 1]; ++k)
+        {
+            const int32_t v = d.f2e[k], e = pid(v);
+            circ += psg(v) * dte[e] * E[e];
+        }
+        B[f] -= circ;
+        return;
+    }
+    if (d.fdeg == 3)
+    {
+        // triangles: the three edge entries in one 12-byte load, then the gathers, summed in entry order
+        const int3 q = reinterpret_cast<const int3 *>(d.f2e)[f];
+        const R x = E[pid(q.x)], y = E[pid(q.y)], z = E[pid(q.z)];
+        circ += psg(q.x) * x;
+        circ += psg(q.y) * y;
+        circ += psg(q.z) * z;
+    }
+    else
+        for (int32_t k = d.f2e_ptr[f]; k < d.f2e_ptr[f + 1]; ++k)
+        {
+            const int32_t v = d.f2e[k];
+            circ += psg(v) * E[pid(v)];
+        }
+    const R dt = dt_dev ? dt_dev[0] : dt_val;
+    B[f] -= dt * circ;
+}
+
+// One edge of valence at most `vmax` per thread (IdealEMF.cpp:59-128)
+template <class R>
+__device__ __forceinline__ void edge_emf_light(const DevMesh &d, const Params &P, const R *Ef, const R *u_cell, double cuct, int32_t vmax,
+                                               int32_t e, const R *E_in, R *E_out, int32_t apply_bc)
+{
+    if (e >= d.ne) return;
+    const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1];
+    const int32_t nf = f1 - f0;
+    if (nf > vmax) return;
+    R out = E_in ? E_in[e] : 0.0;
+    const int32_t c0 = d.ec_ptr[e], c1 = d.ec_ptr[e + 1];
+    const int32_t nc = c1 - c0;
+    const bool fast = nf <= kEmfFast && nc <= kEmfFast;
+    // common valence: the row indices are loaded once, together, before their gathers
+    int32_t fid[kEmfFast], cid[kEmfFast];
+    bool any_fluid = false;
+    if (fast)
+    {
+#pragma unroll
+        for (int i = 0; i < kEmfFast; ++i)
+        {
+            if (i < nf) fid[i] = pid(d.e2f[f0 + i]);
+            if (i < nc) cid[i] = d.ec_cell[c0 + i];
+        }
+#pragma unroll
+        for (int k = 0; k < kEmfFast; ++k)
+            if (k < nc) any_fluid |= d.mat[cid[k]] == 0;
+    }
+    else
+        for (int32_t k = c0; k < c1 && !any_fluid; ++k) any_fluid = d.mat[d.ec_cell[k]] == 0;
+    if (nf > 0 && d.elen[e] > 0 && any_fluid)
+    {
+        const V3 t = L3(d.evec, e);
+        const double L = d.elen[e];
+        const V3 th = (1.0 / L) * t;
+        R Ec = 0;
+        if (fast)
+        {
+            V3T<R> ef[kEmfFast];
+#pragma unroll
+            for (int i = 0; i < kEmfFast; ++i)
+                if (i < nf) ef[i] = emf_of(Ef, fid[i]);
+#pragma unroll
+            for (int i = 0; i < kEmfFast; ++i)
+                if (i < nf) Ec += d.efw[f0 + i] * dot(ef[i], t);
+        }
+        else
+            for (int32_t i = f0; i < f1; ++i) Ec += d.efw[i] * dot(emf_of(Ef, pid(d.e2f[i])), t);
+        V3 e1, e2;
+        plane_basis(th, e1, e2);
+        R M11 = 0, M12 = 0, M22 = 0, g1 = 0, g2 = 0, Eu = 0;
+        if (fast)
+        {
+            // the edge's cell velocities and the per-face terms stay in registers, so the second pass re-reads
+            // nothing (same operations in the same order as the general path)
+            V3T<R> uc[kEmfFast];
+#pragma unroll
+            for (int k = 0; k < kEmfFast; ++k)
+                if (k < nc) uc[k] = L3(u_cell, cid[k]);
+            R fqa[kEmfFast], fqb[kEmfFast], faef[kEmfFast], fsig[kEmfFast];
+#pragma unroll
+            for (int i = 0; i < kEmfFast; ++i)
+                if (i < nf)
+                {
+                    const int32_t f = fid[i];
+                    V3 m, nrm;
+                    face_dirs(d, f, e, th, m, nrm);
+                    R aef = 0.0;
+#pragma unroll
+                    for (int k = 0; k < kEmfFast; ++k)
+                        if (k < nc) aef = mx(aef, fabs(dot(uc[k], m)));
+                    const R sig = dot(th, cross(m, nrm));
+                    const V3T<R> qv = (aef * sig) * nrm;
+                    const R qa = dot(qv, e1), qb = dot(qv, e2), w = d.efw[f0 + i];
+                    M11 += w * qa * qa;
+                    M12 += w * qa * qb;
+                    M22 += w * qb * qb;
+                    g1 += w * qa;
+                    g2 += w * qb;
+                    fqa[i] = qa; fqb[i] = qb; faef[i] = aef; fsig[i] = sig;
+                }
+            R l1, l2;
+            uct_solve(M11, M12, M22, g1, g2, l1, l2);
+            // the face weight and flux are loaded again (cache hits) rather than held across the solve
+#pragma unroll
+            for (int i = 0; i < kEmfFast; ++i)
+                if (i < nf)
+                {
+                    const R omega = d.efw[f0 + i] * (1.0 - (fqa[i] * l1 + fqb[i] * l2));
+                    Eu += omega * faef[i] * fsig[i] * Ef[4 * size_t(fid[i]) + 3];
+                }
+        }
+        else
+        {
+            for (int32_t i = f0; i < f1; ++i)
+            {
+                const int32_t f = pid(d.e2f[i]);
+                V3 m, nrm;
+                face_dirs(d, f, e, th, m, nrm);
+                const R aef = edge_amax(d, u_cell, c0, c1, m);
+                const V3T<R> qv = (aef * dot(th, cross(m, nrm))) * nrm;
+                const R qa = dot(qv, e1), qb = dot(qv, e2), w = d.efw[i];
+                M11 += w * qa * qa;
+                M12 += w * qa * qb;
+                M22 += w * qb * qb;
+                g1 += w * qa;
+                g2 += w * qb;
+            }
+            R l1, l2;
+            uct_solve(M11, M12, M22, g1, g2, l1, l2);
+            for (int32_t i = f0; i < f1; ++i)
+            {
+                const int32_t f = pid(d.e2f[i]);
+                V3 m, nrm;
+                face_dirs(d, f, e, th, m, nrm);
+                const R aef = edge_amax(d, u_cell, c0, c1, m);
+                const V3T<R> qv = (aef * dot(th, cross(m, nrm))) * nrm;
+                const R qa = dot(qv, e1), qb = dot(qv, e2), w = d.efw[i];
+                const R omega = w * (1.0 - (qa * l1 + qb * l2));
+                const R sig = dot(th, cross(m, nrm));
+                Eu += omega * aef * sig * Ef[4 * size_t(f) + 3];
+            }
+        }
+        out += Ec + 2.0 * cuct * L * Eu;
+    }
+    E_out[e] = apply_bc ? edge_bc(d, P, e, out) : out;
 }
 } // namespace
 } // namespace mhdg

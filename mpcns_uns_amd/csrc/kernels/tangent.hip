@@ -219,7 +219,7 @@ void mhdg_ctx::tangent_alloc()
     tw.U[0] = D(5 * C); tw.U[1] = D(5 * C); tw.Phi = D(F); tw.PhiAdd = D(F); tw.Badd = D(3 * C);
     tw.W[0] = D(5 * C); tw.W[1] = D(5 * C); tw.grad[0] = D(15 * C); tw.grad[1] = D(15 * C);
     tw.Bind = D(3 * C); tw.Btot = D(3 * C); tw.uplus = D(3 * C); tw.J = D(3 * C); tw.alpha = D(C);
-    tw.FA = D(10 * F); tw.Ef = D(3 * F); tw.E = D(E);
+    tw.FA = D(10 * F); tw.Ef = D(4 * F); tw.E = D(E);
     tw.dt_part = D(size_t(nbk(nc)) + 1); tw.dt_dev = D(1); tw.part = D(size_t(nbk(nc)));
     if (!energy_part) energy_part = static_cast<double *>(alloc(size_t(nbk(nc)) * 8));
 }
@@ -252,17 +252,13 @@ void mhdg_ctx::explicit_tangent(int n_steps, double dt_max, const Params &Pt)
                1, static_cast<const Dual *>(tw.Bind), tw.J);
         LAUNCH("face_t", k_face<Dual>, dim3(nbk(nf)), dim3(256), 0, stream, d, Pt, 2, 0, Ws, gradsC, none, tw.FA,
                static_cast<const Dual *>(tw.uplus), static_cast<const Dual *>(tw.Btot), static_cast<const Dual *>(tw.Bind),
-               static_cast<const Dual *>(tw.Phi), static_cast<const Dual *>(tw.PhiAdd), tw.Ef);
+               static_cast<const Dual *>(tw.Phi), static_cast<const Dual *>(tw.PhiAdd), static_cast<const Dual *>(tw.Phi), tw.Ef);
         LAUNCH("cell_update_t", k_cell_update<Dual>, dim3(nb), dim3(256), 0, stream, d, Pt, 2, 0, static_cast<const Dual *>(tw.FA), none,
                Ws, static_cast<const Dual *>(tw.Btot),
                static_cast<const Dual *>(tw.J), static_cast<const Dual *>(tw.dt_dev), 0.0, 1, 1, Us, noneW);
-        LAUNCH("edge_emf_t", k_edge_emf<Dual>, dim3(nbk(ne)), dim3(256), 0, stream, d, Pt, static_cast<const Dual *>(tw.Ef),
-               static_cast<const Dual *>(tw.uplus), static_cast<const Dual *>(tw.Phi), Pt.cuct, kLightMax, static_cast<const Dual *>(nullptr),
-               tw.E, 1);
-        if (n_heavy)
-            LAUNCH("edge_emf_heavy_t", k_edge_emf_heavy<Dual>, dim3(n_heavy), dim3(256), 0, stream, d, Pt, static_cast<const Dual *>(tw.Ef),
-                   static_cast<const Dual *>(tw.uplus), static_cast<const Dual *>(tw.Phi), Pt.cuct, static_cast<const int32_t *>(heavy),
-                   static_cast<const Dual *>(nullptr), tw.E, 1);
+        LAUNCH("edge_emf_t", k_edge_emf<Dual>, dim3(n_heavy + nbk(ne)), dim3(256), n_heavy ? 6 * size_t(max_valence) * sizeof(Dual) : 0, stream,
+               d, Pt, static_cast<const Dual *>(tw.Ef), static_cast<const Dual *>(tw.uplus), Pt.cuct, kLightMax,
+               static_cast<const Dual *>(nullptr), tw.E, 1, static_cast<const int32_t *>(heavy), n_heavy, max_valence);
         LAUNCH("faraday_t", k_faraday<Dual>, dim3(nbk(nf)), dim3(256), 0, stream, d, static_cast<const Dual *>(tw.E),
                static_cast<const double *>(nullptr), static_cast<const Dual *>(tw.dt_dev), 0.0, tw.Phi);
         check_launch("explicit tangent step");
