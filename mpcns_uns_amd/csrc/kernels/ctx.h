@@ -1,6 +1,7 @@
 #pragma once
 // Device context: mesh tables, resident state, work buffers and the host drivers of the step and of the
 // implicit induction solves.
+#include <algorithm>
 #include <map>
 #include <string>
 #include <vector>
@@ -37,7 +38,8 @@ struct mhdg_ctx
     double *phi_w = nullptr, *bcell = nullptr, *gcell = nullptr, *corr = nullptr;
     bool have_corr = false;
     double *x0 = nullptr, *bvec = nullptr, *rvec = nullptr, *wvec = nullptr, *invdiag = nullptr, *delta = nullptr, *tmp = nullptr;
-    double *scal = nullptr, *hcol = nullptr, *ydev = nullptr;
+    double *scal = nullptr; // norms on the device
+    double *ortho_part = nullptr, *ortho_cols = nullptr, *ortho_norms = nullptr, *ortho_h = nullptr, *gram = nullptr;
     // ImplicitInduction flags (ImplicitInduction.cpp:11) and the parts apply_op evaluates
     bool op_res = false, op_hall = false, ideal_cfg = false, skip_implicit = false;
     double *u_ideal = nullptr, *ide = nullptr, *Ef_i = nullptr; // implicit ideal part (set_ideal_state)
@@ -68,7 +70,6 @@ struct mhdg_ctx
     std::vector<double *> V;
     double **Vptrs = nullptr;
     int restart = 2;
-    mhdg::RedScratch rs{};
     mhdg::MixedSolver *mixed = nullptr;
     // multigrid preconditioner (multigrid.hip): the host arrays the hierarchy is built from (kept when the mesh
     // descriptor carries e2n), the device hierarchy, and the Dirichlet set it was built for
@@ -80,8 +81,12 @@ struct mhdg_ctx
     void mg_prepare(double dt);
     void mg_cycle(int l, const float *b, float *x);
     void op32(int mode, int hall_on, const float *pv, const float *v, const float *b, float omega, float *out);
-    // pinned host memory: the step's time step at offset 0, small read-backs staged at kPinStageOffset
-    static constexpr size_t kPinBytes = 4096, kPinStageOffset = 2048, kPinStageBytes = 2048;
+    // pinned host memory: what kernels hand over (the solvers' in `box`, the step's time step in `dt_box`), small read-backs
+    // staged at kPinStageOffset
+    static constexpr size_t kPinBytes = 4096, kPinBoxOffset = 0, kPinDtBoxOffset = 1024, kPinStageOffset = 2048, kPinStageBytes = 2048;
+    mhdg::HostBox *box = nullptr, *dt_box = nullptr;
+    uint64_t ticket = 0;                              // of the last launched kernel that writes a box
+    const double *wait_box(const mhdg::HostBox *b);   // the values of the box it writes, once they are there
     void *host_pin = nullptr;
     std::vector<void *> owned;
     std::map<int, std::pair<void *, size_t>> staging;
@@ -116,17 +121,53 @@ struct mhdg_ctx
     // the explicit stage, with_ct: and the CT update with its EMF; the state is untouched when it throws
     double explicit_stage(double dt_max, bool with_ct);
     void get_record(int32_t first, int32_t n, double *host);
-    double dot(const double *a, const double *b, int op, int slot);
+    const double *norms(const double *a, const double *b); // <a, a> and <b, b> (b nullable) on the host, |a| and |b| in scal
+    mhdg::Ortho<double> ortho64(int j); // the FP64 solvers' Arnoldi step j
+    // One classical Gram-Schmidt step, with a second projection when the first kept less than `dgks` of the norm: the
+    // coefficients (valid until the next kernel that writes the box) and h_{j+1,j}
+    template <class T> const double *arnoldi_cgs(mhdg::Ortho<T> o, double dgks, double &hn)
+    {
+        o.ticket = ++ticket;
+        prof_begin("multidot");
+        mhdg::ortho_dots(o, false, stream);
+        prof_end();
+        prof_begin("multiaxpy");
+        mhdg::ortho_update(o, mhdg::kCgs, dgks, stream);
+        prof_end();
+        check_launch("arnoldi");
+        const double *h = wait_box(box);
+        if (h[62] == 0.0)
+        {
+            hn = h[o.nv];
+            return h;
+        }
+        std::copy(h, h + o.nv, h_first);
+        o.ticket = ++ticket;
+        prof_begin("multidot");
+        mhdg::ortho_dots(o, false, stream);
+        prof_end();
+        prof_begin("multiaxpy");
+        mhdg::ortho_update(o, mhdg::kPlain, 0.0, stream);
+        mhdg::ortho_scale(o, stream);
+        prof_end();
+        check_launch("arnoldi (second projection)");
+        h = wait_box(box);
+        for (int i = 0; i < o.nv; ++i) h_first[i] += h[i];
+        hn = h[o.nv];
+        return h_first;
+    }
+    double h_first[64]{};
     void apply_op(const double *phi, const double *v, const double *inv, const int8_t *dir, double dt, int mode, int mask, const double *b,
                   double *out);
     // bvec = E_expl + F(Phi_n) and rvec = bvec - A x (no Jacobi scaling), the two products in one pass over the
     // tables where they allow it (no implicit ideal part, no tangent operator); the same bits as two apply_op calls
     void rhs_residual(const double *Phi_n, const double *E_expl, const double *x, const int8_t *dir, double dt);
+    const double *freeze_B = nullptr; // the step's B_tot for the solve's frozen field (B0 then takes it), else B0 as it is
+    void freeze(float *aB0);
     double *bcell2 = nullptr, *gcell2 = nullptr; // the second vector's cell fields of rhs_residual
     int solve64(const double *Phi_n, const double *E_expl, const int8_t *dir, double dt, double *E, double *rel_res);
     // the same system and iteration with classical Gram-Schmidt (cgs64.hip, precision 3)
     int solve64_cgs(const double *Phi_n, const double *E_expl, const int8_t *dir, double dt, double *E, double *rel_res);
-    double *cgs_part = nullptr, *cgs_h = nullptr;
     void mixed_build();
     // use_mg: the inner solve is flexible GMRES preconditioned by one V-cycle of the multigrid hierarchy built for dir_host
     // (the host copy of dir); otherwise GMRES with the Jacobi preconditioner

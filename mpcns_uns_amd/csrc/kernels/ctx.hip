@@ -290,18 +290,21 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     // induction work
     phi_w = D(F); bcell = D(3 * C); gcell = D(3 * C); corr = D(E); have_corr = false;
     x0 = D(E); bvec = D(E); rvec = D(E); wvec = D(E); invdiag = D(E); delta = D(E); tmp = D(E);
-    scal = D(64);
-    rs.partial = D(kRedBlocks);
-    rs.ticket = static_cast<unsigned *>(alloc(64));
-    hip_check(hipMemset(rs.ticket, 0, 64), "memset");
+    scal = D(2);
+    ortho_part = D(size_t(kCols) * kOrthoBlocks);
+    ortho_cols = D(kCols);
+    ortho_norms = D(kOrthoBlocks);
+    ortho_h = D(64);
+    gram = D(64 * 64);
     restart = std::max(2, c.ind_restart);
     V.resize(restart + 1);
     for (auto &v : V) v = D(E);
     Vptrs = static_cast<double **>(alloc(sizeof(double *) * V.size()));
     hip_check(hipMemcpy(Vptrs, V.data(), sizeof(double *) * V.size(), hipMemcpyHostToDevice), "upload");
-    hcol = D(restart + 2);
-    ydev = D(restart + 1);
     hip_check(hipHostMalloc(&host_pin, kPinBytes), "hipHostMalloc");
+    std::memset(host_pin, 0, kPinBytes);
+    box = reinterpret_cast<HostBox *>(static_cast<char *>(host_pin) + kPinBoxOffset);
+    dt_box = reinterpret_cast<HostBox *>(static_cast<char *>(host_pin) + kPinDtBoxOffset);
     hip_check(hipDeviceSynchronize(), "sync");
 }
 
@@ -314,14 +317,45 @@ void mhdg_ctx::launch_edge_emf(const double *Efp, const double *u, double cuct, 
     check_launch("edge emf");
 }
 
-double mhdg_ctx::dot(const double *a, const double *b, int op, int slot)
+const double *mhdg_ctx::wait_box(const HostBox *b)
 {
-    LAUNCH("dot", k_dot<double>, dim3(kRedBlocks), dim3(kRedThreads), 0, stream, a, b, ne, RedScratch{rs.partial, nullptr}, scal + slot, op);
-    LAUNCH("finish", k_finish, dim3(1), dim3(kRedThreads), 0, stream, static_cast<const double *>(rs.partial), kRedBlocks, scal + slot, op);
-    check_launch("dot");
-    double v;
-    d2h(&v, scal + slot, 8);
-    return v;
+    for (uint64_t spin = 1;; ++spin)
+    {
+        if (__atomic_load_n(&b->ticket, __ATOMIC_ACQUIRE) == ticket) return b->v;
+        if (spin % 65536 == 0)
+        {
+            // every few milliseconds: has the stream ended, or failed, without it?
+            const hipError_t e = hipStreamQuery(stream);
+            if (e == hipErrorNotReady) continue;
+            hip_check(e, "wait for the device");
+            if (__atomic_load_n(&b->ticket, __ATOMIC_ACQUIRE) == ticket) return b->v;
+            throw std::runtime_error("the device's result did not arrive");
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+const double *mhdg_ctx::norms(const double *a, const double *b)
+{
+    prof_begin("dot");
+    norms2(a, b, ne, ortho_part, scal, box, ++ticket, stream);
+    prof_end();
+    check_launch("norms");
+    return wait_box(box);
+}
+
+// The frozen field of a step's solve, in FP64 and (aB0) times alpha in FP32, in one pass over the cells
+void mhdg_ctx::freeze(float *aB0)
+{
+    if (freeze_B || aB0)
+        LAUNCH("freeze", k_freeze, dim3(nblk(nc)), dim3(256), 0, stream, static_cast<const double *>(alpha), freeze_B ? freeze_B : B0, nc,
+               freeze_B ? B0 : nullptr, aB0);
+    freeze_B = nullptr;
+}
+
+Ortho<double> mhdg_ctx::ortho64(int j)
+{
+    return {Vptrs, j + 1, ne, wvec, V[j + 1], V[j], nullptr, nullptr, nullptr, ortho_part, ortho_cols, ortho_h, gram, ortho_norms, box, 0};
 }
 
 // F(phi) for a face vector phi into out (mode 0), or A x (mode 1) with x = precond(v) / v, optional mask /
@@ -350,11 +384,9 @@ void mhdg_ctx::apply_op(const double *phi_in, const double *v, const double *inv
         launch_edge_emf(Ef_i, u_ideal, P.cuct, nullptr, ide, 0);
     }
     const double *idp = ideal_part ? ide : nullptr;
-    LAUNCH("edge_apply", k_edge_apply, dim3(nblk(ne)), dim3(256), 0, stream, d, int32_t(op_res), int32_t(op_hall), phi, gcell, idp,
-           imask, v, inv, dir, dt, mode, mask, b, out);
-    if (n_heavy)
-        LAUNCH("edge_apply_heavy", k_edge_apply_heavy, dim3(n_heavy), dim3(256), 0, stream, d, int32_t(op_res), int32_t(op_hall),
-               static_cast<const int32_t *>(heavy), phi, gcell, idp, imask, v, inv, dir, dt, mode, mask, b, out);
+    const size_t lds = n_heavy ? kApplyHeavyRows * size_t(max_valence) * sizeof(double) : 0;
+    LAUNCH("edge_apply", k_edge_apply, dim3(n_heavy + nblk(ne)), dim3(256), lds, stream, d, int32_t(op_res), int32_t(op_hall), phi, gcell, idp,
+           imask, v, inv, dir, dt, mode, mask, b, out, static_cast<const int32_t *>(heavy), n_heavy, max_valence);
     check_launch("apply_op");
 }
 
@@ -379,79 +411,58 @@ void mhdg_ctx::rhs_residual(const double *Phi_n, const double *Eex, const double
         LAUNCH("hall_g", k_hall_g2_g<kCellLanes64>, dim3(nblk(lanes)), dim3(256), 0, stream, d, static_cast<const double *>(bcell),
                static_cast<const double *>(bcell2), alpha, B0, gcell, gcell2);
     }
-    LAUNCH("edge_apply", k_edge_rhs_residual, dim3(nblk(ne)), dim3(256), 0, stream, d, int32_t(op_res), int32_t(op_hall), Phi_n,
+    const size_t lds = n_heavy ? kResidualHeavyRows * size_t(max_valence) * sizeof(double) : 0;
+    LAUNCH("edge_apply", k_edge_rhs_residual, dim3(n_heavy + nblk(ne)), dim3(256), lds, stream, d, int32_t(op_res), int32_t(op_hall), Phi_n,
            static_cast<const double *>(gcell), static_cast<const double *>(phi_w), static_cast<const double *>(gcell2), Eex, x, dir, dt, bvec,
-           rvec);
-    if (n_heavy)
-        LAUNCH("edge_apply_heavy", k_edge_rhs_residual_heavy, dim3(n_heavy), dim3(256), 0, stream, d, int32_t(op_res), int32_t(op_hall),
-               static_cast<const int32_t *>(heavy), Phi_n, static_cast<const double *>(gcell), static_cast<const double *>(phi_w),
-               static_cast<const double *>(gcell2), Eex, x, dir, dt, bvec, rvec);
+           rvec, static_cast<const int32_t *>(heavy), n_heavy, max_valence);
     check_launch("rhs_residual");
 }
 
-// ImplicitInduction::solve (Common/induction/ImplicitInduction.cpp:299-390), FP64, Jacobi, MGS Arnoldi:
-// the reference's control flow with the Hessenberg / Givens arithmetic on the host.
+// ImplicitInduction::solve (Common/induction/ImplicitInduction.cpp:299-390), FP64, Jacobi, MGS Arnoldi (its
+// coefficients from one pass of dot products, krylov.hip): the reference's control flow with the Hessenberg / Givens
+// arithmetic on the host.
 int mhdg_ctx::solve64(const double *Phi_n, const double *Eex, const int8_t *dir, double dt, double *Eout, double *rel_res)
 {
     const int m = restart;
     const int max_it = cfg.ind_max_it;
     const double rtol = rtol_override > 0 ? rtol_override : cfg.ind_rtol;
+    freeze(nullptr);
     LAUNCH("solve_init", k_solve_init, dim3(nblk(ne)), dim3(256), 0, stream, Eex, have_corr ? corr : nullptr, dir, d.m_e, d.d2, dt,
-           dte_cur, ne, x0, invdiag);
+           dte_cur, ne, x0, invdiag, static_cast<float *>(nullptr), delta);
     rhs_residual(Phi_n, Eex, x0, dir, dt); // b = E_expl + F(Phi^n), r = b - A x0
-    hip_check(hipMemsetAsync(delta, 0, size_t(ne) * 8, stream), "memset");
-    const double bb = dot(bvec, bvec, 0, 0);
-    const double bnorm = std::sqrt(std::max(bb, 1e-300));
-    double beta = dot(rvec, rvec, 1, 1);
+    const double *nn = norms(rvec, bvec);
+    const double bnorm = std::sqrt(std::max(nn[1], 1e-300));
+    double beta = std::sqrt(nn[0]);
     int total = 0;
-    std::vector<std::vector<double>> H(m + 1, std::vector<double>(m, 0.0));
-    std::vector<double> cs(m), sn(m), g(m + 1), yv(m), hc(m + 2);
+    Hessenberg hs(m);
     while (beta > rtol * bnorm && total < max_it)
     {
-        LAUNCH("scale", k_div_scalar, dim3(nblk(ne)), dim3(256), 0, stream, rvec, scal + 1, ne, V[0]);
-        std::fill(g.begin(), g.end(), 0.0);
-        g[0] = beta;
+        LAUNCH("scale", k_div_scalar, dim3(nblk(ne)), dim3(256), 0, stream, rvec, scal, ne, V[0]);
+        hs.start(beta);
         int j = 0;
         for (; j < m && total < max_it; ++j, ++total)
         {
             apply_op(nullptr, V[j], invdiag, dir, dt, 1, 1, nullptr, wvec);
-            const RedScratch parts{rs.partial, nullptr};
-            for (int i = 0; i <= j; ++i)
-            {
-                LAUNCH("mgs", k_mgs<double>, dim3(kRedBlocks), dim3(kRedThreads), 0, stream, wvec, i > 0 ? V[i - 1] : nullptr, V[i], ne,
-                       hcol, i, 0, parts);
-                LAUNCH("finish", k_finish, dim3(1), dim3(kRedThreads), 0, stream, static_cast<const double *>(rs.partial), kRedBlocks, hcol + i, 0);
-            }
-            LAUNCH("mgs", k_mgs<double>, dim3(kRedBlocks), dim3(kRedThreads), 0, stream, wvec, V[j], nullptr, ne, hcol, j + 1, 1, parts);
-            LAUNCH("finish", k_finish, dim3(1), dim3(kRedThreads), 0, stream, static_cast<const double *>(rs.partial), kRedBlocks, hcol + j + 1, 1);
-            LAUNCH("scale", k_scale_div<double>, dim3(nblk(ne)), dim3(256), 0, stream, wvec, hcol + j + 1, ne, V[j + 1]);
+            Ortho<double> o = ortho64(j);
+            o.ticket = ++ticket;
+            prof_begin("multidot64");
+            ortho_dots(o, true, stream);
+            prof_end();
+            prof_begin("multiaxpy64");
+            ortho_update(o, kMgs, 0.0, stream);
+            prof_end();
+            prof_begin("scale");
+            ortho_scale(o, stream);
+            prof_end();
             check_launch("arnoldi");
-            d2h(hc.data(), hcol, sizeof(double) * (j + 2));
-            for (int i = 0; i <= j + 1; ++i) H[i][j] = hc[i];
-            for (int i = 0; i < j; ++i)
-            {
-                const double tt = cs[i] * H[i][j] + sn[i] * H[i + 1][j];
-                H[i + 1][j] = -sn[i] * H[i][j] + cs[i] * H[i + 1][j];
-                H[i][j] = tt;
-            }
-            const double den = std::hypot(H[j][j], H[j + 1][j]);
-            cs[j] = den > 0 ? H[j][j] / den : 1.0; sn[j] = den > 0 ? H[j + 1][j] / den : 0.0;
-            H[j][j] = den; H[j + 1][j] = 0.0;
-            g[j + 1] = -sn[j] * g[j]; g[j] = cs[j] * g[j];
-            if (std::abs(g[j + 1]) <= rtol * bnorm) { ++j; ++total; break; }
+            const double *h = wait_box(box);
+            if (hs.add(j, h, 0.0, h[j + 1]) <= rtol * bnorm) { ++j; ++total; break; }
         }
-        for (int i = j - 1; i >= 0; --i)
-        {
-            double s = g[i];
-            for (int k = i + 1; k < j; ++k) s -= H[i][k] * yv[k];
-            yv[i] = s / H[i][i];
-        }
-        hip_check(hipMemcpyAsync(ydev, yv.data(), sizeof(double) * std::max(j, 1), hipMemcpyHostToDevice, stream), "H2D");
-        LAUNCH("gmres_update", k_gmres_update, dim3(nblk(ne)), dim3(256), 0, stream, static_cast<const double *const *>(Vptrs), ydev, j,
-                           invdiag, dir, ne, delta);
-        LAUNCH("axpy", k_add, dim3(nblk(ne)), dim3(256), 0, stream, x0, delta, ne, tmp);
+        prof_begin("gmres_update");
+        solution_update<double>(Vptrs, hs.solve(j), j, invdiag, dir, ne, x0, delta, tmp, stream);
+        prof_end();
         apply_op(nullptr, tmp, nullptr, dir, dt, 1, 0, bvec, rvec);
-        beta = dot(rvec, rvec, 1, 1);
+        beta = std::sqrt(norms(rvec, nullptr)[0]);
     }
     LAUNCH("solve_final", k_solve_final, dim3(nblk(ne)), dim3(256), 0, stream, x0, delta, Eex, dir, ne, Eout, corr);
     check_launch("solve final");
@@ -475,7 +486,12 @@ double mhdg_ctx::step(double dt_max, int precision, int *iters, double *res)
     *res = 0.0;
     if (implicit)
     {
-        hip_check(hipMemcpyAsync(B0, Btot, 3 * size_t(nc) * 8, hipMemcpyDeviceToDevice, stream), "copy");
+        struct Frozen // a solve that throws before it took the field leaves none behind
+        {
+            mhdg_ctx *c;
+            ~Frozen() { c->freeze_B = nullptr; }
+        } frozen{this};
+        freeze_B = Btot;
         if (precision == 0) *iters = solve64(Phi, E_expl, dir_mercury, gdt, E_last, res);
         else if (precision == 3) *iters = solve64_cgs(Phi, E_expl, dir_mercury, gdt, E_last, res);
         else *iters = solve_mixed(Phi, E_expl, dir_mercury, gdt, E_last, res, precision == 2, dir_mercury_h.data());

@@ -12,6 +12,7 @@
 //   FA   per face and ion: the flux through the face (5).
 //   Ef   per face, 32 bytes: the EMF candidate (3) and Phi / |A|, what the edge sum reads of a face besides geo.
 #include "kernels.h"
+#include "krylov.h"
 
 namespace mhdg
 {

@@ -550,7 +550,7 @@ __device__ __forceinline__ void face_emf_role(const DevMesh &d, const StepFields
 }
 
 // min of the blocks' time steps, at most dt_max, on the device and into host memory (one block)
-__device__ __forceinline__ void dt_role(const double *part, int32_t n, double dt_max, double *out, double *sh)
+__device__ __forceinline__ void dt_role(const double *part, int32_t n, double dt_max, double *out, double *sh, HostBox *box, uint64_t ticket)
 {
     const int32_t t = threadIdx.x, nt = blockDim.x;
     double v = __builtin_inf();
@@ -562,8 +562,11 @@ __device__ __forceinline__ void dt_role(const double *part, int32_t n, double dt
 #pragma unroll
         for (int u = 0; u < 4; ++u) v = mn(v, x[u]);
     }
-    v = block_min(v, sh);
-    if (t == 0) out[0] = mn(v, dt_max);
+    v = mn(block_min(v, sh), dt_max);
+    __syncthreads(); // every thread has read the minimum
+    if (t == 0) out[0] = sh[0] = v;
+    __syncthreads();
+    publish(box, ticket, sh, 1);
 }
 
 // Rusanov flux through a face (FluxRHS.cpp:43-70) for one ion: thread (face, ion), the ions of a face side by side
@@ -673,14 +676,14 @@ __device__ __forceinline__ void update_role(const DevMesh &d, const Params &P, c
 template <int DEG, int NS>
 __global__ void __launch_bounds__(kStatesThreads, DEG == 6 ? 2 : 3) k_step_states(DevMesh d, Params P, StepFields F, const double *Phi, const double *PhiAdd,
                                                                    int32_t n_cell, int32_t n_face, const double *dt_part, int32_t n_part,
-                                                                   double dt_max, double *dt_dev)
+                                                                   double dt_max, double *dt_dev, HostBox *box, uint64_t ticket)
 {
     // the larger of the staged face states (5 DEG per thread) and the reduction of the time step
     __shared__ double stage[kStatesThreads * (DEG > 0 ? 5 * DEG : 1)];
     const int32_t b = blockIdx.x;
     if (b < n_cell) states_role<DEG, NS>(d, P, F, b, stage);
     else if (b < n_cell + n_face) face_emf_role(d, F, Phi, PhiAdd, (b - n_cell) * kStatesThreads + int32_t(threadIdx.x));
-    else dt_role(dt_part, n_part, dt_max, dt_dev, stage);
+    else dt_role(dt_part, n_part, dt_max, dt_dev, stage, box, ticket);
 }
 // Dynamic LDS: the heavy edges' rows (fv.h) when there are any
 template <int NS>
@@ -775,25 +778,16 @@ void mhdg_ctx::launch_states(int32_t n_face, double *dt_out, double dt_max)
     by_shape(cdeg, P.ns, [&](auto deg, auto ns) {
         LAUNCH("states", (k_step_states<decltype(deg)::value, decltype(ns)::value>), dim3(n_cell + n_face + (dt_out ? 1 : 0)),
                dim3(kStatesThreads), 0, stream, d, P, sf, static_cast<const double *>(Phi), static_cast<const double *>(PhiAdd), n_cell, n_face,
-               static_cast<const double *>(dt_part), n_part, dt_max, dt_out);
+               static_cast<const double *>(dt_part), n_part, dt_max, dt_out, dt_box, ticket);
     });
 }
 
 double mhdg_ctx::explicit_stage(double dt_max, bool with_ct)
 {
-    double *dth = static_cast<double *>(host_pin);
-    hipEvent_t ev;
-    auto read_dt = [&] {
-        chk(hipMemcpyAsync(dth, dt_dev, 8, hipMemcpyDeviceToHost, stream), "D2H");
-        chk(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
-        chk(hipEventRecord(ev, stream), "event");
-    };
     // nothing before this wrote U or Phi (only derived fields), so the state is unchanged when it throws
-    auto wait_dt = [&] {
-        chk(hipEventSynchronize(ev), "event sync");
-        (void)hipEventDestroy(ev);
-        if (!std::isfinite(dth[0]) || dth[0] <= 0) throw std::runtime_error("invalid time step");
-        return dth[0];
+    auto checked = [](double v) {
+        if (!std::isfinite(v) || v <= 0) throw std::runtime_error("invalid time step");
+        return v;
     };
     launch_prepare();
     // Strang split of the ions' gyration (Solver.cpp:237-241): half a step, then prepare again.  The rotation changes
@@ -803,21 +797,21 @@ double mhdg_ctx::explicit_stage(double dt_max, bool with_ct)
     if (split)
     {
         LAUNCH("dt_final", k_dt_final<double>, dim3(1), dim3(256), 0, stream, static_cast<const double *>(dt_part), blocks(nc, 256), dt_max, dt_dev);
-        read_dt();
-        gdt = wait_dt();
+        d2h(&gdt, dt_dev, 8);
+        checked(gdt);
         LAUNCH("gyrate", k_gyrate, dim3(blocks(nc, 256)), dim3(256), 0, stream, d, P, U[0], U[1], static_cast<const double *>(Btot),
                static_cast<const double *>(dt_dev), 0.5);
         launch_prepare();
     }
+    ++ticket;
     launch_states(blocks(nf, kStatesThreads), split ? nullptr : dt_dev, dt_max);
-    if (!split) read_dt();
     const int n_edge = blocks(ne, kRoleThreads), n_flux = blocks(nf, kRoleThreads / P.ns);
     const size_t lds = sizeof(double) * std::max<size_t>(5 * kRoleThreads, n_heavy ? 6 * size_t(max_valence) : 0);
     auto kflux = P.ns == 2 ? k_step_fluxes<2> : k_step_fluxes<0>;
     LAUNCH("fluxes", kflux, dim3(n_heavy + n_edge + n_flux), dim3(kRoleThreads), lds, stream, d, P, sf, E_expl, static_cast<const int32_t *>(heavy),
            n_heavy, max_valence, n_edge);
     check_launch("explicit stage");
-    if (!split) gdt = wait_dt();
+    if (!split) gdt = checked(wait_box(dt_box)[0]); // written while the states were formed
     SpW Us{};
     for (int s = 0; s < P.ns; ++s) Us.p[s] = U[s];
     const int n_cell = blocks(nc, kRoleThreads / P.ns), n_face = with_ct ? blocks(nf, kRoleThreads) : 0;

@@ -1,121 +1,10 @@
 // Implicit Hall/resistive induction operator (ImplicitInduction::apply_F / apply_A,
 // Common/induction/ImplicitInduction.cpp:127-198) as face, cell and edge gathers, plus the GMRES vector
-// kernels.  Reductions are deterministic: a fixed grid, a fixed per-block tree, and one block combines the
-// block partials in a fixed tree (k_finish, a second launch), so reruns are bit-identical.  (A last-block
-// ticket in the same launch costs ~90 us per reduction here: the 1024 blocks finish together and their
-// fenced atomics on one counter serialise.)
+// kernels that are not reductions (those are in krylov.hip).
 #include "induction.h"
 
 namespace mhdg
 {
-// ------------------------------------------------------------------------------------ reductions
-__device__ __forceinline__ double block_sum(double v, double *sh)
-{
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int s = kRedThreads / 2; s > 0; s >>= 1)
-    {
-        if (t < s) sh[t] += sh[t + s];
-        __syncthreads();
-    }
-    const double r = sh[0];
-    __syncthreads();
-    return r;
-}
-
-// Called by every thread of every block with the block's partial value (valid in thread 0).  The last
-// block writes op(sum of partials) to *out.  op: 0 = sum, 1 = sqrt(sum).
-__device__ void grid_finish(double part, RedScratch rs, double *out, int op)
-{
-    __shared__ double sh[kRedThreads];
-    __shared__ int last;
-    if (!rs.ticket)
-    {
-        // partials only; k_finish combines them
-        if (threadIdx.x == 0) rs.partial[blockIdx.x] = part;
-        return;
-    }
-    if (threadIdx.x == 0)
-    {
-        rs.partial[blockIdx.x] = part;
-        __threadfence();
-        const unsigned prev = atomicAdd(rs.ticket, 1u);
-        last = prev == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    double v = 0.0;
-    for (int i = threadIdx.x; i < static_cast<int>(gridDim.x); i += kRedThreads)
-        v += __hip_atomic_load(&rs.partial[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    v = block_sum(v, sh);
-    if (threadIdx.x == 0)
-    {
-        *out = op == 1 ? sqrt(v) : v;
-        *rs.ticket = 0u;
-    }
-}
-
-// out = op(sum of the n block partials) in the fixed tree of grid_finish's last block (one block)
-__global__ void __launch_bounds__(kRedThreads) k_finish(const double *partial, int32_t n, double *out, int op)
-{
-    __shared__ double sh[kRedThreads];
-    double v = 0.0;
-    for (int i = threadIdx.x; i < n; i += kRedThreads) v += partial[i];
-    v = block_sum(v, sh);
-    if (threadIdx.x == 0) *out = op == 1 ? sqrt(v) : v;
-}
-
-template <class T>
-__global__ void __launch_bounds__(kRedThreads) k_dot(const T *a, const T *b, int32_t n, RedScratch rs, double *out, int op)
-{
-    __shared__ double sh[kRedThreads];
-    double s = 0.0;
-    for (int32_t i = blockIdx.x * kRedThreads + threadIdx.x; i < n; i += gridDim.x * kRedThreads)
-        s += static_cast<double>(a[i]) * static_cast<double>(b[i]);
-    grid_finish(block_sum(s, sh), rs, out, op);
-}
-template __global__ void k_dot<double>(const double *, const double *, int32_t, RedScratch, double *, int);
-template __global__ void k_dot<float>(const float *, const float *, int32_t, RedScratch, double *, int);
-
-// Modified Gram-Schmidt step i (ImplicitInduction.cpp:341-347): w -= h[i-1] V_{i-1} (i > 0), then
-// h[i] = <w, V_i>; with `norm` set: w -= h[i-1] V_{i-1}, then h[i] = |w|.
-template <class T>
-__global__ void __launch_bounds__(kRedThreads) k_mgs(T *w, const T *Vprev, const T *Vi, int32_t n, double *h, int32_t i, int32_t norm,
-                                                    RedScratch rs)
-{
-    __shared__ double sh[kRedThreads];
-    const double hp = i > 0 ? h[i - 1] : 0.0;
-    double s = 0.0;
-    for (int32_t e = blockIdx.x * kRedThreads + threadIdx.x; e < n; e += gridDim.x * kRedThreads)
-    {
-        double we = static_cast<double>(w[e]);
-        if (i > 0)
-        {
-            we -= hp * static_cast<double>(Vprev[e]);
-            w[e] = static_cast<T>(we);
-            we = static_cast<double>(w[e]);
-        }
-        s += norm ? we * we : we * static_cast<double>(Vi[e]);
-    }
-    grid_finish(block_sum(s, sh), rs, h + i, norm ? 1 : 0);
-}
-template __global__ void k_mgs<double>(double *, const double *, const double *, int32_t, double *, int32_t, int32_t, RedScratch);
-template __global__ void k_mgs<float>(float *, const float *, const float *, int32_t, double *, int32_t, int32_t, RedScratch);
-
-// V_{j+1} = w / h (reference divides, ImplicitInduction.cpp:342)
-template <class T>
-__global__ void __launch_bounds__(256) k_scale_div(const T *w, const double *h, int32_t n, T *out)
-{
-    const int32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    const double hv = h[0];
-    if (e >= n || !(hv > 1e-300)) return;
-    out[e] = static_cast<T>(static_cast<double>(w[e]) / hv);
-}
-template __global__ void k_scale_div<double>(const double *, const double *, int32_t, double *);
-template __global__ void k_scale_div<float>(const float *, const double *, int32_t, float *);
-
 // r / beta into V_0 (ImplicitInduction.cpp:330)
 __global__ void __launch_bounds__(256) k_div_scalar(const double *r, const double *beta, int32_t n, double *out)
 {
@@ -328,19 +217,96 @@ template <int G> __global__ void __launch_bounds__(256) k_hall_g_g(DevMesh d, co
 template __global__ void k_bcell_g<kCellLanes64>(DevMesh, const double *, double *);
 template __global__ void k_hall_g_g<kCellLanes64>(DevMesh, const double *, const double *, const double *, double *);
 
+// The row of the result from the edge's two sums
+__device__ __forceinline__ void edge_apply_out(const DevMesh &d, int32_t e, double p0, double p1, const double *ide, const int8_t *imask,
+                                               const double *v, const double *invdiag, const int8_t *dir, double dt, int32_t mode, int32_t mask,
+                                               const double *bvec, double *out)
+{
+    const double p2 = ide ? (imask[e] ? ide[e] : 0.0) : 0.0;
+    const double F = d.m_e[e] * p0 + p1 + p2;
+    double r;
+    if (mode == 0) r = F;
+    else
+    {
+        const double x = invdiag ? (dir[e] ? 0.0 : v[e] * invdiag[e]) : v[e];
+        r = x + dt * F;
+    }
+    if (mask && dir[e]) r = 0.0;
+    if (bvec) r = dir[e] ? 0.0 : bvec[e] - r; // residual form r = b - A x
+    out[e] = r;
+}
+// sum of n values of LDS in their order, the loads of a group ahead of its additions
+__device__ __forceinline__ double ordered_sum(const double *x, int32_t n)
+{
+    double s = 0.0;
+    int32_t i = 0;
+    for (; i + 8 <= n; i += 8)
+    {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = x[i + u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; i < n; ++i) s += x[i];
+    return s;
+}
+// One high-valence edge per block: terms in parallel into LDS (hv the largest valence of the mesh: hv face terms, then up
+// to 2 hv cell terms), each sum sequential in the reference's order (faces ascending, cells ascending) on a wave of its own.
+__device__ __forceinline__ void edge_apply_heavy(const DevMesh &d, int32_t resistive, int32_t hall, int32_t e, const double *phi, const double *g,
+                                                 const double *ide, const int8_t *imask, const double *v, const double *invdiag,
+                                                 const int8_t *dir, double dt, int32_t mode, int32_t mask, const double *bvec, double *out,
+                                                 double *sh, int32_t hv)
+{
+    __shared__ double tot[2];
+    double *t0 = sh, *t1 = sh + hv;
+    const int32_t f0 = d.e2f_ptr[e], nf = d.e2f_ptr[e + 1] - f0;
+    const int32_t c0 = d.ec_ptr[e], ncl = d.ec_ptr[e + 1] - c0;
+    if (resistive)
+        for (int32_t i = threadIdx.x; i < nf; i += blockDim.x)
+        {
+            const int32_t q = d.e2f[f0 + i], f = pid(q);
+            const double val = d.star2[f] * phi[f];
+            t0[i] = psg(q) * val;
+        }
+    if (hall)
+    {
+        const V3 t = L3(d.evec, e);
+        for (int32_t i = threadIdx.x; i < ncl; i += blockDim.x)
+        {
+            const V3 wt = d.ecw[c0 + i] * t;
+            t1[i] = dot(L3(g, d.ec_cell[c0 + i]), wt);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) tot[0] = resistive ? ordered_sum(t0, nf) : 0.0;
+    if (threadIdx.x == 64) tot[1] = hall ? ordered_sum(t1, ncl) : 0.0;
+    __syncthreads();
+    if (threadIdx.x == 0) edge_apply_out(d, e, tot[0], tot[1], ide, imask, v, invdiag, dir, dt, mode, mask, bvec, out);
+}
+
 // Edge assembly of apply_F (ImplicitInduction.cpp:139-182): part0 = sum_f f2e star2 Phi (faces ascending),
 // part1 = sum_c g_c . (w_ec t_e) (cells ascending), part2 = imask ? ide : 0 (implicit ideal part, ide nullable),
 // F = m part0 + part1 + part2.
 // mode 0: out = F.  mode 1 (apply_A): out = x + dt F with x = dir ? 0 : v*invdiag (invdiag non-null) or v;
 // with `mask` set, Dirichlet rows of the result are zeroed (Arnoldi vector, ImplicitInduction.cpp:340).
+// The first n_heavy blocks take one high-valence edge each (a launch of their own cost 5 to 12 us per product).
 __global__ void __launch_bounds__(256) k_edge_apply(DevMesh d, int32_t resistive, int32_t hall, const double *phi, const double *g,
                                                     const double *ide, const int8_t *imask, const double *v, const double *invdiag,
-                                                    const int8_t *dir, double dt, int32_t mode, int32_t mask, const double *bvec, double *out)
+                                                    const int8_t *dir, double dt, int32_t mode, int32_t mask, const double *bvec, double *out,
+                                                    const int32_t *heavy, int32_t n_heavy, int32_t hv)
 {
-    const int32_t e = gid();
+    extern __shared__ double shared[];
+    const int32_t b = blockIdx.x;
+    if (b < n_heavy)
+    {
+        edge_apply_heavy(d, resistive, hall, heavy[b], phi, g, ide, imask, v, invdiag, dir, dt, mode, mask, bvec, out, shared, hv);
+        return;
+    }
+    const int32_t e = (b - n_heavy) * 256 + int32_t(threadIdx.x);
     if (e >= d.ne) return;
     const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1];
-    if (f1 - f0 > kLightMax) return; // k_edge_apply_heavy
+    if (f1 - f0 > kLightMax) return; // a heavy block's
     double p0 = 0.0, p1 = 0.0;
     // each group's index loads, then its gathers, then the sums in entry order
     if (resistive)
@@ -386,64 +352,7 @@ __global__ void __launch_bounds__(256) k_edge_apply(DevMesh d, int32_t resistive
                 }
         }
     }
-    const double p2 = ide ? (imask[e] ? ide[e] : 0.0) : 0.0;
-    const double F = d.m_e[e] * p0 + p1 + p2;
-    double r;
-    if (mode == 0) r = F;
-    else
-    {
-        const double x = invdiag ? (dir[e] ? 0.0 : v[e] * invdiag[e]) : v[e];
-        r = x + dt * F;
-    }
-    if (mask && dir[e]) r = 0.0;
-    if (bvec) r = dir[e] ? 0.0 : bvec[e] - r; // residual form r = b - A x
-    out[e] = r;
-}
-
-// k_edge_apply for the high-valence edges, one block per edge: terms in parallel into LDS, sums sequential
-// in the reference's order (faces ascending, cells ascending).
-__global__ void __launch_bounds__(256) k_edge_apply_heavy(DevMesh d, int32_t resistive, int32_t hall, const int32_t *heavy, const double *phi,
-                                                          const double *g, const double *ide, const int8_t *imask, const double *v,
-                                                          const double *invdiag, const int8_t *dir, double dt, int32_t mode, int32_t mask,
-                                                          const double *bvec, double *out)
-{
-    __shared__ double t0[kHeavyMax], t1[2 * kHeavyMax];
-    const int32_t e = heavy[blockIdx.x];
-    const int32_t f0 = d.e2f_ptr[e], nf = d.e2f_ptr[e + 1] - f0;
-    const int32_t c0 = d.ec_ptr[e], ncl = d.ec_ptr[e + 1] - c0;
-    if (resistive)
-        for (int32_t i = threadIdx.x; i < nf; i += blockDim.x)
-        {
-            const int32_t q = d.e2f[f0 + i], f = pid(q);
-            const double val = d.star2[f] * phi[f];
-            t0[i] = psg(q) * val;
-        }
-    if (hall)
-    {
-        const V3 t = L3(d.evec, e);
-        for (int32_t i = threadIdx.x; i < ncl; i += blockDim.x)
-        {
-            const V3 wt = d.ecw[c0 + i] * t;
-            t1[i] = dot(L3(g, d.ec_cell[c0 + i]), wt);
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    double p0 = 0.0, p1 = 0.0;
-    if (resistive) for (int32_t i = 0; i < nf; ++i) p0 += t0[i];
-    if (hall) for (int32_t i = 0; i < ncl; ++i) p1 += t1[i];
-    const double p2 = ide ? (imask[e] ? ide[e] : 0.0) : 0.0;
-    const double F = d.m_e[e] * p0 + p1 + p2;
-    double r;
-    if (mode == 0) r = F;
-    else
-    {
-        const double x = invdiag ? (dir[e] ? 0.0 : v[e] * invdiag[e]) : v[e];
-        r = x + dt * F;
-    }
-    if (mask && dir[e]) r = 0.0;
-    if (bvec) r = dir[e] ? 0.0 : bvec[e] - r;
-    out[e] = r;
+    edge_apply_out(d, e, p0, p1, ide, imask, v, invdiag, dir, dt, mode, mask, bvec, out);
 }
 
 // ---------------------------------------------------------------- right-hand side and first residual, fused
@@ -558,14 +467,60 @@ __device__ __forceinline__ void rhs_residual_out(const DevMesh &d, int32_t e, do
     bvec[e] = bv;
     r[e] = rr;
 }
+// One high-valence edge per block, as edge_apply_heavy: four sums, a wave each
+__device__ __forceinline__ void rhs_residual_heavy(const DevMesh &d, int32_t resistive, int32_t hall, int32_t e, const double *phi1,
+                                                   const double *g1, const double *phi2, const double *g2, const double *E_expl, const double *x,
+                                                   const int8_t *dir, double dt, double *bvec, double *r, double *sh, int32_t hv)
+{
+    __shared__ double tot[4];
+    double *t0 = sh, *t1 = sh + 2 * hv; // face terms of both vectors, cell terms of both
+    const int32_t f0 = d.e2f_ptr[e], nf = d.e2f_ptr[e + 1] - f0;
+    const int32_t c0 = d.ec_ptr[e], ncl = d.ec_ptr[e + 1] - c0;
+    if (resistive)
+        for (int32_t i = threadIdx.x; i < nf; i += blockDim.x)
+        {
+            const int32_t q = d.e2f[f0 + i], f = pid(q);
+            const double va = d.star2[f] * phi1[f], vb = d.star2[f] * phi2[f];
+            t0[i] = psg(q) * va;
+            t0[hv + i] = psg(q) * vb;
+        }
+    if (hall)
+    {
+        const V3 t = L3(d.evec, e);
+        for (int32_t i = threadIdx.x; i < ncl; i += blockDim.x)
+        {
+            const V3 wt = d.ecw[c0 + i] * t;
+            const int32_t c = d.ec_cell[c0 + i];
+            t1[i] = dot(L3(g1, c), wt);
+            t1[2 * hv + i] = dot(L3(g2, c), wt);
+        }
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0)
+    {
+        const int32_t k = threadIdx.x >> 6; // face sum and cell sum of the first vector, then of the second
+        const bool cells = k & 1;
+        tot[k] = cells ? (hall ? ordered_sum(t1 + (k >> 1) * 2 * hv, ncl) : 0.0) : (resistive ? ordered_sum(t0 + (k >> 1) * hv, nf) : 0.0);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) rhs_residual_out(d, e, tot[0], tot[1], tot[2], tot[3], E_expl, x, dir, dt, bvec, r);
+}
 __global__ void __launch_bounds__(256) k_edge_rhs_residual(DevMesh d, int32_t resistive, int32_t hall, const double *phi1, const double *g1,
                                                            const double *phi2, const double *g2, const double *E_expl, const double *x,
-                                                           const int8_t *dir, double dt, double *bvec, double *r)
+                                                           const int8_t *dir, double dt, double *bvec, double *r, const int32_t *heavy,
+                                                           int32_t n_heavy, int32_t hv)
 {
-    const int32_t e = gid();
+    extern __shared__ double shared[];
+    const int32_t b = blockIdx.x;
+    if (b < n_heavy)
+    {
+        rhs_residual_heavy(d, resistive, hall, heavy[b], phi1, g1, phi2, g2, E_expl, x, dir, dt, bvec, r, shared, hv);
+        return;
+    }
+    const int32_t e = (b - n_heavy) * 256 + int32_t(threadIdx.x);
     if (e >= d.ne) return;
     const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1];
-    if (f1 - f0 > kLightMax) return; // k_edge_rhs_residual_heavy
+    if (f1 - f0 > kLightMax) return; // a heavy block's
     double p0[2] = {0.0, 0.0}, p1[2] = {0.0, 0.0};
     if (resistive)
         for (int32_t k = f0; k < f1; k += kEdgeUnroll)
@@ -614,67 +569,36 @@ __global__ void __launch_bounds__(256) k_edge_rhs_residual(DevMesh d, int32_t re
     }
     rhs_residual_out(d, e, p0[0], p1[0], p0[1], p1[1], E_expl, x, dir, dt, bvec, r);
 }
-// the high-valence edges, one block per edge (terms in parallel into LDS, sums sequential, as k_edge_apply_heavy)
-__global__ void __launch_bounds__(256) k_edge_rhs_residual_heavy(DevMesh d, int32_t resistive, int32_t hall, const int32_t *heavy,
-                                                                 const double *phi1, const double *g1, const double *phi2, const double *g2,
-                                                                 const double *E_expl, const double *x, const int8_t *dir, double dt,
-                                                                 double *bvec, double *r)
-{
-    __shared__ double t0[2][kHeavyMax], t1[2][2 * kHeavyMax];
-    const int32_t e = heavy[blockIdx.x];
-    const int32_t f0 = d.e2f_ptr[e], nf = d.e2f_ptr[e + 1] - f0;
-    const int32_t c0 = d.ec_ptr[e], ncl = d.ec_ptr[e + 1] - c0;
-    if (resistive)
-        for (int32_t i = threadIdx.x; i < nf; i += blockDim.x)
-        {
-            const int32_t q = d.e2f[f0 + i], f = pid(q);
-            const double va = d.star2[f] * phi1[f], vb = d.star2[f] * phi2[f];
-            t0[0][i] = psg(q) * va;
-            t0[1][i] = psg(q) * vb;
-        }
-    if (hall)
-    {
-        const V3 t = L3(d.evec, e);
-        for (int32_t i = threadIdx.x; i < ncl; i += blockDim.x)
-        {
-            const V3 wt = d.ecw[c0 + i] * t;
-            const int32_t c = d.ec_cell[c0 + i];
-            t1[0][i] = dot(L3(g1, c), wt);
-            t1[1][i] = dot(L3(g2, c), wt);
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    double p0[2] = {0.0, 0.0}, p1[2] = {0.0, 0.0};
-    for (int n = 0; n < 2; ++n)
-    {
-        if (resistive) for (int32_t i = 0; i < nf; ++i) p0[n] += t0[n][i];
-        if (hall) for (int32_t i = 0; i < ncl; ++i) p1[n] += t1[n][i];
-    }
-    rhs_residual_out(d, e, p0[0], p1[0], p0[1], p1[1], E_expl, x, dir, dt, bvec, r);
-}
-
-// delta += dir ? 0 : (sum_i y_i V_i) * invdiag  (ImplicitInduction.cpp:366-376)
-__global__ void __launch_bounds__(256) k_gmres_update(const double *const *V, const double *y, int32_t j, const double *invdiag,
-                                                      const int8_t *dir, int32_t n, double *delta)
-{
-    const int32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    double s = 0.0;
-    for (int32_t i = 0; i < j; ++i) s += y[i] * V[i][e];
-    delta[e] += dir[e] ? 0.0 : s * invdiag[e];
-}
 
 // elementwise helpers of solve()
+// B0 = B (nullable) and alpha_c B_c in FP32, formed in FP64 (nullable): the FP32 Hall kernel reads one 3-vector per cell
+// instead of alpha and B0
+__global__ void __launch_bounds__(256) k_freeze(const double *alpha, const double *B, int32_t nc, double *B0, float *aB0)
+{
+    const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= nc) return;
+    const double a = aB0 ? alpha[c] : 0.0;
+    for (int k = 0; k < 3; ++k)
+    {
+        const double b = B[3 * size_t(c) + k];
+        if (B0) B0[3 * size_t(c) + k] = b;
+        if (aB0) aB0[3 * size_t(c) + k] = static_cast<float>(a * b);
+    }
+}
+// x0 = E_expl + the warm start, the Jacobi diagonal (and its FP32 copy, inv32 nullable), delta = 0
 __global__ void __launch_bounds__(256) k_solve_init(const double *E_expl, const double *corr, const int8_t *dir, const double *m_e,
-                                                    const double *d2, double dt, const double *dte, int32_t n, double *x0, double *invdiag)
+                                                    const double *d2, double dt, const double *dte, int32_t n, double *x0, double *invdiag,
+                                                    float *inv32, double *delta)
 {
     const int32_t e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
     double x = E_expl[e];
     if (corr && !dir[e]) x += corr[e];
     x0[e] = x;
-    invdiag[e] = 1.0 / (1.0 + (dte ? dte[e] : dt) * m_e[e] * d2[e]);
+    const double iv = 1.0 / (1.0 + (dte ? dte[e] : dt) * m_e[e] * d2[e]);
+    invdiag[e] = iv;
+    if (inv32) inv32[e] = static_cast<float>(iv);
+    delta[e] = 0.0;
 }
 __global__ void __launch_bounds__(256) k_add(const double *a, const double *b, int32_t n, double *out)
 {

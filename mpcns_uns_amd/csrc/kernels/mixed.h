@@ -37,8 +37,6 @@ struct DevMesh32
 };
 
 constexpr int kEdgeBlock = 256; // threads per block of the FP32 edge kernel (a multiple of 64: whole slices)
-constexpr int kDotChunk = 16; // basis vectors per multi-dot pass
-constexpr int kOrthoBlocks = 1024; // grid of the FP32 orthogonalisation kernels (512 and 2048 measured no better)
 
 __global__ void k_d1_f32(DevMesh d, DevMesh32 s, const float *pv, const float *dte, float *phi);
 constexpr int kCellLanes = 4; // lanes per cell of the FP32 cell kernels
@@ -50,15 +48,10 @@ __global__ void k_edge_apply_f32(DevMesh d, DevMesh32 s, int32_t resistive, int3
                                  const float *pv, const int8_t *dir, float dt, float *out, const int32_t *heavy, int32_t n_light, const float *b,
                                  float omega);
 __global__ void k_tables_f32(DevMesh d, float *aV, int32_t *nbr);
-__global__ void k_multiaxpy_f32(const float *const *V, int32_t nv, const double *h, float *w, int32_t n, RedScratch rs, double *nrm);
 __global__ void k_to_f32_scaled(const double *x, const double *s, const float *invdiag, const int8_t *dir, int32_t n, float *out, float *pv);
-__global__ void k_scale_f32(const float *w, const double *h, const float *invdiag, const int8_t *dir, int32_t n, float *out, float *pv);
-__global__ void k_update_mixed(const float *const *V, const double *y, int32_t j, const float *invdiag, const int8_t *dir, int32_t n,
-                               double *delta);
 __global__ void k_f64_to_f32(const double *x, int64_t n, float *out);
-__global__ void k_alpha_f32(const double *alpha, const double *B0, int32_t nc, float *aB0);
 // multigrid.hip
-__global__ void k_update_flex(const float *const *Z, const double *y, int32_t j, const int8_t *dir, int32_t n, double *delta);
+__global__ void k_update_flex(const float *const *Z, Coefs y, int32_t j, const int8_t *dir, int32_t n, const double *x0, double *delta, double *x);
 
 struct MgDevice; // multigrid.hip
 
@@ -68,7 +61,6 @@ struct MixedSolver
     float *phi = nullptr, *b = nullptr, *g = nullptr, *w = nullptr, *dte32 = nullptr, *pv = nullptr;
     std::vector<float *> V, Z;      // Krylov basis; Z_j = M V_j of the flexible (multigrid) inner solve
     float **Vptrs = nullptr, **Zptrs = nullptr;
-    double *h = nullptr, *part = nullptr, *part_axpy = nullptr;
     int m = 30;
     bool built = false;
 };

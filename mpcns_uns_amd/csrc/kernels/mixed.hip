@@ -26,15 +26,8 @@ __device__ __forceinline__ F3 f3(const float *p, long i) { return {p[3 * i], p[3
 __device__ __forceinline__ F3 fcross(const F3 &a, const F3 &b) { return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
 __device__ __forceinline__ float fdot(const F3 &a, const F3 &b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 __device__ __forceinline__ float fsg(int32_t v) { return v >= 0 ? 1.0f : -1.0f; }
-// a float4 load through a pointer known to be global memory (a pointer read from LDS or an array is generic, and its
-// loads become flat loads that also count against the LDS wait counter)
-typedef float F4v __attribute__((ext_vector_type(4)));
-typedef const __attribute__((address_space(1))) F4v *GlobalF4;
-__device__ __forceinline__ float4 ldg4(const float *p, int32_t q)
-{
-    const F4v v = ((GlobalF4)p)[q];
-    return make_float4(v.x, v.y, v.z, v.w);
-}
+// loads through pointers known to be global memory (a pointer read from an array is generic, and its loads become flat
+// loads that also count against the LDS wait counter)
 typedef int I4v __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) I4v *GlobalI4;
 typedef const __attribute__((address_space(1))) int32_t *GlobalI32;
@@ -52,12 +45,6 @@ __device__ __forceinline__ int3 ld_compact(const int32_t *words, int32_t w, int3
 {
     const GlobalI32 p = (GlobalI32)words + w;
     return make_int3(p[0] & mask, p[1] & mask, p[2] & mask);
-}
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
 }
 } // namespace
 
@@ -401,310 +388,6 @@ __global__ void __launch_bounds__(256) k_tables_f32(DevMesh d, float *aV, int32_
     }
 }
 
-// h[i0+k] = <w, V_{i0+k}> for k < NV (FP64 accumulation, 4 elements per thread and iteration); with_ww
-// also <w, w> into out[63].  NV is a template argument so that the NV loads of an iteration are issued together (a
-// run-time count guarded each load by a branch and kept one load in flight per thread).
-template <int NV>
-__global__ void __launch_bounds__(256) k_multidot_f32(const float *const *V, int32_t i0, const float *w, int32_t n, double *part,
-                                                      int32_t with_ww, RedScratch rs, double *out)
-{
-    __shared__ double sh[4][kDotChunk + 1];
-    __shared__ int last;
-    double acc[kDotChunk + 1];
-#pragma unroll
-    for (int k = 0; k <= kDotChunk; ++k) acc[k] = 0.0;
-    const float *Vk[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) Vk[k] = V[i0 + k];
-    const int32_t n4 = n >> 2;
-    for (int32_t q = blockIdx.x * 256 + threadIdx.x; q < n4; q += gridDim.x * 256)
-    {
-        const float4 a = ldg4(w, q);
-        float4 b[NV];
-#pragma unroll
-        for (int k = 0; k < NV; ++k) b[k] = ldg4(Vk[k], q);
-#pragma unroll
-        for (int k = 0; k < NV; ++k)
-            acc[k] += (double(a.x) * b[k].x + double(a.y) * b[k].y) + (double(a.z) * b[k].z + double(a.w) * b[k].w);
-        acc[kDotChunk] += (double(a.x) * a.x + double(a.y) * a.y) + (double(a.z) * a.z + double(a.w) * a.w);
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3))
-    {
-        const int32_t e = 4 * n4 + threadIdx.x;
-        const double a = w[e];
-#pragma unroll
-        for (int k = 0; k < NV; ++k) acc[k] += a * Vk[k][e];
-        acc[kDotChunk] += a * a;
-    }
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k <= kDotChunk; ++k)
-        if (k < NV || k == kDotChunk)
-        {
-            const double sm = wave_sum(acc[k]);
-            if (lane == 0) sh[wv][k] = sm;
-        }
-    __syncthreads();
-    if (threadIdx.x < NV || threadIdx.x == kDotChunk)
-    {
-        const int k = threadIdx.x;
-        part[size_t(blockIdx.x) * (kDotChunk + 1) + k] = ((sh[0][k] + sh[1][k]) + sh[2][k]) + sh[3][k];
-    }
-    if (!rs.ticket) return; // partials only: k_multidot_final sums them
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(rs.ticket, 1u) == gridDim.x - 1;
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    double t[kDotChunk + 1];
-#pragma unroll
-    for (int k = 0; k <= kDotChunk; ++k) t[k] = 0.0;
-    for (uint32_t bl = threadIdx.x; bl < gridDim.x; bl += 256)
-#pragma unroll
-        for (int k = 0; k <= kDotChunk; ++k)
-            if (k < NV || k == kDotChunk)
-                t[k] += __hip_atomic_load(&part[size_t(bl) * (kDotChunk + 1) + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int k = 0; k <= kDotChunk; ++k)
-        if (k < NV || k == kDotChunk)
-        {
-            const double s2 = wave_sum(t[k]);
-            if (lane == 0) sh[wv][k] = s2;
-        }
-    __syncthreads();
-    if (threadIdx.x < NV || threadIdx.x == kDotChunk)
-    {
-        const int k = threadIdx.x;
-        const double s2 = ((sh[0][k] + sh[1][k]) + sh[2][k]) + sh[3][k];
-        if (k < NV) out[i0 + k] = s2;
-        if (k == kDotChunk && with_ww) out[63] = s2;
-    }
-    if (threadIdx.x == 0) *rs.ticket = 0u;
-}
-using MultidotFn = void (*)(const float *const *, int32_t, const float *, int32_t, double *, int32_t, RedScratch, double *);
-template <int... I> constexpr std::array<MultidotFn, sizeof...(I) + 1> multidot_table(std::integer_sequence<int, I...>)
-{
-    return {nullptr, &k_multidot_f32<I + 1>...};
-}
-// kMultidot[nv]: the multi-dot pass over nv basis vectors, 1 <= nv <= kDotChunk
-const std::array<MultidotFn, kDotChunk + 1> kMultidot = multidot_table(std::make_integer_sequence<int, kDotChunk>{});
-
-// x -= h_i V_i for the G vectors from i0 on, in order (their G loads issued together)
-template <int G>
-__device__ __forceinline__ void axpy_group(const float *const *vp, const double *hs, int32_t i0, int32_t q, double &x, double &y, double &z,
-                                           double &u)
-{
-    float4 b[G];
-#pragma unroll
-    for (int k = 0; k < G; ++k) b[k] = ldg4(vp[i0 + k], q);
-#pragma unroll
-    for (int k = 0; k < G; ++k)
-    {
-        const double hi = hs[i0 + k];
-        x -= hi * b[k].x; y -= hi * b[k].y; z -= hi * b[k].z; u -= hi * b[k].w;
-    }
-}
-constexpr int kAxpyGroup = 8;
-// x -= sum_{i < nv} h_i V_i in order of i: groups of kAxpyGroup loads, then the remainder's loads together
-__device__ __forceinline__ void axpy_all(const float *const *vp, const double *hs, int32_t nv, int32_t q, double &x, double &y, double &z,
-                                         double &u)
-{
-    int32_t i = 0;
-    for (; i + kAxpyGroup <= nv; i += kAxpyGroup) axpy_group<kAxpyGroup>(vp, hs, i, q, x, y, z, u);
-    switch (nv - i)
-    {
-    case 7: axpy_group<7>(vp, hs, i, q, x, y, z, u); break;
-    case 6: axpy_group<6>(vp, hs, i, q, x, y, z, u); break;
-    case 5: axpy_group<5>(vp, hs, i, q, x, y, z, u); break;
-    case 4: axpy_group<4>(vp, hs, i, q, x, y, z, u); break;
-    case 3: axpy_group<3>(vp, hs, i, q, x, y, z, u); break;
-    case 2: axpy_group<2>(vp, hs, i, q, x, y, z, u); break;
-    case 1: axpy_group<1>(vp, hs, i, q, x, y, z, u); break;
-    default: break;
-    }
-}
-
-// w -= sum_{i < nv} h_i V_i (FP64 arithmetic, FP32 storage, 4 elements per thread); nrm[0] = |w| after
-__global__ void __launch_bounds__(256) k_multiaxpy_f32(const float *const *V, int32_t nv, const double *h, float *w, int32_t n,
-                                                       RedScratch rs, double *nrm)
-{
-    __shared__ double sh[4];
-    __shared__ int last;
-    __shared__ double hs[64];
-    __shared__ const float *vp[64];
-    if (threadIdx.x < nv) { hs[threadIdx.x] = h[threadIdx.x]; vp[threadIdx.x] = V[threadIdx.x]; }
-    __syncthreads();
-    double acc = 0.0;
-    const int32_t n4 = n >> 2;
-    float4 *w4 = reinterpret_cast<float4 *>(w);
-    for (int32_t q = blockIdx.x * 256 + threadIdx.x; q < n4; q += gridDim.x * 256)
-    {
-        const float4 a = w4[q];
-        double x = a.x, y = a.y, z = a.z, u = a.w;
-        axpy_all(vp, hs, nv, q, x, y, z, u);
-        const float4 r = make_float4(float(x), float(y), float(z), float(u));
-        w4[q] = r;
-        acc += (double(r.x) * r.x + double(r.y) * r.y) + (double(r.z) * r.z + double(r.w) * r.w);
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3))
-    {
-        const int32_t e = 4 * n4 + threadIdx.x;
-        double we = w[e];
-        for (int32_t i = 0; i < nv; ++i) we -= hs[i] * static_cast<double>(vp[i][e]);
-        const float wf = static_cast<float>(we);
-        w[e] = wf;
-        acc += double(wf) * wf;
-    }
-    const double s = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        rs.partial[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
-        __threadfence();
-        last = atomicAdd(rs.ticket, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    double t = 0.0;
-    for (uint32_t bl = threadIdx.x; bl < gridDim.x; bl += 256)
-        t += __hip_atomic_load(&rs.partial[bl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const double s2 = wave_sum(t);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s2;
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        nrm[0] = sqrt(((sh[0] + sh[1]) + sh[2]) + sh[3]);
-        *rs.ticket = 0u;
-    }
-}
-
-// out[i0 + k] (k < nv) and out[63] (with_ww) from the per-block partials of k_multidot_f32 (one block)
-__global__ void __launch_bounds__(256) k_multidot_final(const double *part, int32_t nblocks, int32_t i0, int32_t nv, int32_t with_ww,
-                                                        double *out)
-{
-    __shared__ double sh[4][kDotChunk + 1];
-    double t[kDotChunk + 1];
-#pragma unroll
-    for (int k = 0; k <= kDotChunk; ++k) t[k] = 0.0;
-    for (int32_t bl = threadIdx.x; bl < nblocks; bl += 256)
-#pragma unroll
-        for (int k = 0; k <= kDotChunk; ++k) t[k] += part[size_t(bl) * (kDotChunk + 1) + k];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k <= kDotChunk; ++k)
-    {
-        const double s = wave_sum(t[k]);
-        if (lane == 0) sh[wv][k] = s;
-    }
-    __syncthreads();
-    if (threadIdx.x <= kDotChunk)
-    {
-        const int k = threadIdx.x;
-        const double s = ((sh[0][k] + sh[1][k]) + sh[2][k]) + sh[3][k];
-        if (k < nv) out[i0 + k] = s;
-        if (k == kDotChunk && with_ww) out[63] = s;
-    }
-}
-
-// Classical Gram-Schmidt update fused with the normalisation: with h[0..nv) = <w, V_i> and h[63] = <w, w> from the
-// multi-dot pass, hn = sqrt(<w,w> - sum h_i^2) (Pythagoras, FP64) is the norm of w' = w - sum h_i V_i.  When
-// hn >= dgks |w| the kernel writes V_nv = w' / hn and pv = dir ? 0 : V_nv invdiag directly and h[nv] = hn; else
-// (severe cancellation: a second projection follows) it writes w' into w and h[nv] = |w'| computed from w'.
-// h[62] = 1 in the second case, 0 in the first.  Every block takes the same branch (same h).
-__global__ void __launch_bounds__(256) k_multiaxpy_scale_f32(const float *const *V, int32_t nv, double *h, float *w, int32_t n, double dgks,
-                                                             const float *invdiag, const int8_t *dir, float *vnext, float *pv, RedScratch rs)
-{
-    __shared__ double sh[4];
-    __shared__ int last;
-    __shared__ double hs[64];
-    __shared__ const float *vp[64];
-    if (threadIdx.x < nv) { hs[threadIdx.x] = h[threadIdx.x]; vp[threadIdx.x] = V[threadIdx.x]; }
-    __syncthreads();
-    double ss = 0.0;
-    for (int32_t i = 0; i < nv; ++i) ss += hs[i] * hs[i];
-    const double ww = h[63];
-    const double hn2 = ww - ss;
-    const double hp = hn2 > 0 ? sqrt(hn2) : 0.0;
-    const bool direct = hp >= dgks * sqrt(ww > 0 ? ww : 0.0) && hp > 1e-300;
-    const double inv = direct ? 1.0 / hp : 0.0;
-    double acc = 0.0;
-    const int32_t n4 = n >> 2;
-    float4 *w4 = reinterpret_cast<float4 *>(w);
-    for (int32_t q = blockIdx.x * 256 + threadIdx.x; q < n4; q += gridDim.x * 256)
-    {
-        const float4 a = w4[q];
-        double x = a.x, y = a.y, z = a.z, u = a.w;
-        axpy_all(vp, hs, nv, q, x, y, z, u);
-        if (direct)
-        {
-            const float4 v = make_float4(float(x * inv), float(y * inv), float(z * inv), float(u * inv));
-            reinterpret_cast<float4 *>(vnext)[q] = v;
-            const float4 iv = reinterpret_cast<const float4 *>(invdiag)[q];
-            const int32_t e = 4 * q;
-            reinterpret_cast<float4 *>(pv)[q] = make_float4(dir[e] ? 0.0f : v.x * iv.x, dir[e + 1] ? 0.0f : v.y * iv.y,
-                                                            dir[e + 2] ? 0.0f : v.z * iv.z, dir[e + 3] ? 0.0f : v.w * iv.w);
-        }
-        else
-        {
-            const float4 r = make_float4(float(x), float(y), float(z), float(u));
-            w4[q] = r;
-            acc += (double(r.x) * r.x + double(r.y) * r.y) + (double(r.z) * r.z + double(r.w) * r.w);
-        }
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3))
-    {
-        const int32_t e = 4 * n4 + threadIdx.x;
-        double we = w[e];
-        for (int32_t i = 0; i < nv; ++i) we -= hs[i] * static_cast<double>(vp[i][e]);
-        if (direct)
-        {
-            const float v = static_cast<float>(we * inv);
-            vnext[e] = v;
-            pv[e] = dir[e] ? 0.0f : v * invdiag[e];
-        }
-        else
-        {
-            const float wf = static_cast<float>(we);
-            w[e] = wf;
-            acc += double(wf) * wf;
-        }
-    }
-    if (direct)
-    {
-        if (blockIdx.x == 0 && threadIdx.x == 0) { h[nv] = hp; h[62] = 0.0; }
-        return;
-    }
-    const double s = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        rs.partial[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
-        __threadfence();
-        last = atomicAdd(rs.ticket, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    double t = 0.0;
-    for (uint32_t bl = threadIdx.x; bl < gridDim.x; bl += 256)
-        t += __hip_atomic_load(&rs.partial[bl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const double s2 = wave_sum(t);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s2;
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        h[nv] = sqrt(((sh[0] + sh[1]) + sh[2]) + sh[3]);
-        h[62] = 1.0;
-        *rs.ticket = 0u;
-    }
-}
-
 // V_0 = r / beta in FP32 and its preconditioned copy pv = dir ? 0 : V_0 invdiag
 __global__ void __launch_bounds__(256) k_to_f32_scaled(const double *x, const double *s, const float *invdiag, const int8_t *dir, int32_t n,
                                                        float *out, float *pv)
@@ -714,47 +397,6 @@ __global__ void __launch_bounds__(256) k_to_f32_scaled(const double *x, const do
     const float v = static_cast<float>(x[e] / s[0]);
     out[e] = v;
     pv[e] = dir[e] ? 0.0f : v * invdiag[e];
-}
-// V_{j+1} = w / h and pv = dir ? 0 : V_{j+1} invdiag
-__global__ void __launch_bounds__(256) k_scale_f32(const float *w, const double *h, const float *invdiag, const int8_t *dir, int32_t n,
-                                                   float *out, float *pv)
-{
-    const int32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    const double hv = h[0];
-    if (e >= n || !(hv > 1e-300)) return;
-    const float v = static_cast<float>(static_cast<double>(w[e]) / hv);
-    out[e] = v;
-    pv[e] = dir[e] ? 0.0f : v * invdiag[e];
-}
-// delta += P sum_{i < j} y_i V_i on the non-Dirichlet edges, four edges per thread (the grid covers n / 4 + 1
-// threads), the sum in order of i with the loads of a group of vectors issued together
-__global__ void __launch_bounds__(256) k_update_mixed(const float *const *V, const double *y, int32_t j, const float *invdiag,
-                                                      const int8_t *dir, int32_t n, double *delta)
-{
-    __shared__ double ny[64];
-    __shared__ const float *vp[64];
-    if (threadIdx.x < j) { ny[threadIdx.x] = -y[threadIdx.x]; vp[threadIdx.x] = V[threadIdx.x]; }
-    __syncthreads();
-    const int32_t q = blockIdx.x * blockDim.x + threadIdx.x, n4 = n >> 2;
-    if (q < n4)
-    {
-        // s - (-y_i) v = s + y_i v exactly
-        double s[4] = {0.0, 0.0, 0.0, 0.0};
-        axpy_all(vp, ny, j, q, s[0], s[1], s[2], s[3]);
-        const float4 iv = ldg4(invdiag, q);
-        const float ivs[4] = {iv.x, iv.y, iv.z, iv.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (!dir[4 * q + k]) delta[4 * q + k] += s[k] * static_cast<double>(ivs[k]);
-    }
-    else if (q == n4)
-        for (int32_t e = 4 * n4; e < n; ++e)
-        {
-            if (dir[e]) continue;
-            double s = 0.0;
-            for (int32_t i = 0; i < j; ++i) s += y[i] * static_cast<double>(vp[i][e]);
-            delta[e] += s * static_cast<double>(invdiag[e]);
-        }
 }
 // Slices of the edge kernel's rows (DevMesh32::fdesc/fwords, cdesc/cwords).  Per 64-edge slice: the pairs per
 // edge its longest light row needs and the smallest and largest id in its light rows ({pairs, min, max, 0}; a slice
@@ -853,13 +495,6 @@ __global__ void __launch_bounds__(256) k_f64_to_f32(const double *x, int64_t n, 
 {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) out[i] = static_cast<float>(x[i]);
-}
-// alpha_c B0_c in FP32 (formed in FP64): the FP32 Hall kernel reads one 3-vector per cell instead of alpha and B0
-__global__ void __launch_bounds__(256) k_alpha_f32(const double *alpha, const double *B0, int32_t nc, float *aB0)
-{
-    const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nc) return;
-    for (int k = 0; k < 3; ++k) aB0[3 * size_t(c) + k] = static_cast<float>(alpha[c] * B0[3 * size_t(c) + k]);
 }
 } // namespace mhdg
 
@@ -991,10 +626,6 @@ void mhdg_ctx::mixed_build()
     for (auto &v : M.V) v = static_cast<float *>(alloc(E * sizeof(float)));
     M.Vptrs = static_cast<float **>(alloc(sizeof(float *) * M.V.size()));
     chk(hipMemcpy(M.Vptrs, M.V.data(), sizeof(float *) * M.V.size(), hipMemcpyHostToDevice), "upload");
-    M.h = static_cast<double *>(alloc(64 * sizeof(double)));
-    // partial rows of the multi-dot: kOrthoBlocks in the main pass, kRedBlocks in the DGKS re-projection
-    M.part = static_cast<double *>(alloc(size_t(std::max(kOrthoBlocks, kRedBlocks)) * (kDotChunk + 1) * sizeof(double)));
-    M.part_axpy = static_cast<double *>(alloc(size_t(kOrthoBlocks) * sizeof(double)));
     chk(hipStreamSynchronize(stream), "sync");
     M.built = true;
 }
@@ -1024,10 +655,9 @@ int mhdg_ctx::solve_mixed(const double *Phi_n, const double *Eex, const int8_t *
         dte32 = M.dte32;
     }
     // frozen state and Jacobi diagonal in FP32
-    LAUNCH("alpha_f32", k_alpha_f32, dim3(nb(nc)), dim3(256), 0, stream, alpha, B0, nc, M.s.aB0);
+    freeze(M.s.aB0);
     LAUNCH("solve_init", k_solve_init, dim3(nb(ne)), dim3(256), 0, stream, Eex, have_corr ? corr : nullptr, dir, d.m_e, d.d2, dt, dte_cur, ne, x0,
-           invdiag);
-    LAUNCH("f64_to_f32", k_f64_to_f32, dim3(nb(ne)), dim3(256), 0, stream, invdiag, int64_t(ne), const_cast<float *>(M.s.invdiag));
+           invdiag, const_cast<float *>(M.s.invdiag), delta);
     if (use_mg)
     {
         mg_set_solve(dir, static_cast<float>(dt));
@@ -1035,14 +665,12 @@ int mhdg_ctx::solve_mixed(const double *Phi_n, const double *Eex, const int8_t *
     }
     // b = E_expl + F(Phi^n) and the first cycle's residual b - A x0, in one pass
     rhs_residual(Phi_n, Eex, x0, dir, dt);
-    chk(hipMemsetAsync(delta, 0, size_t(ne) * 8, stream), "memset");
-    const double bb = dot(bvec, bvec, 0, 0);
-    const double bnorm = std::sqrt(std::max(bb, 1e-300));
+    const double *nn = norms(rvec, bvec);
+    const double bnorm = std::sqrt(std::max(nn[1], 1e-300));
+    double beta = std::sqrt(nn[0]);
     const float dtf = dte32 ? 1.0f : static_cast<float>(dt); // with dt_e, d1 carries the step
     int total = 0;
-    double beta = 0;
-    std::vector<std::vector<double>> H(m + 1, std::vector<double>(m, 0.0));
-    std::vector<double> cs(m), sn(m), g(m + 1), yv(m), hc(64), c2(64);
+    Hessenberg hs(m);
     const float *const *Vp = M.Vptrs;
     // MHDG_SOLVE_TRACE=1: one stderr line per refinement cycle (FP64 residual, inner iterations, inner estimate)
     static const bool trace = std::getenv("MHDG_SOLVE_TRACE") && std::getenv("MHDG_SOLVE_TRACE")[0] == '1';
@@ -1050,21 +678,19 @@ int mhdg_ctx::solve_mixed(const double *Phi_n, const double *Eex, const int8_t *
     double est = 0;
     for (int outer = 0; outer < 200; ++outer)
     {
-        // FP64 residual of x0 + delta (delta = 0 in the first cycle: rhs_residual formed it)
+        // FP64 residual of x0 + delta (delta = 0 in the first cycle: rhs_residual formed it; the update left the sum in tmp)
         if (outer > 0)
         {
-            LAUNCH("axpy", k_add, dim3(nb(ne)), dim3(256), 0, stream, x0, delta, ne, tmp);
             apply_op(nullptr, tmp, nullptr, dir, dt, 1, 0, bvec, rvec);
+            beta = std::sqrt(norms(rvec, nullptr)[0]);
         }
-        beta = dot(rvec, rvec, 1, 1);
         if (trace)
             std::fprintf(stderr, "[mixed] cycle %d: residual %.3e |b|, previous cycle %d iterations, inner estimate %.3e |b|\n", outer,
                          beta / bnorm, total - cycle_start, est / bnorm);
         cycle_start = total;
         if (!(beta > rtol * bnorm) || total >= max_it) break;
-        LAUNCH("scale", k_to_f32_scaled, dim3(nb(ne)), dim3(256), 0, stream, rvec, scal + 1, M.s.invdiag, dir, ne, M.V[0], M.pv);
-        std::fill(g.begin(), g.end(), 0.0);
-        g[0] = beta;
+        LAUNCH("scale", k_to_f32_scaled, dim3(nb(ne)), dim3(256), 0, stream, rvec, scal, M.s.invdiag, dir, ne, M.V[0], M.pv);
+        hs.start(beta);
         const double stop = std::max(inner_rtol * beta, kStopFloor * rtol * bnorm);
         int j = 0;
         for (; j < m && total < max_it; ++j, ++total)
@@ -1089,60 +715,25 @@ int mhdg_ctx::solve_mixed(const double *Phi_n, const double *Eex, const int8_t *
                        int32_t(op_res), int32_t(op_hall), M.phi, M.g, M.V[j], M.pv, dir, dtf, M.w, static_cast<const int32_t *>(heavy), n_light,
                        static_cast<const float *>(nullptr), 0.0f);
             }
-            // classical Gram-Schmidt against V_0..V_j; the update also normalises V_{j+1} unless the DGKS test asks
-            // for a second projection
-            for (int i0 = 0; i0 <= j; i0 += kDotChunk)
-            {
-                const int nv = std::min(kDotChunk, j + 1 - i0);
-                LAUNCH("multidot", kMultidot[nv], dim3(kOrthoBlocks), dim3(256), 0, stream, Vp, i0, M.w, ne, M.part, i0 == 0 ? 1 : 0,
-                       RedScratch{nullptr, nullptr}, M.h);
-                LAUNCH("multidot_final", k_multidot_final, dim3(1), dim3(256), 0, stream, static_cast<const double *>(M.part), kOrthoBlocks,
-                       i0, nv, i0 == 0 ? 1 : 0, M.h);
-            }
-            LAUNCH("multiaxpy", k_multiaxpy_scale_f32, dim3(kOrthoBlocks), dim3(256), 0, stream, Vp, j + 1, M.h, M.w, ne, double(kDgks),
-                   M.s.invdiag, dir, M.V[j + 1], M.pv, RedScratch{M.part_axpy, rs.ticket});
-            d2h(hc.data(), M.h, sizeof(double) * 64);
-            double hn = hc[j + 1];
-            if (hc[62] != 0.0)
-            {
-                // DGKS: one more projection
-                for (int i0 = 0; i0 <= j; i0 += kDotChunk)
-                    LAUNCH("multidot", kMultidot[std::min(kDotChunk, j + 1 - i0)], dim3(kRedBlocks), dim3(256), 0, stream, Vp, i0, M.w,
-                           ne, M.part, 0, rs, M.h);
-                LAUNCH("multiaxpy", k_multiaxpy_f32, dim3(kRedBlocks), dim3(256), 0, stream, Vp, j + 1, M.h, M.w, ne, rs, M.h + j + 1);
-                d2h(c2.data(), M.h, sizeof(double) * 64);
-                for (int i = 0; i <= j; ++i) hc[i] += c2[i];
-                hn = c2[j + 1];
-                chk(hipMemcpyAsync(M.h + j + 1, &hn, 8, hipMemcpyHostToDevice, stream), "H2D");
-                LAUNCH("scale", k_scale_f32, dim3(nb(ne)), dim3(256), 0, stream, M.w, M.h + j + 1, M.s.invdiag, dir, ne, M.V[j + 1], M.pv);
-            }
-            for (int i = 0; i <= j; ++i) H[i][j] = hc[i];
-            if (!use_mg) H[j][j] += 1.0; // Arnoldi ran on A P - I
-            H[j + 1][j] = hn;
-            for (int i = 0; i < j; ++i)
-            {
-                const double tt = cs[i] * H[i][j] + sn[i] * H[i + 1][j];
-                H[i + 1][j] = -sn[i] * H[i][j] + cs[i] * H[i + 1][j];
-                H[i][j] = tt;
-            }
-            const double den = std::hypot(H[j][j], H[j + 1][j]);
-            cs[j] = den > 0 ? H[j][j] / den : 1.0; sn[j] = den > 0 ? H[j + 1][j] / den : 0.0;
-            H[j][j] = den; H[j + 1][j] = 0.0;
-            g[j + 1] = -sn[j] * g[j]; g[j] = cs[j] * g[j];
-            est = std::abs(g[j + 1]);
-            if (std::abs(g[j + 1]) <= stop || !(hn > 1e-300)) { ++j; ++total; break; }
+            // classical Gram-Schmidt against V_0..V_j; the update also normalises V_{j+1} and preconditions it unless the
+            // DGKS test asks for a second projection
+            const Ortho<float> o{Vp, j + 1, ne, M.w, M.V[j + 1], M.V[j], M.s.invdiag, dir, M.pv, ortho_part, ortho_cols, ortho_h, nullptr,
+                                 ortho_norms, box, 0};
+            double hn;
+            const double *h = arnoldi_cgs(o, kDgks, hn);
+            est = hs.add(j, h, use_mg ? 0.0 : 1.0, hn); // without multigrid Arnoldi ran on A P - I
+            if (est <= stop || !(hn > 1e-300)) { ++j; ++total; break; }
         }
-        for (int i = j - 1; i >= 0; --i)
-        {
-            double s = g[i];
-            for (int k = i + 1; k < j; ++k) s -= H[i][k] * yv[k];
-            yv[i] = s / H[i][i];
-        }
-        chk(hipMemcpyAsync(ydev, yv.data(), sizeof(double) * std::max(j, 1), hipMemcpyHostToDevice, stream), "H2D");
+        const Coefs y = hs.solve(j);
         if (use_mg)
-            LAUNCH("update_flex", k_update_flex, dim3(nb(ne)), dim3(256), 0, stream, static_cast<const float *const *>(M.Zptrs), ydev, j, dir, ne, delta);
+            LAUNCH("update_flex", k_update_flex, dim3(nb(ne)), dim3(256), 0, stream, static_cast<const float *const *>(M.Zptrs), y, j, dir, ne, x0,
+                   delta, tmp);
         else
-            LAUNCH("update_mixed", k_update_mixed, dim3(nb(ne / 4 + 1)), dim3(256), 0, stream, Vp, ydev, j, M.s.invdiag, dir, ne, delta);
+        {
+            prof_begin("update_mixed");
+            solution_update<float>(Vp, y, j, M.s.invdiag, dir, ne, x0, delta, tmp, stream);
+            prof_end();
+        }
     }
     LAUNCH("solve_final", k_solve_final, dim3(nb(ne)), dim3(256), 0, stream, x0, delta, Eex, dir, ne, Eout, corr);
     check_launch("mixed solve");

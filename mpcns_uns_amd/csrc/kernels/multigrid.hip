@@ -139,14 +139,20 @@ __global__ void __launch_bounds__(256) k_mg_prolong(int32_t n_fine, const int32_
     xf[i] += v >= 0 ? xc[v] : -xc[~v];
 }
 // flexible GMRES update: delta += sum_i y_i Z_i (Z already preconditioned, zero on Dirichlet edges)
-__global__ void __launch_bounds__(256) k_update_flex(const float *const *Z, const double *y, int32_t j, const int8_t *dir, int32_t n,
-                                                     double *delta)
+__global__ void __launch_bounds__(256) k_update_flex(const float *const *Z, Coefs y, int32_t j, const int8_t *dir, int32_t n, const double *x0,
+                                                     double *delta, double *x)
 {
     const int32_t e = gid();
-    if (e >= n || dir[e]) return;
-    double s = 0.0;
-    for (int32_t i = 0; i < j; ++i) s += y[i] * static_cast<double>(Z[i][e]);
-    delta[e] += s;
+    if (e >= n) return;
+    double dl = delta[e];
+    if (!dir[e])
+    {
+        double s = 0.0;
+        for (int32_t i = 0; i < j; ++i) s += y.v[i] * static_cast<double>(Z[i][e]);
+        dl += s;
+        delta[e] = dl;
+    }
+    x[e] = x0[e] + dl;
 }
 __global__ void __launch_bounds__(256) k_f32_to_f64(const float *x, int64_t n, double *out)
 {
@@ -343,7 +349,7 @@ extern "C" int mhdg_mg_apply(mhdg_ctx *c, const int8_t *dir, double dt, const do
         hip_check(hipMemcpyAsync(dd, dir, size_t(c->ne), hipMemcpyHostToDevice, c->stream), "H2D");
         const double *vd = c->stage_in(0, v, c->ne);
         double *zd = c->stage(3, c->ne);
-        hipLaunchKernelGGL(k_alpha_f32, dim3(nbk(c->nc)), dim3(256), 0, c->stream, c->alpha, c->B0, c->nc, M.s.aB0);
+        c->freeze(M.s.aB0);
         hipLaunchKernelGGL(k_mg_fine_invdiag, dim3(nbk(c->ne)), dim3(256), 0, c->stream, c->ne, c->d.m_e, c->d.d2, dt,
                            const_cast<float *>(M.s.invdiag));
         c->mg_set_solve(dd, static_cast<float>(dt));

@@ -110,14 +110,11 @@ void mhdg_ctx::apply_G(const double *phi, double *out)
         LAUNCH("field_of_flux", k_field_of_flux, dim3(nbk(3 * int64_t(nc))), dim3(256), 0, stream, Badd, bcell, 3 * int64_t(nc), nt.B0);
         LAUNCH("hall_g", k_hall_g, dim3(nbk(nc)), dim3(256), 0, stream, d, bcell, alpha, nt.B0, gcell);
     }
-    LAUNCH("edge_apply", k_edge_apply, dim3(nbk(ne)), dim3(256), 0, stream, d, int32_t(op_res), int32_t(op_hall), phi, gcell,
+    const size_t lds = n_heavy ? kApplyHeavyRows * size_t(max_valence) * sizeof(double) : 0;
+    LAUNCH("edge_apply", k_edge_apply, dim3(n_heavy + nbk(ne)), dim3(256), lds, stream, d, int32_t(op_res), int32_t(op_hall), phi, gcell,
            static_cast<const double *>(nullptr), static_cast<const int8_t *>(nullptr), static_cast<const double *>(nullptr),
-           static_cast<const double *>(nullptr), static_cast<const int8_t *>(nullptr), 0.0, 0, 0, static_cast<const double *>(nullptr), out);
-    if (n_heavy)
-        LAUNCH("edge_apply_heavy", k_edge_apply_heavy, dim3(n_heavy), dim3(256), 0, stream, d, int32_t(op_res), int32_t(op_hall),
-               static_cast<const int32_t *>(heavy), phi, gcell, static_cast<const double *>(nullptr), static_cast<const int8_t *>(nullptr),
-               static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), static_cast<const int8_t *>(nullptr), 0.0, 0, 0,
-               static_cast<const double *>(nullptr), out);
+           static_cast<const double *>(nullptr), static_cast<const int8_t *>(nullptr), 0.0, 0, 0, static_cast<const double *>(nullptr), out,
+           static_cast<const int32_t *>(heavy), n_heavy, max_valence);
     check_launch("apply_G");
 }
 
@@ -143,7 +140,7 @@ int mhdg_ctx::newton(const double *Phi_n, const double *Eex, const int8_t *dir, 
     // scale of the system: |E_expl + G(Phi^n)|
     apply_G(Phi_n, nt.G);
     LAUNCH("axpy", k_add, dim3(nbk(ne)), dim3(256), 0, stream, Eex, nt.G, ne, nt.rhs);
-    const double bnorm = std::sqrt(std::max(dot(nt.rhs, nt.rhs, 0, 0), 1e-300));
+    const double bnorm = std::sqrt(std::max(norms(nt.rhs, nullptr)[0], 1e-300));
     // the warm-start correction of the semi-implicit solve is not touched
     const bool had_corr = have_corr;
     if (had_corr) chk(hipMemcpyAsync(nt.corr_save, corr, E8, hipMemcpyDeviceToDevice, stream), "copy");
@@ -165,7 +162,7 @@ int mhdg_ctx::newton(const double *Phi_n, const double *Eex, const int8_t *dir, 
                static_cast<const double *>(nullptr), dt, nt.phik);
         apply_G(nt.phik, nt.G);
         LAUNCH("newton_residual", k_newton_residual, dim3(nbk(ne)), dim3(256), 0, stream, nt.E, Eex, nt.G, dir, ne, nt.R);
-        rn = std::sqrt(dot(nt.R, nt.R, 0, 0));
+        rn = std::sqrt(norms(nt.R, nullptr)[0]);
         if (!(rn > rtol * bnorm) || k >= max_newton) break;
         // J delta = -R, J = I + dt G'(Phi_k) d1, Dirichlet rows identity
         LAUNCH("bcell", k_bcell, dim3(nbk(nc)), dim3(256), 0, stream, d, nt.phik, nt.lin_b);
