@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../../include/mhdg.h"
+#include "adjoint.h"
 #include "explicit_step.h"
 #include "induction.h"
 #include "mixed.h"
@@ -54,17 +55,9 @@ struct mhdg_ctx
                          *dt_part = nullptr, *dt_dev = nullptr, *part = nullptr; } tw;
     double *energy_part = nullptr;
     double *snapshot = nullptr; // mhdg_state_save: U of every species and Phi
-    // reverse mode of the explicit step (adjoint.hip): gather maps, recomputed intermediates, adjoints, slots,
-    // and the state of every step of the forward sweep
-    struct AdjointWork { int32_t *fsl = nullptr, *f2e_pos = nullptr, *cec_ptr = nullptr, *cec = nullptr, *argc = nullptr;
-                         double *U[2]{}, *W[2]{}, *G[2]{}, *Ub[2]{}, *Wb[2]{}, *Gb[2]{}, *sF[2]{}, *sG[2]{}, *sFA[2]{};
-                         double *Phi = nullptr, *Bind = nullptr, *Btot = nullptr, *up = nullptr, *J = nullptr, *alpha = nullptr, *FA = nullptr,
-                                *Ef = nullptr, *E = nullptr, *dt_part = nullptr, *dt_dev = nullptr;
-                         double *Phib = nullptr, *PhiAddb = nullptr, *Baddb = nullptr, *Eb = nullptr, *Efb = nullptr, *FAb = nullptr, *upb = nullptr,
-                                *Btb = nullptr, *Bib = nullptr, *Jb = nullptr, *sE = nullptr, *sPhi = nullptr, *eF = nullptr, *eC = nullptr,
-                                *part = nullptr;
-                         mhdg::Dual *wd = nullptr;
-                         std::vector<double *> ck; } aw;
+    // reverse mode of the explicit step (adjoint.hip): its own step fields, gather maps, adjoints and slots, and the state
+    // before every step of the forward sweep and after the last
+    struct AdjointWork { mhdg::StepRun x{}; mhdg::AdjFields g{}; double *Ub[2]{}; std::vector<double *> ck; } aw;
     struct NewtonWork { double *phik = nullptr, *G = nullptr, *R = nullptr, *rhs = nullptr, *delta = nullptr, *E = nullptr,
                         *lin_b = nullptr, *B0 = nullptr, *zero_phi = nullptr, *corr_save = nullptr; } nt;
     std::vector<double *> V;
@@ -115,11 +108,14 @@ struct mhdg_ctx
     void check_launch(const char *what);
     void launch_edge_emf(const double *Ef, const double *u, double cuct, const double *Ein, double *Eout, int bc);
     // explicit_step.hip
+    mhdg::StepFields step_fields(double *Bt, double *up, double *cur, double *al); // allocated, with the face tables of sf
+    mhdg::StepRun resident_run();
     void step_build();
-    void launch_prepare();
-    void launch_states(int32_t n_face, double *dt_out, double dt_max); // n_face face-EMF blocks and (dt_out) the CFL minimum with them
-    // the explicit stage, with_ct: and the CT update with its EMF; the state is untouched when it throws
-    double explicit_stage(double dt_max, bool with_ct);
+    void launch_prepare(const mhdg::StepRun &x);
+    // n_face face-EMF blocks and (dt_out) the CFL minimum with them
+    void launch_states(const mhdg::StepRun &x, int32_t n_face, double *dt_out, double dt_max);
+    // the explicit stage; the state is untouched when it throws.  Returns the time step, checked (kStageNone: 0, unchecked)
+    double explicit_stage(const mhdg::StepRun &x, double dt_max, mhdg::StageEnd end);
     void get_record(int32_t first, int32_t n, double *host);
     const double *norms(const double *a, const double *b); // <a, a> and <b, b> (b nullable) on the host, |a| and |b| in scal
     mhdg::Ortho<double> ortho64(int j); // the FP64 solvers' Arnoldi step j
@@ -179,7 +175,6 @@ struct mhdg_ctx
     void explicit_tangent(int n_steps, double dt_max, const mhdg::Params &Pt);
     template <class R> void shell_energy(const R *phi, const R *badd, double r0, double r1, R *out);
     void vjp_alloc(int n_steps);
-    double vjp_stage(double dt_max, bool update);
     double step_vjp(int n_steps, double dt_max, double r0, double r1, double *fs_b, double *einf_b);
     void apply_G(const double *phi, double *out);
     void jvp(const double *phi_lin, const double *dphi, double *out);

@@ -481,7 +481,7 @@ double mhdg_ctx::step(double dt_max, int precision, int *iters, double *res)
     if ((precision == 1 || precision == 2) && ideal_cfg && u_ideal)
         throw std::runtime_error("mixed-precision solve: the implicit ideal part has no FP32 operator; use precision 0");
     const bool implicit = (op_hall || op_res || ideal_cfg) && !skip_implicit; // ImplicitInduction::active()
-    const double gdt = explicit_stage(dt_max, !implicit);
+    const double gdt = explicit_stage(resident_run(), dt_max, implicit ? kStageCells : kStageState);
     *iters = 0;
     *res = 0.0;
     if (implicit)
@@ -941,9 +941,9 @@ int mhdg_step_vjp(mhdg_ctx *c, int n_steps, double dt_max, double r0, double r1,
         if (J) *J = v;
         if (gU_H) c->d2h(gU_H, c->aw.Ub[0], 5 * C * 8);
         if (gU_Na) c->d2h(gU_Na, c->aw.Ub[1], 5 * C * 8);
-        if (gPhi) c->d2h(gPhi, c->aw.Phib, F * 8);
-        if (gPhiAdd) c->d2h(gPhiAdd, c->aw.PhiAddb, F * 8);
-        if (gBadd) c->d2h(gBadd, c->aw.Baddb, 3 * C * 8);
+        if (gPhi) c->d2h(gPhi, c->aw.g.Phib, F * 8);
+        if (gPhiAdd) c->d2h(gPhiAdd, c->aw.g.PhiAddb, F * 8);
+        if (gBadd) c->d2h(gBadd, c->aw.g.Baddb, 3 * C * 8);
     })
 }
 int mhdg_set_state(mhdg_ctx *c, const double *UH, const double *UNa, const double *Ph)
@@ -1054,8 +1054,8 @@ int mhdg_state_restore(mhdg_ctx *c)
 int mhdg_prepare(mhdg_ctx *c)
 {
     MHDG_TRY(c, {
-        c->launch_prepare();
-        c->launch_states(0, nullptr, 0);
+        c->launch_prepare(c->resident_run());
+        c->launch_states(c->resident_run(), 0, nullptr, 0);
         c->check_launch("prepare");
         hip_check(hipStreamSynchronize(c->stream), "sync");
     })

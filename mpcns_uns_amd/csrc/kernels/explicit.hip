@@ -28,34 +28,7 @@ template <class R> __global__ void __launch_bounds__(256) k_prepare(DevMesh d, P
         // the species rows through the kernel argument's pointer table itself (a local copy of the table, indexed by
         // a run-time species number, went to scratch memory)
         const R *const *Wc = Ws.p;
-        // up to kGradFast faces: the face rows are loaded once, together, for the cell vector and the time step
-        const int32_t k0 = d.c2f_ptr[c], k1 = d.c2f_ptr[c + 1], nk = k1 - k0;
-        const bool fast = kRowsInRegisters<R> && nk <= kGradFast;
-        double Ak[kGradFast];
-        V3 ak[kGradFast];
-        V3T<R> bi;
-        if (fast)
-        {
-            int32_t vk[kGradFast];
-            R fl[kGradFast];
-#pragma unroll
-            for (int i = 0; i < kGradFast; ++i)
-                if (i < nk) vk[i] = d.c2f[k0 + i];
-#pragma unroll
-            for (int i = 0; i < kGradFast; ++i)
-                if (i < nk)
-                {
-                    const int32_t f = pid(vk[i]);
-                    Ak[i] = d.famag[f]; ak[i] = L3(d.farea, f); fl[i] = Phi[f];
-                }
-            R M[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, r[3] = {0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < kGradFast; ++i)
-                if (i < nk) cell_vector_add(M, r, vk[i], R(Ak[i]), ak[i], fl[i]);
-            bi = cell_vector_solve(M, r);
-        }
-        else
-            bi = cell_vector(d, c, Phi);
+        const V3T<R> bi = cell_vector(d, c, Phi);
         const V3T<R> ba = L3(Badd, c);
         const V3T<R> bt(bi.x + ba.x, bi.y + ba.y, bi.z + ba.z);
         st3(Bind, c, bi);
@@ -74,7 +47,7 @@ template <class R> __global__ void __launch_bounds__(256) k_prepare(DevMesh d, P
                 else up = V3T<R>(up.x + chi * w[1], up.y + chi * w[2], up.z + chi * w[3]);
             }
             al = (P.hall && ne_eff > 0) ? d.taper[c] * P.hall_coef / ne_eff : 0.0;
-            dtc = fast ? cell_dt_rows<R, kGradFast>(P, d.cvol[c], Wc, bt, size_t(c), nk, Ak, ak) : cell_dt(d, P, c, Wc, bt, size_t(c));
+            dtc = cell_dt(d, P, c, Wc, bt, size_t(c));
         }
         st3(uplus, c, up);
         alpha[c] = al;
@@ -627,7 +600,6 @@ __global__ void __launch_bounds__(256) k_shell_energy(DevMesh d, const R *phi, c
 // the step (double) and its tangent-linear (Dual)
 template __global__ void k_shell_energy<double>(DevMesh, const double *, const double *, double, double, double *);
 template __global__ void k_shell_energy<Dual>(DevMesh, const Dual *, const Dual *, double, double, Dual *);
-template __global__ void k_prepare<double>(DevMesh d, Params P, SpCT<double> Us, const double *Phi, const double *Badd, SpWT<double> Ws, double *Bind, double *Btot, double *uplus, double *alpha, double *dt_part);
 template __global__ void k_dt_final<double>(const double *part, int32_t n, double dt_max, double *out);
 template __global__ void k_grad_current<double>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<double> Ws, SpCT<double> ghosts, SpWT<double> grads, int32_t limit, const double *Bind, double *J);
 template __global__ void k_face<double>(DevMesh d, Params P, int32_t ns, int32_t s0, SpCT<double> Ws, SpCT<double> grads, SpCT<double> ghosts, double *FA, const double *uplus, const double *Btot, const double *Bind, const double *Phi, const double *PhiAdd, const double *phi_ind, double *Ef);

@@ -23,6 +23,15 @@ struct StepFields
     const int8_t *fcls; // per face: kFluxNone, kFluxInner, kFluxLeft (the inside cell sees it outward), kFluxRight
     int32_t rs, ns;
 };
+// What a stage reads and writes: a state (U, Phi), the fields formed from it, the edge EMF and the time step
+struct StepRun
+{
+    double *U[kMaxSpecies], *Phi;
+    StepFields F;
+    double *E, *dt_part, *dt_dev;
+};
+// How far a stage goes: no update of the state, of its cells, of its cells and faces
+enum StageEnd { kStageNone, kStageCells, kStageState };
 enum : int8_t { kFluxNone = 0, kFluxInner = 1, kFluxLeft = 2, kFluxRight = 3 };
 inline int32_t step_row(int32_t ns) { return (5 * ns + 6 + 7) / 8 * 8; }
 

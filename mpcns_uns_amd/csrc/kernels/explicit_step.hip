@@ -24,7 +24,7 @@
 
 #include "ctx.h"
 #include "explicit_step.h"
-#include "fv.h"
+#include "step_cell.h"
 
 namespace mhdg
 {
@@ -82,37 +82,6 @@ constexpr int kStatesThreads = 128; // block of the (cell, ion) kernels: 20 KB o
 constexpr int kRoleThreads = 256;
 constexpr int kBatch = 2; // neighbour rows in flight per thread in the gradients (all four at once spilled at three waves per SIMD)
 
-__device__ __forceinline__ double2 ld2(const double *p) { return *reinterpret_cast<const double2 *>(p); }
-__device__ __forceinline__ V3 geo_normal(const DevMesh &d, int32_t f, double &A)
-{
-    const double2 p = ld2(d.geo + 4 * size_t(f)), q = ld2(d.geo + 4 * size_t(f) + 2);
-    A = q.y;
-    return V3(p.x, p.y, q.x);
-}
-// row of cell c in a (cell, face) table: the fixed length DEG, or the row pointers (DEG 0)
-template <int DEG> __device__ __forceinline__ void row_of(const DevMesh &d, int32_t c, int32_t &k0, int32_t &nk)
-{
-    if (DEG > 0) { k0 = c * DEG; nk = DEG; }
-    else { k0 = d.c2f_ptr[c]; nk = d.c2f_ptr[c + 1] - k0; }
-}
-// the DEG entries of row k0 of a (cell, face) id table
-template <int DEG> __device__ __forceinline__ void row_ids(const int32_t *tab, int32_t k0, int32_t (&v)[DEG])
-{
-    if constexpr (DEG == 4)
-    {
-        const int4 q = *reinterpret_cast<const int4 *>(tab + k0);
-        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-    }
-    else
-    {
-#pragma unroll
-        for (int i = 0; i < DEG; i += 2)
-        {
-            const int2 q = *reinterpret_cast<const int2 *>(tab + k0 + i);
-            v[i] = q.x; v[i + 1] = q.y;
-        }
-    }
-}
 // cell_vector_add (fv.h) with the unit normal given: (s / |A|) a is s ((1 / |A|) a) bit for bit
 __device__ __forceinline__ void vector_add(double (&M)[3][3], double (&r)[3], double s, double A, const V3 &n, double flux)
 {
@@ -617,49 +586,14 @@ template <int DEG, int NS>
 __device__ __forceinline__ void update_role(const DevMesh &d, const Params &P, const StepFields &F, const double *dt_dev, const SpW &Us,
                                             int32_t block)
 {
-    constexpr int N = DEG > 0 ? DEG : 1;
     const int32_t ns = NS > 0 ? NS : P.ns, per = kRoleThreads / ns, t = threadIdx.x, cl = t / ns, s = t - cl * ns;
     const int32_t c = block * per + cl;
     if (cl >= per || c >= d.nc || d.mat[c] != 0) return;
     const double dt = dt_dev[0], V = d.cvol[c];
     const double *row = F.rec + (NS == 2 ? 16 : size_t(F.rs)) * size_t(c);
-    const double *W = row + 5 * s;
     double *u = Us.p[s] + 5 * size_t(c);
-    double rhs[5] = {0, 0, 0, 0, 0};
-    int32_t k0, nk;
-    row_of<DEG>(d, c, k0, nk);
-    auto add = [&](int32_t v, const double *fa) {
-        if (v >= 0) for (int m = 0; m < 5; ++m) rhs[m] -= fa[m] / V;
-        else for (int m = 0; m < 5; ++m) rhs[m] += fa[m] / V;
-    };
-    if constexpr (DEG > 0)
-    {
-        int32_t v[N];
-        double fa[N][5];
-        row_ids<DEG>(d.cfs, k0, v);
-#pragma unroll
-        for (int i = 0; i < DEG; ++i)
-            for (int m = 0; m < 5; ++m) fa[i][m] = F.FA[5 * (size_t(pid(v[i])) * size_t(ns) + s) + m];
-#pragma unroll
-        for (int i = 0; i < DEG; ++i) add(v[i], fa[i]);
-    }
-    else
-        for (int32_t k = k0; k < k0 + nk; ++k) add(d.cfs[k], F.FA + 5 * (size_t(pid(d.cfs[k])) * size_t(ns) + s));
-    double ne = ion_density(P, 0, row[0]);
-    for (int q = 1; q < ns; ++q) ne = ne + ion_density(P, q, row[5 * q]);
-    const double ws = ion_density(P, s, W[0]) / sqrt(ne * ne + P.ne_floor * P.ne_floor);
-    const double rho = mx(W[0], 0.0);
-    const V3 vel(W[1], W[2], W[3]);
-    V3 S;
-    if (P.lorentz) S += (P.inver_MA2 * ws) * cross(L3(F.J, c), L3(F.Btot, c));
-    rhs[1] += S.x; rhs[2] += S.y; rhs[3] += S.z;
-    rhs[4] += dot(vel, S) + (rho > 1e-30 ? 0.5 * dt * dot(S, S) / rho : 0.0);
-    if (P.src_rate[s] != 0.0 && d.atm)
-    {
-        const double q = P.src_rate[s] * d.atm[c];
-        rhs[0] += q;
-        rhs[4] += q * P.src_T / (P.gamma - 1.0);
-    }
+    double rhs[5];
+    cell_rhs<DEG>(d, P, F, c, s, ns, row, V, dt, rhs);
     double q[5];
     for (int m = 0; m < 5; ++m) q[m] = u[m] + dt * rhs[m];
     const double ke = q[0] > 0 ? 0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0] : 0.0;
@@ -738,18 +672,34 @@ template <class Fn> void by_shape(int32_t cdeg, int32_t ns, Fn f)
         prof_end();                                                                                                          \
     } while (0)
 
-void mhdg_ctx::step_build()
+StepFields mhdg_ctx::step_fields(double *Bt, double *up, double *cur, double *al)
 {
     const size_t F = nf, C = nc, ns = size_t(P.ns);
     auto D = [&](size_t n) { return static_cast<double *>(alloc(n * sizeof(double))); };
-    sf.rs = step_row(P.ns);
-    sf.ns = P.ns;
-    sf.rec = D(size_t(sf.rs) * C);
-    chk(hipMemset(sf.rec, 0, size_t(sf.rs) * C * 8), "memset");
-    sf.Btot = Btot; sf.uplus = uplus; sf.J = J; sf.alpha = alpha;
-    sf.FS = D(5 * ns * c2f_nnz);
-    sf.FA = D(5 * ns * F);
-    sf.Ef = D(4 * F);
+    StepFields o = sf; // the face tables
+    o.rs = step_row(P.ns);
+    o.ns = P.ns;
+    o.rec = D(size_t(o.rs) * C);
+    chk(hipMemset(o.rec, 0, size_t(o.rs) * C * 8), "memset");
+    o.Btot = Bt; o.uplus = up; o.J = cur; o.alpha = al;
+    o.FS = D(5 * ns * c2f_nnz);
+    o.FA = D(5 * ns * F);
+    o.Ef = D(4 * F);
+    return o;
+}
+
+StepRun mhdg_ctx::resident_run()
+{
+    StepRun r{};
+    for (int s = 0; s < P.ns; ++s) r.U[s] = U[s];
+    r.Phi = Phi; r.F = sf; r.E = E_expl; r.dt_part = dt_part; r.dt_dev = dt_dev;
+    return r;
+}
+
+void mhdg_ctx::step_build()
+{
+    const size_t F = nf;
+    sf = step_fields(Btot, uplus, J, alpha);
     int2 *fent = static_cast<int2 *>(alloc(F * sizeof(int2)));
     int8_t *fcls = static_cast<int8_t *>(alloc(F));
     hipLaunchKernelGGL(k_face_entries, dim3(blocks(nf, 256)), dim3(256), 0, stream, d, fent, fcls);
@@ -757,67 +707,68 @@ void mhdg_ctx::step_build()
     sf.fent = fent; sf.fcls = fcls;
 }
 
-void mhdg_ctx::launch_prepare()
+void mhdg_ctx::launch_prepare(const StepRun &x)
 {
     SpC Uc{};
-    for (int s = 0; s < P.ns; ++s) Uc.p[s] = U[s];
+    for (int s = 0; s < P.ns; ++s) Uc.p[s] = x.U[s];
     by_shape(cdeg, P.ns, [&](auto deg, auto ns) {
         constexpr int DEG = decltype(deg)::value;
         if constexpr (decltype(ns)::value == 2)
-            LAUNCH("prepare", k_step_prepare2<DEG>, dim3(blocks(nc, 256)), dim3(256), 0, stream, d, P, Uc, static_cast<const double *>(Phi),
-                   static_cast<const double *>(Badd), sf, dt_part);
+            LAUNCH("prepare", k_step_prepare2<DEG>, dim3(blocks(nc, 256)), dim3(256), 0, stream, d, P, Uc, static_cast<const double *>(x.Phi),
+                   static_cast<const double *>(Badd), x.F, x.dt_part);
         else
             LAUNCH("prepare", k_step_prepare_many<DEG>, dim3(blocks(nc, 256 / P.ns)), dim3(256), 0, stream, d, P, Uc,
-                   static_cast<const double *>(Phi), static_cast<const double *>(Badd), sf, dt_part);
+                   static_cast<const double *>(x.Phi), static_cast<const double *>(Badd), x.F, x.dt_part);
     });
 }
 
-void mhdg_ctx::launch_states(int32_t n_face, double *dt_out, double dt_max)
+void mhdg_ctx::launch_states(const StepRun &x, int32_t n_face, double *dt_out, double dt_max)
 {
     const int32_t n_cell = blocks(nc, kStatesThreads / P.ns), n_part = blocks(nc, P.ns == 2 ? 256 : 256 / P.ns);
     by_shape(cdeg, P.ns, [&](auto deg, auto ns) {
         LAUNCH("states", (k_step_states<decltype(deg)::value, decltype(ns)::value>), dim3(n_cell + n_face + (dt_out ? 1 : 0)),
-               dim3(kStatesThreads), 0, stream, d, P, sf, static_cast<const double *>(Phi), static_cast<const double *>(PhiAdd), n_cell, n_face,
-               static_cast<const double *>(dt_part), n_part, dt_max, dt_out, dt_box, ticket);
+               dim3(kStatesThreads), 0, stream, d, P, x.F, static_cast<const double *>(x.Phi), static_cast<const double *>(PhiAdd), n_cell, n_face,
+               static_cast<const double *>(x.dt_part), n_part, dt_max, dt_out, dt_box, ticket);
     });
 }
 
-double mhdg_ctx::explicit_stage(double dt_max, bool with_ct)
+double mhdg_ctx::explicit_stage(const StepRun &x, double dt_max, StageEnd end)
 {
     // nothing before this wrote U or Phi (only derived fields), so the state is unchanged when it throws
     auto checked = [](double v) {
         if (!std::isfinite(v) || v <= 0) throw std::runtime_error("invalid time step");
         return v;
     };
-    launch_prepare();
+    launch_prepare(x);
     // Strang split of the ions' gyration (Solver.cpp:237-241): half a step, then prepare again.  The rotation changes
     // U, so the time step is checked first, as the reference throws before it touches the state (Solver.cpp:236).
     const bool split = P.induce_coeff > 0 && P.lorentz;
     double gdt = 0;
     if (split)
     {
-        LAUNCH("dt_final", k_dt_final<double>, dim3(1), dim3(256), 0, stream, static_cast<const double *>(dt_part), blocks(nc, 256), dt_max, dt_dev);
-        d2h(&gdt, dt_dev, 8);
+        LAUNCH("dt_final", k_dt_final<double>, dim3(1), dim3(256), 0, stream, static_cast<const double *>(x.dt_part), blocks(nc, 256), dt_max, x.dt_dev);
+        d2h(&gdt, x.dt_dev, 8);
         checked(gdt);
-        LAUNCH("gyrate", k_gyrate, dim3(blocks(nc, 256)), dim3(256), 0, stream, d, P, U[0], U[1], static_cast<const double *>(Btot),
-               static_cast<const double *>(dt_dev), 0.5);
-        launch_prepare();
+        LAUNCH("gyrate", k_gyrate, dim3(blocks(nc, 256)), dim3(256), 0, stream, d, P, x.U[0], x.U[1], static_cast<const double *>(x.F.Btot),
+               static_cast<const double *>(x.dt_dev), 0.5);
+        launch_prepare(x);
     }
     ++ticket;
-    launch_states(blocks(nf, kStatesThreads), split ? nullptr : dt_dev, dt_max);
+    launch_states(x, blocks(nf, kStatesThreads), split ? nullptr : x.dt_dev, dt_max);
     const int n_edge = blocks(ne, kRoleThreads), n_flux = blocks(nf, kRoleThreads / P.ns);
     const size_t lds = sizeof(double) * std::max<size_t>(5 * kRoleThreads, n_heavy ? 6 * size_t(max_valence) : 0);
     auto kflux = P.ns == 2 ? k_step_fluxes<2> : k_step_fluxes<0>;
-    LAUNCH("fluxes", kflux, dim3(n_heavy + n_edge + n_flux), dim3(kRoleThreads), lds, stream, d, P, sf, E_expl, static_cast<const int32_t *>(heavy),
+    LAUNCH("fluxes", kflux, dim3(n_heavy + n_edge + n_flux), dim3(kRoleThreads), lds, stream, d, P, x.F, x.E, static_cast<const int32_t *>(heavy),
            n_heavy, max_valence, n_edge);
     check_launch("explicit stage");
+    if (end == kStageNone) return 0.0;
     if (!split) gdt = checked(wait_box(dt_box)[0]); // written while the states were formed
     SpW Us{};
-    for (int s = 0; s < P.ns; ++s) Us.p[s] = U[s];
-    const int n_cell = blocks(nc, kRoleThreads / P.ns), n_face = with_ct ? blocks(nf, kRoleThreads) : 0;
+    for (int s = 0; s < P.ns; ++s) Us.p[s] = x.U[s];
+    const int n_cell = blocks(nc, kRoleThreads / P.ns), n_face = end == kStageState ? blocks(nf, kRoleThreads) : 0;
     by_shape(cdeg, P.ns, [&](auto deg, auto ns) {
         LAUNCH("update", (k_step_update<decltype(deg)::value, decltype(ns)::value>), dim3(n_cell + n_face), dim3(kRoleThreads), 0, stream, d, P,
-               sf, static_cast<const double *>(dt_dev), Us, n_cell, static_cast<const double *>(E_expl), Phi);
+               x.F, static_cast<const double *>(x.dt_dev), Us, n_cell, static_cast<const double *>(x.E), x.Phi);
     });
     check_launch("cell update");
     return gdt;

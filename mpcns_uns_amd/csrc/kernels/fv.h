@@ -87,45 +87,6 @@ template <class R> __device__ R cell_dt(const DevMesh &d, const Params &P, int32
     return dt;
 }
 
-// cell_dt for a cell whose N or fewer faces are given as (|A|, area vector) rows: the face normal and the normal
-// Alfven term, which do not depend on the species, are formed once (same operations as cell_dt)
-template <class R, int N>
-__device__ R cell_dt_rows(const Params &P, double vol, const R *const *Ws, const V3T<R> &b, size_t row, int nk, const double (&A)[N],
-                          const V3 (&area)[N])
-{
-    R dt = __builtin_inf();
-    const R B2 = dot(b, b);
-    R rho_sum = Ws[0][5 * row];
-    for (int s = 1; s < P.ns; ++s) rho_sum = rho_sum + Ws[s][5 * row];
-    const R rho_tot = mx(rho_sum, P.rho_floor_dt);
-    const R vA2 = P.inver_MA2 * B2 / rho_tot;
-    V3T<R> n[N];
-    R vAn2[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-        if (i < nk)
-        {
-            n[i] = (1.0 / A[i]) * area[i];
-            vAn2[i] = P.inver_MA2 * dot(b, n[i]) * dot(b, n[i]) / rho_tot;
-        }
-    for (int s = 0; s < P.ns; ++s)
-    {
-        const R *w = Ws[s] + 5 * row;
-        const R cs2 = P.gamma * w[4] / mx(w[0], 1e-30);
-        R denom = 0;
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-            if (i < nk)
-            {
-                const R term = cs2 + vA2;
-                const R cf = sqrt(0.5 * (term + sqrt(mx(0.0, term * term - 4 * cs2 * vAn2[i]))));
-                denom += (fabs(w[1] * n[i].x + w[2] * n[i].y + w[3] * n[i].z) + cf) * A[i];
-            }
-        if (denom > 0) dt = mn(dt, P.cfl * vol / denom);
-    }
-    return dt;
-}
-
 template <class R> __device__ __forceinline__ R block_min(R v, R *sh)
 {
     const int t = threadIdx.x;
