@@ -728,7 +728,7 @@ __global__ void __launch_bounds__(kAdjThreads, 3) k_adj_update(DevMesh d, Params
     else if (b < n_heavy + n_dt) dt_cell_role(d, P, F, G, dt_part, n_part, dt);
     else if (b < n_heavy + n_dt + n_edge)
     {
-        const int32_t i = b - n_heavy - n_dt;
+        const int32_t i = near_block(d, b, n_heavy + n_dt, n_edge);
         double part[4] = {0, 0, 0, 0};
         edge_adjoint_light(d, F, G, P.cuct, dt, E, i * kAdjThreads + int32_t(threadIdx.x), part);
         double *o = G.e_part + 4 * size_t(n_heavy + i);
@@ -744,7 +744,7 @@ __global__ void __launch_bounds__(kAdjThreads, 3) k_adj_update(DevMesh d, Params
     }
     else
     {
-        const int32_t i = b - n_heavy - n_dt - n_edge;
+        const int32_t first = n_heavy + n_dt + n_edge, i = near_block(d, b, first, int32_t(gridDim.x) - first);
         const double s = block_sum(update_adjoint_role<DEG>(d, P, F, G, Us, Ub, dt, i), sh);
         if (threadIdx.x == 0) G.c_part[i] = s;
     }
@@ -764,8 +764,8 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_faces(DevMesh d, Params P, 
         v = block_sum(v, sh);
         if (threadIdx.x == 0) G.dtb[0] = v;
     }
-    else if (b <= n_emf) face_emf_adjoint_role(d, F, G, Phi, PhiAdd, (b - 1) * kAdjThreads + int32_t(threadIdx.x));
-    else flux_adjoint_role(d, P, F, G, b - 1 - n_emf, sh);
+    else if (b <= n_emf) face_emf_adjoint_role(d, F, G, Phi, PhiAdd, near_block(d, b, 1, n_emf) * kAdjThreads + int32_t(threadIdx.x));
+    else flux_adjoint_role(d, P, F, G, near_block(d, b, 1 + n_emf, int32_t(gridDim.x) - 1 - n_emf), sh);
 }
 
 // Limited gradients (Reconstruction.cpp:80-142) and the states formed from them (FluxRHS.cpp:16-27), transposed: thread
@@ -776,7 +776,8 @@ __global__ void __launch_bounds__(kGradThreads, DEG == 6 ? 2 : 3) k_adj_gradient
 {
     constexpr int N = DEG > 0 ? DEG : 1, kCells = kGradThreads / kAdjNs;
     __shared__ double stage[kGradThreads * (DEG > 0 ? 5 * DEG : 1)];
-    const int32_t t = threadIdx.x, s = t & 1, cl = t >> 1, c0 = blockIdx.x * kCells, c = c0 + cl;
+    const int32_t t = threadIdx.x, s = t & 1, cl = t >> 1;
+    const int32_t c0 = near_block(d, int32_t(blockIdx.x), 0, int32_t(gridDim.x)) * kCells, c = c0 + cl;
     const int32_t n_here = min(kCells, d.nc - c0) * (DEG * kAdjNs * 5 / 2);
     if constexpr (DEG > 0)
     {
@@ -1000,7 +1001,7 @@ template <int DEG>
 __global__ void __launch_bounds__(kAdjThreads) k_adj_cells(DevMesh d, Params P, StepFields F, AdjFields G, SpC Us, SpW Ub, int32_t with_dt)
 {
     constexpr int N = DEG > 0 ? DEG / 2 : 1;
-    const int32_t t = threadIdx.x, s = t & 1, c = blockIdx.x * (kAdjThreads / kAdjNs) + (t >> 1);
+    const int32_t t = threadIdx.x, s = t & 1, c = gid(d) >> 1;
     if (c >= d.nc) return; // both threads of a cell
     // the face normals' matrix of the reconstruction (Reconstruct.cpp:11-45), the faces' and edges' parts: this thread's half
     int32_t k0, nk;
@@ -1123,7 +1124,7 @@ __global__ void __launch_bounds__(kAdjThreads) k_adj_energy(DevMesh d, const dou
 // Face gather of the reconstruction parts: Phib_f += both cells' slots; the first one of a sweep sets Phib and PhiAddb
 __global__ void __launch_bounds__(kAdjThreads) k_adj_flux(DevMesh d, const int2 *fent, AdjFields G, int32_t first)
 {
-    const int32_t f = gid();
+    const int32_t f = gid(d);
     if (f >= d.nf) return;
     const int2 e = fent[f];
     const double x = (e.x >= 0 ? G.sPhi[e.x] : 0.0) + (e.y >= 0 ? G.sPhi[e.y] : 0.0);

@@ -28,6 +28,7 @@ using Prim = PrimT<double>;
 struct DevMesh
 {
     int32_t nc, nf, ne;
+    int32_t xcd_ranges;             // near_block: each XCD takes one range of a kernel's blocks
     int32_t cdeg, fdeg;             // faces per cell / edges per face when every row has that many (tets: 4, 3), else 0
     const int32_t *c2f_ptr, *c2f;   // cell -> faces, stored order
     const int32_t *cfs;             // cell -> faces sorted by face id (same ptr as c2f), signed
@@ -107,9 +108,18 @@ template <class R> __device__ __forceinline__ R electron_density(const Params &P
     return ne;
 }
 
-// Global thread index of a one-entity-per-thread launch.  (An XCD-contiguous block order, which keeps the
-// blocks of one XCD on one index range, was measured on the gather kernels: 4 % faster for the FP32 edge
-// kernel, which uses it, and no gain or a loss for the others, where the 256 MB MALL already serves the data
-// the eight L2s share.)
+// Global thread index of a one-entity-per-thread launch
 __device__ __forceinline__ int32_t gid() { return static_cast<int32_t>(blockIdx.x * blockDim.x + threadIdx.x); }
+// Which block of a role's n the launch's block b is, the role starting at block `first`.  The hardware runs block b on XCD
+// b % 8.  With xcd_ranges each XCD takes one contiguous eighth of the role, the same eighth in every kernel, so it finds
+// its neighbours' data, and what it wrote in the kernel before, in its own L2.
+__device__ __forceinline__ int32_t near_block(const DevMesh &d, int32_t b, int32_t first, int32_t n)
+{
+    const int32_t i = b - first, per = n >> 3;
+    return d.xcd_ranges && i < 8 * per ? (b & 7) * per + (i >> 3) : i;
+}
+__device__ __forceinline__ int32_t gid(const DevMesh &d)
+{
+    return near_block(d, int32_t(blockIdx.x), 0, int32_t(gridDim.x)) * int32_t(blockDim.x) + int32_t(threadIdx.x);
+}
 } // namespace mhdg

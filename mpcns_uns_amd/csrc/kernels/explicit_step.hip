@@ -12,11 +12,12 @@
 // measurable (8M tetrahedra: 6181 us per step with the face EMFs in the states' launch, 6200 in one of their own).
 //
 // Measured, microseconds per explicit step, against one kernel per operation with gradients in memory (8 launches; one
-// MI355X): 9.5k tetrahedra 90 -> 46, 60k 113 -> 73, 484k 547 -> 402, 1.95M 1982 -> 1553, 7.83M 7723 -> 6247.  At 7.83M
+// MI355X): 9.5k tetrahedra 90 -> 36, 60k 113 -> 59, 484k 547 -> 396, 1.95M 1982 -> 1553, 7.83M 7723 -> 6235.  At 7.83M
 // prepare takes 623 us (994 before), states 2486 and fluxes 2596 (5660 for the gradients, fluxes, EMF candidates and
 // edge sums before), update 871 (1073).  prepare, the flux half of fluxes and update run at 5.0-5.5 TB/s of their bytes
 // (the streaming copy reaches 6.1); states is bound by its FP64 instructions and the loads' latency at three waves per
-// SIMD, the edge half of fluxes by the L1's outstanding requests.
+// SIMD, the edge half of fluxes by the L1's outstanding requests.  The roles' blocks follow one another: taking them in
+// turn, one or eight each, let the two working sets evict each other (484k: fluxes 153 -> 213 us, states 154 -> 206).
 #include <algorithm>
 #include <cmath>
 #include <stdexcept>
@@ -173,7 +174,7 @@ __global__ void __launch_bounds__(256) k_step_prepare2(DevMesh d, Params P, SpC 
                                                        double *dt_part)
 {
     __shared__ double stage[256 * 17];
-    const int32_t c = gid();
+    const int32_t block = near_block(d, int32_t(blockIdx.x), 0, int32_t(gridDim.x)), c = block * 256 + int32_t(threadIdx.x);
     double dtc = __builtin_inf();
     if (c < d.nc)
     {
@@ -208,11 +209,11 @@ __global__ void __launch_bounds__(256) k_step_prepare2(DevMesh d, Params P, SpC 
         q[10] = bi.x; q[11] = bi.y; q[12] = bi.z; q[13] = xc.x; q[14] = xc.y; q[15] = xc.z;
     }
     __syncthreads();
-    const int32_t c0 = blockIdx.x * 256, n_here = min(256, d.nc - c0);
+    const int32_t c0 = block * 256, n_here = min(256, d.nc - c0);
     for (int32_t i = threadIdx.x; i < 16 * n_here; i += 256) F.rec[16 * size_t(c0) + i] = stage[17 * (i >> 4) + (i & 15)];
     __syncthreads();
     const double m = block_min(dtc, stage);
-    if (threadIdx.x == 0) dt_part[blockIdx.x] = m;
+    if (threadIdx.x == 0) dt_part[block] = m;
 }
 
 // The same for more than two ions: one thread per (cell, ion), the ions of a cell side by side, so the record rows and
@@ -222,7 +223,8 @@ __global__ void __launch_bounds__(256) k_step_prepare_many(DevMesh d, Params P, 
                                                            double *dt_part)
 {
     __shared__ double sW[256 * 5], sn[256];
-    const int32_t ns = P.ns, per = 256 / ns, t = threadIdx.x, cl = t / ns, s = t - cl * ns, c = blockIdx.x * per + cl;
+    const int32_t ns = P.ns, per = 256 / ns, t = threadIdx.x, cl = t / ns, s = t - cl * ns;
+    const int32_t c = near_block(d, int32_t(blockIdx.x), 0, int32_t(gridDim.x)) * per + cl;
     const bool act = cl < per && c < d.nc;
     double dtc = __builtin_inf();
     if (act)
@@ -615,8 +617,8 @@ __global__ void __launch_bounds__(kStatesThreads, DEG == 6 ? 2 : 3) k_step_state
     // the larger of the staged face states (5 DEG per thread) and the reduction of the time step
     __shared__ double stage[kStatesThreads * (DEG > 0 ? 5 * DEG : 1)];
     const int32_t b = blockIdx.x;
-    if (b < n_cell) states_role<DEG, NS>(d, P, F, b, stage);
-    else if (b < n_cell + n_face) face_emf_role(d, F, Phi, PhiAdd, (b - n_cell) * kStatesThreads + int32_t(threadIdx.x));
+    if (b < n_cell) states_role<DEG, NS>(d, P, F, near_block(d, b, 0, n_cell), stage);
+    else if (b < n_cell + n_face) face_emf_role(d, F, Phi, PhiAdd, near_block(d, b, n_cell, n_face) * kStatesThreads + int32_t(threadIdx.x));
     else dt_role(dt_part, n_part, dt_max, dt_dev, stage, box, ticket);
 }
 // Dynamic LDS: the heavy edges' rows (fv.h) when there are any
@@ -628,16 +630,17 @@ __global__ void __launch_bounds__(kRoleThreads) k_step_fluxes(DevMesh d, Params 
     const int32_t b = blockIdx.x;
     if (b < n_heavy) edge_emf_heavy<double>(d, P, F.Ef, F.uplus, P.cuct, heavy[b], nullptr, E, 1, shared, hv);
     else if (b < n_heavy + n_edge)
-        edge_emf_light<double>(d, P, F.Ef, F.uplus, P.cuct, kLightMax, (b - n_heavy) * kRoleThreads + int32_t(threadIdx.x), nullptr, E, 1);
-    else flux_role<NS>(d, P, F, b - n_heavy - n_edge, shared);
+        edge_emf_light<double>(d, P, F.Ef, F.uplus, P.cuct, kLightMax,
+                               near_block(d, b, n_heavy, n_edge) * kRoleThreads + int32_t(threadIdx.x), nullptr, E, 1);
+    else flux_role<NS>(d, P, F, near_block(d, b, n_heavy + n_edge, int32_t(gridDim.x) - n_heavy - n_edge), shared);
 }
 template <int DEG, int NS>
 __global__ void __launch_bounds__(kRoleThreads) k_step_update(DevMesh d, Params P, StepFields F, const double *dt_dev, SpW Us, int32_t n_cell,
                                                               const double *E, double *Phi)
 {
     const int32_t b = blockIdx.x;
-    if (b < n_cell) update_role<DEG, NS>(d, P, F, dt_dev, Us, b);
-    else faraday_face(d, E, nullptr, dt_dev, 0.0, Phi, (b - n_cell) * kRoleThreads + int32_t(threadIdx.x));
+    if (b < n_cell) update_role<DEG, NS>(d, P, F, dt_dev, Us, near_block(d, b, 0, n_cell));
+    else faraday_face(d, E, nullptr, dt_dev, 0.0, Phi, near_block(d, b, n_cell, int32_t(gridDim.x) - n_cell) * kRoleThreads + int32_t(threadIdx.x));
 }
 } // namespace mhdg
 

@@ -18,7 +18,7 @@ __global__ void __launch_bounds__(256) k_div_scalar(const double *r, const doubl
 __global__ void __launch_bounds__(256) k_d1(DevMesh d, const double *v, const double *invdiag, const int8_t *dir, const double *dte,
                                             double *phi)
 {
-    const int32_t f = gid();
+    const int32_t f = gid(d);
     if (f >= d.nf) return;
     double s = 0.0;
     if (d.fdeg == 3 && !dte)
@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(256) k_hall_g(DevMesh d, const double *b, cons
 // runs in the order of the one-thread kernels and the results are the same bit for bit.
 template <int G> __global__ void __launch_bounds__(256) k_bcell_g(DevMesh d, const double *phi, double *b)
 {
-    const int32_t t = int32_t(blockIdx.x * blockDim.x + threadIdx.x);
+    const int32_t t = gid(d);
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     // a fixed row length (tetrahedra) spares the row-bound loads ahead of the gathers
@@ -176,7 +176,7 @@ template <int G> __global__ void __launch_bounds__(256) k_bcell_g(DevMesh d, con
 }
 template <int G> __global__ void __launch_bounds__(256) k_hall_g_g(DevMesh d, const double *b, const double *alpha, const double *B0, double *g)
 {
-    const int32_t t = int32_t(blockIdx.x * blockDim.x + threadIdx.x);
+    const int32_t t = gid(d);
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     const double a = ok ? alpha[c] : 0.0;
@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(256) k_edge_apply(DevMesh d, int32_t resistive
         edge_apply_heavy(d, resistive, hall, heavy[b], phi, g, ide, imask, v, invdiag, dir, dt, mode, mask, bvec, out, shared, hv);
         return;
     }
-    const int32_t e = (b - n_heavy) * 256 + int32_t(threadIdx.x);
+    const int32_t e = near_block(d, b, n_heavy, int32_t(gridDim.x) - n_heavy) * 256 + int32_t(threadIdx.x);
     if (e >= d.ne) return;
     const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1];
     if (f1 - f0 > kLightMax) return; // a heavy block's
@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(256) k_edge_apply(DevMesh d, int32_t resistive
 // k_bcell_g, k_hall_g_g and k_edge_apply, so b and r0 are the same bits as the two separate products give.
 template <int G> __global__ void __launch_bounds__(256) k_bcell2_g(DevMesh d, const double *phi1, const double *phi2, double *b1, double *b2)
 {
-    const int32_t t = int32_t(blockIdx.x * blockDim.x + threadIdx.x);
+    const int32_t t = gid(d);
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     const int32_t k0 = !ok ? 0 : d.cdeg > 0 ? c * d.cdeg : d.c2f_ptr[c];
@@ -399,7 +399,7 @@ template <int G>
 __global__ void __launch_bounds__(256) k_hall_g2_g(DevMesh d, const double *b1, const double *b2, const double *alpha, const double *B0,
                                                    double *g1, double *g2)
 {
-    const int32_t t = int32_t(blockIdx.x * blockDim.x + threadIdx.x);
+    const int32_t t = gid(d);
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     const double a = ok ? alpha[c] : 0.0;
@@ -517,7 +517,7 @@ __global__ void __launch_bounds__(256) k_edge_rhs_residual(DevMesh d, int32_t re
         rhs_residual_heavy(d, resistive, hall, heavy[b], phi1, g1, phi2, g2, E_expl, x, dir, dt, bvec, r, shared, hv);
         return;
     }
-    const int32_t e = (b - n_heavy) * 256 + int32_t(threadIdx.x);
+    const int32_t e = near_block(d, b, n_heavy, int32_t(gridDim.x) - n_heavy) * 256 + int32_t(threadIdx.x);
     if (e >= d.ne) return;
     const int32_t f0 = d.e2f_ptr[e], f1 = d.e2f_ptr[e + 1];
     if (f1 - f0 > kLightMax) return; // a heavy block's

@@ -11,7 +11,8 @@ constexpr int32_t kLightMax = 32;   // edges up to this valence use one thread e
 constexpr int kEdgeUnroll = 8; // entries of an edge row (faces or cells around the edge)
 constexpr int kRowUnroll = 4;  // entries of a face or cell row (edges of a face, faces of a cell)
 // Block index that gives each XCD one contiguous range of blocks (the hardware runs block b on XCD b % 8), so that
-// neighbouring edges share an L2 for their gathers: 4 % faster for the FP32 edge kernel, slower for the cell kernels
+// neighbouring edges share an L2 for their gathers: 4 % faster for the FP32 edge kernel at every size; the other kernels
+// gain on small meshes only (near_block, dev.h)
 __device__ __forceinline__ int32_t xcd_block(uint32_t nb)
 {
     const uint32_t b = blockIdx.x, per = nb / 8;

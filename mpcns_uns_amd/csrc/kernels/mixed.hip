@@ -58,7 +58,7 @@ __device__ __forceinline__ void rows(int32_t deg, const int32_t *ptr, int32_t r,
 // Phi'_f = sum_k f2e_k pv_e with pv = P v (0 on Dirichlet edges), times dt_e with a per-edge step
 __global__ void __launch_bounds__(256) k_d1_f32(DevMesh d, DevMesh32 s, const float *pv, const float *dte, float *phi)
 {
-    const int32_t f = gid();
+    const int32_t f = gid(d);
     if (f >= d.nf) return;
     if (s.fdeg == 3 && !dte)
     {
@@ -287,7 +287,7 @@ template <int G> __device__ __forceinline__ float group_sum(float v)
 }
 template <int G> __global__ void __launch_bounds__(256) k_bcell_f32_g(DevMesh d, DevMesh32 s, const float *phi, float *b)
 {
-    const int32_t t = int32_t(blockIdx.x * blockDim.x + threadIdx.x);
+    const int32_t t = gid(d);
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     float bx = 0.0f, by = 0.0f, bz = 0.0f;
@@ -315,7 +315,7 @@ template <int G> __global__ void __launch_bounds__(256) k_bcell_f32_g(DevMesh d,
 // zero where alpha_c B0_c is
 template <int G> __global__ void __launch_bounds__(256) k_hall_g_f32_g(DevMesh d, DevMesh32 s, const float *b, float *g)
 {
-    const int32_t t = int32_t(blockIdx.x * blockDim.x + threadIdx.x);
+    const int32_t t = gid(d);
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     // alpha B0 gates only the result: a test of it ahead of the neighbour gathers made every load of the cell wait
