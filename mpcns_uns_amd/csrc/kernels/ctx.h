@@ -9,6 +9,7 @@
 #include "../../../include/mhdg.h"
 #include "adjoint.h"
 #include "explicit_step.h"
+#include "flux_cell.h"
 #include "induction.h"
 #include "mixed.h"
 
@@ -153,6 +154,11 @@ struct mhdg_ctx
         return h_first;
     }
     double h_first[64]{};
+    mhdg::CellEdges ce{};
+    void flux_cell_build();
+    // phi = d1 x and b = its cell field in one launch, x = v, or dir ? 0 : v inv; false if the mesh has no tables for it
+    bool flux_cell(const double *v, const double *inv, const int8_t *dir, double *phi, double *b);
+    bool flux_cell(const float *pv, float *phi, float *b);
     void apply_op(const double *phi, const double *v, const double *inv, const int8_t *dir, double dt, int mode, int mask, const double *b,
                   double *out);
     // bvec = E_expl + F(Phi_n) and rvec = bvec - A x (no Jacobi scaling), the two products in one pass over the

@@ -287,6 +287,7 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     Btot = D(3 * C); uplus = D(3 * C); J = D(3 * C); alpha = D(C); B0 = D(3 * C);
     hip_check(hipMemset(alpha, 0, C * 8), "memset"); hip_check(hipMemset(B0, 0, 3 * C * 8), "memset");
     step_build(); // the layouts of the explicit stage
+    flux_cell_build();
     E_expl = D(E); E_last = D(E);
     dt_part = D(size_t(nblk(nc, 256 / P.ns)) + 1); dt_dev = D(1);
     // induction work
@@ -366,15 +367,21 @@ void mhdg_ctx::apply_op(const double *phi_in, const double *v, const double *inv
                         const double *b, double *out)
 {
     const double *phi = phi_in;
-    if (!phi)
+    const bool ideal_part = ideal_cfg && u_ideal, field = op_hall || ideal_part;
+    bool have_field = false;
+    if (!phi && field && !dte_cur && flux_cell(v, inv, dir, phi_w, bcell))
+    {
+        phi = phi_w;
+        have_field = true;
+    }
+    else if (!phi)
     {
         LAUNCH("d1", k_d1, dim3(nblk(nf)), dim3(256), 0, stream, d, v, inv, dir, dte_cur, phi_w);
         phi = phi_w;
         if (dte_cur) dt = 1.0; // d1 already carries dt_e: y = x + F (ImplicitInduction.cpp:196)
     }
-    const bool ideal_part = ideal_cfg && u_ideal;
     const int64_t lanes = kCellLanes64 * int64_t(nc);
-    if (op_hall || ideal_part) LAUNCH("bcell", k_bcell_g<kCellLanes64>, dim3(nblk(lanes)), dim3(256), 0, stream, d, phi, bcell);
+    if (field && !have_field) LAUNCH("bcell", k_bcell_g<kCellLanes64>, dim3(nblk(lanes)), dim3(256), 0, stream, d, phi, bcell);
     if (op_hall && lin_b) LAUNCH("hall_g_tangent", k_hall_g_tangent, dim3(nblk(nc)), dim3(256), 0, stream, d, lin_b, bcell, alpha, Badd, gcell);
     else if (op_hall) LAUNCH("hall_g", k_hall_g_g<kCellLanes64>, dim3(nblk(lanes)), dim3(256), 0, stream, d, bcell, alpha, B0, gcell);
     if (ideal_part)

@@ -256,10 +256,12 @@ void mhdg_ctx::op32(int mode, int hall_on, const float *pv, const float *v, cons
     MixedSolver &M = *mixed;
     const int8_t *dir = mg->dir_dev;
     const float dtf = mg->dt;
-    LAUNCH("d1_f32", k_d1_f32, dim3(nbk(nf)), dim3(256), 0, stream, d, M.s, pv, static_cast<const float *>(nullptr), M.phi);
+    const bool have_field = hall_on && flux_cell(pv, M.phi, M.b);
+    if (!have_field) LAUNCH("d1_f32", k_d1_f32, dim3(nbk(nf)), dim3(256), 0, stream, d, M.s, pv, static_cast<const float *>(nullptr), M.phi);
     if (hall_on)
     {
-        LAUNCH("bcell_f32", k_bcell_f32_g<kCellLanes>, dim3(nbk(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.phi, M.b);
+        if (!have_field)
+            LAUNCH("bcell_f32", k_bcell_f32_g<kCellLanes>, dim3(nbk(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.phi, M.b);
         LAUNCH("hall_g_f32", k_hall_g_f32_g<kCellLanes>, dim3(nbk(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.b, M.g);
     }
     const int32_t n_light = int32_t((int64_t(ne) + kEdgeBlock - 1) / kEdgeBlock);
