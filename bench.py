@@ -56,6 +56,8 @@ def kernel_bytes(mesh, name, precision_bytes=8, ns=2):
         "d1": E * b + F * b + 4 * (F + 1) + 4 * nf2e,
         # phi (F), recon (3 per c2f entry), b (3C) write, c2f ptr+idx
         "bcell": F * b + 3 * nc2f * 8 + 3 * C * b + 4 * (C + 1) + 4 * nc2f,
+        # x, invdiag, dir, the cell-edge tables (6 ids and 4 codes of a tetrahedron), face ids, recon, phi and b written
+        "flux_cell": 2 * E * 8 + E + 24 * C + 8 * nc2f + 3 * nc2f * 8 + F * 8 + 3 * C * 8,
         # b (3C), alpha (C), B0 (3C), area (3F), f2c (2F), volume, g (3C) write, c2f
         "hall_g": 3 * C * b + C * 8 + 3 * C * 8 + 3 * F * 8 + 8 * F + C * 8 + 3 * C * b + 4 * (C + 1) + 4 * nc2f,
         # phi, star2, e2f, g (3C), ec lists + weights, edge vec, m_e, v, invdiag, dir, out
@@ -75,6 +77,7 @@ def kernel_bytes(mesh, name, precision_bytes=8, ns=2):
         # FP32 operator of the mixed solve (int32 incidence, FP32 values)
         "d1_f32": 4 * (F + 1) + 4 * nf2e + 4 * E + 4 * E + E + 4 * F,
         "bcell_f32": 4 * (C + 1) + 4 * nc2f + 12 * nc2f + 4 * F + 12 * C,
+        "flux_cell_f32": 4 * E + 24 * C + 8 * nc2f + 12 * nc2f + 4 * F + 12 * C,
         # alpha B0 (3C), b (3C), c2f ptr + idx, f2c, area, volume, g (3C) write
         "hall_g_f32": 12 * C + 4 * (C + 1) + 4 * nc2f + 8 * F + 12 * F + 4 * C + 12 * C + 12 * C,
         # dir, the two rows in compact CSR form (row offsets + (index, weight) entries: e2f with signed star2, edge-cell
@@ -92,8 +95,8 @@ def kernel_bytes(mesh, name, precision_bytes=8, ns=2):
 
 KERNEL_CLASSES = {
     "explicit": ("prepare", "dt_final", "states", "fluxes", "update", "faraday", "gyrate"),
-    "operator": ("d1", "bcell", "hall_g", "edge_apply", "edge_apply_heavy", "d1_f32", "bcell_f32", "hall_g_f32", "edge_apply_f32",
-                 "mg_apply_f32"),
+    "operator": ("d1", "bcell", "flux_cell", "hall_g", "edge_apply", "d1_f32", "bcell_f32", "flux_cell_f32", "hall_g_f32",
+                 "edge_apply_f32", "mg_apply_f32"),
     "orthogonalisation": ("mgs", "finish", "dot", "multidot", "multidot_final", "multiaxpy", "scale", "multidot64", "multidot64_final",
                           "multiaxpy64", "norm64"),
     "multigrid": ("mg_first", "mg_smooth_f32", "mg_resid_f32", "mg_sweep", "mg_resid", "mg_restrict", "mg_prolong", "mg_dinv"),
