@@ -383,7 +383,7 @@ void mhdg_ctx::apply_op(const double *phi_in, const double *v, const double *inv
     const int64_t lanes = kCellLanes64 * int64_t(nc);
     if (field && !have_field) LAUNCH("bcell", k_bcell_g<kCellLanes64>, dim3(nblk(lanes)), dim3(256), 0, stream, d, phi, bcell);
     if (op_hall && lin_b) LAUNCH("hall_g_tangent", k_hall_g_tangent, dim3(nblk(nc)), dim3(256), 0, stream, d, lin_b, bcell, alpha, Badd, gcell);
-    else if (op_hall) LAUNCH("hall_g", k_hall_g_g<kCellLanes64>, dim3(nblk(lanes)), dim3(256), 0, stream, d, bcell, alpha, B0, gcell);
+    else if (op_hall) LAUNCH("hall_g", (d.xcd_ranges ? k_hall_g_g<kCellLanes64, true> : k_hall_g_g<kCellLanes64, false>), dim3(nblk(lanes)), dim3(256), 0, stream, d, bcell, alpha, B0, gcell);
     if (ideal_part)
     {
         // add_ideal_emf of (u, b, phi) with b as total and induced field (ImplicitInduction.cpp:150-157)

@@ -10,7 +10,9 @@ __global__ void k_bcell(DevMesh d, const double *phi, double *b);
 __global__ void k_hall_g(DevMesh d, const double *b, const double *alpha, const double *B0, double *g);
 constexpr int kCellLanes64 = 4; // lanes per cell of the FP64 cell kernels of apply_F
 template <int G> __global__ void k_bcell_g(DevMesh d, const double *phi, double *b);
-template <int G> __global__ void k_hall_g_g(DevMesh d, const double *b, const double *alpha, const double *B0, double *g);
+// NEAR: near_block's order (dev.h), on meshes with xcd_ranges.  An instantiation, not a test: forming the index from the
+// mesh's flag and the grid's size delays a short kernel's first loads (8M tetrahedra: this one 311 -> 330 us, FP32 149 -> 171).
+template <int G, bool NEAR> __global__ void k_hall_g_g(DevMesh d, const double *b, const double *alpha, const double *B0, double *g);
 // dynamic LDS of the edge kernels' heavy blocks, in doubles per unit of the largest valence
 constexpr int kApplyHeavyRows = 3, kResidualHeavyRows = 6;
 __global__ void k_edge_apply(DevMesh d, int32_t resistive, int32_t hall, const double *phi, const double *g, const double *ide,

@@ -18,7 +18,7 @@ __global__ void __launch_bounds__(256) k_div_scalar(const double *r, const doubl
 __global__ void __launch_bounds__(256) k_d1(DevMesh d, const double *v, const double *invdiag, const int8_t *dir, const double *dte,
                                             double *phi)
 {
-    const int32_t f = gid(d);
+    const int32_t f = gid();
     if (f >= d.nf) return;
     double s = 0.0;
     if (d.fdeg == 3 && !dte)
@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(256) k_hall_g(DevMesh d, const double *b, cons
 // runs in the order of the one-thread kernels and the results are the same bit for bit.
 template <int G> __global__ void __launch_bounds__(256) k_bcell_g(DevMesh d, const double *phi, double *b)
 {
-    const int32_t t = gid(d);
+    const int32_t t = gid();
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     // a fixed row length (tetrahedra) spares the row-bound loads ahead of the gathers
@@ -174,9 +174,10 @@ template <int G> __global__ void __launch_bounds__(256) k_bcell_g(DevMesh d, con
     }
     if (ok && lane == 0) { b[3 * size_t(c)] = bx; b[3 * size_t(c) + 1] = by; b[3 * size_t(c) + 2] = bz; }
 }
-template <int G> __global__ void __launch_bounds__(256) k_hall_g_g(DevMesh d, const double *b, const double *alpha, const double *B0, double *g)
+template <int G, bool NEAR>
+__global__ void __launch_bounds__(256) k_hall_g_g(DevMesh d, const double *b, const double *alpha, const double *B0, double *g)
 {
-    const int32_t t = gid(d);
+    const int32_t t = NEAR ? gid(d) : gid();
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     const double a = ok ? alpha[c] : 0.0;
@@ -215,7 +216,8 @@ template <int G> __global__ void __launch_bounds__(256) k_hall_g_g(DevMesh d, co
     if (ok && lane == 0) st3(g, c, out);
 }
 template __global__ void k_bcell_g<kCellLanes64>(DevMesh, const double *, double *);
-template __global__ void k_hall_g_g<kCellLanes64>(DevMesh, const double *, const double *, const double *, double *);
+template __global__ void k_hall_g_g<kCellLanes64, false>(DevMesh, const double *, const double *, const double *, double *);
+template __global__ void k_hall_g_g<kCellLanes64, true>(DevMesh, const double *, const double *, const double *, double *);
 
 // The row of the result from the edge's two sums
 __device__ __forceinline__ void edge_apply_out(const DevMesh &d, int32_t e, double p0, double p1, const double *ide, const int8_t *imask,
@@ -362,7 +364,7 @@ __global__ void __launch_bounds__(256) k_edge_apply(DevMesh d, int32_t resistive
 // k_bcell_g, k_hall_g_g and k_edge_apply, so b and r0 are the same bits as the two separate products give.
 template <int G> __global__ void __launch_bounds__(256) k_bcell2_g(DevMesh d, const double *phi1, const double *phi2, double *b1, double *b2)
 {
-    const int32_t t = gid(d);
+    const int32_t t = gid();
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     const int32_t k0 = !ok ? 0 : d.cdeg > 0 ? c * d.cdeg : d.c2f_ptr[c];
@@ -399,7 +401,7 @@ template <int G>
 __global__ void __launch_bounds__(256) k_hall_g2_g(DevMesh d, const double *b1, const double *b2, const double *alpha, const double *B0,
                                                    double *g1, double *g2)
 {
-    const int32_t t = gid(d);
+    const int32_t t = gid();
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     const double a = ok ? alpha[c] : 0.0;

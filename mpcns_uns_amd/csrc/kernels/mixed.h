@@ -41,7 +41,7 @@ constexpr int kEdgeBlock = 256; // threads per block of the FP32 edge kernel (a 
 __global__ void k_d1_f32(DevMesh d, DevMesh32 s, const float *pv, const float *dte, float *phi);
 constexpr int kCellLanes = 4; // lanes per cell of the FP32 cell kernels
 template <int G> __global__ void k_bcell_f32_g(DevMesh d, DevMesh32 s, const float *phi, float *b);
-template <int G> __global__ void k_hall_g_f32_g(DevMesh d, DevMesh32 s, const float *b, float *g);
+template <int G, bool NEAR> __global__ void k_hall_g_f32_g(DevMesh d, DevMesh32 s, const float *b, float *g);
 enum : int { kOpShifted = 0, kOpApply = 1, kOpSmooth = 2, kOpResid = 3 }; // output modes of k_edge_apply_f32 (mixed.hip)
 template <int MODE>
 __global__ void k_edge_apply_f32(DevMesh d, DevMesh32 s, int32_t resistive, int32_t hall, const float *phi, const float *g, const float *v,

@@ -58,7 +58,7 @@ __device__ __forceinline__ void rows(int32_t deg, const int32_t *ptr, int32_t r,
 // Phi'_f = sum_k f2e_k pv_e with pv = P v (0 on Dirichlet edges), times dt_e with a per-edge step
 __global__ void __launch_bounds__(256) k_d1_f32(DevMesh d, DevMesh32 s, const float *pv, const float *dte, float *phi)
 {
-    const int32_t f = gid(d);
+    const int32_t f = gid();
     if (f >= d.nf) return;
     if (s.fdeg == 3 && !dte)
     {
@@ -287,7 +287,7 @@ template <int G> __device__ __forceinline__ float group_sum(float v)
 }
 template <int G> __global__ void __launch_bounds__(256) k_bcell_f32_g(DevMesh d, DevMesh32 s, const float *phi, float *b)
 {
-    const int32_t t = gid(d);
+    const int32_t t = gid();
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     float bx = 0.0f, by = 0.0f, bz = 0.0f;
@@ -313,9 +313,9 @@ template <int G> __global__ void __launch_bounds__(256) k_bcell_f32_g(DevMesh d,
 }
 // g_c = J_c x (alpha_c B0_c) with J_c = sum_k (s A_f / V_c)_k x b_f, b_f the face average with the neighbour;
 // zero where alpha_c B0_c is
-template <int G> __global__ void __launch_bounds__(256) k_hall_g_f32_g(DevMesh d, DevMesh32 s, const float *b, float *g)
+template <int G, bool NEAR> __global__ void __launch_bounds__(256) k_hall_g_f32_g(DevMesh d, DevMesh32 s, const float *b, float *g)
 {
-    const int32_t t = gid(d);
+    const int32_t t = NEAR ? gid(d) : gid();
     const int32_t c = t / G, lane = t % G;
     const bool ok = c < d.nc;
     // alpha B0 gates only the result: a test of it ahead of the neighbour gathers made every load of the cell wait
@@ -365,7 +365,8 @@ template <int G> __global__ void __launch_bounds__(256) k_hall_g_f32_g(DevMesh d
     }
 }
 template __global__ void k_bcell_f32_g<4>(DevMesh, DevMesh32, const float *, float *);
-template __global__ void k_hall_g_f32_g<4>(DevMesh, DevMesh32, const float *, float *);
+template __global__ void k_hall_g_f32_g<4, false>(DevMesh, DevMesh32, const float *, float *);
+template __global__ void k_hall_g_f32_g<4, true>(DevMesh, DevMesh32, const float *, float *);
 
 // The same for the high-valence edges, one block per edge (tree sums: order-free in FP32)
 // Operator table of the FP32 path: per (cell, face) s A_f / V_c and the neighbour across the face
@@ -710,7 +711,7 @@ int mhdg_ctx::solve_mixed(const double *Phi_n, const double *Eex, const int8_t *
                 {
                     if (!have_field)
                         LAUNCH("bcell_f32", k_bcell_f32_g<kCellLanes>, dim3(nb(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.phi, M.b);
-                    LAUNCH("hall_g_f32", k_hall_g_f32_g<kCellLanes>, dim3(nb(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.b, M.g);
+                    LAUNCH("hall_g_f32", (d.xcd_ranges ? k_hall_g_f32_g<kCellLanes, true> : k_hall_g_f32_g<kCellLanes, false>), dim3(nb(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.b, M.g);
                 }
                 const int32_t n_light = int32_t((int64_t(ne) + kEdgeBlock - 1) / kEdgeBlock);
                 LAUNCH("edge_apply_f32", k_edge_apply_f32<kOpShifted>, dim3(n_light + n_heavy), dim3(kEdgeBlock), 0, stream, d, M.s,

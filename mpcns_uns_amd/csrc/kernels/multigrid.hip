@@ -262,7 +262,7 @@ void mhdg_ctx::op32(int mode, int hall_on, const float *pv, const float *v, cons
     {
         if (!have_field)
             LAUNCH("bcell_f32", k_bcell_f32_g<kCellLanes>, dim3(nbk(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.phi, M.b);
-        LAUNCH("hall_g_f32", k_hall_g_f32_g<kCellLanes>, dim3(nbk(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.b, M.g);
+        LAUNCH("hall_g_f32", (d.xcd_ranges ? k_hall_g_f32_g<kCellLanes, true> : k_hall_g_f32_g<kCellLanes, false>), dim3(nbk(kCellLanes * int64_t(nc))), dim3(256), 0, stream, d, M.s, M.b, M.g);
     }
     const int32_t n_light = int32_t((int64_t(ne) + kEdgeBlock - 1) / kEdgeBlock);
     const dim3 grid(n_light + n_heavy), block(kEdgeBlock);
