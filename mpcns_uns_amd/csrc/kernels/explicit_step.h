@@ -33,8 +33,8 @@ struct StepRun
 // How far a stage goes: no update of the state, of its cells, of its cells and faces
 enum StageEnd { kStageNone, kStageCells, kStageState };
 enum : int8_t { kFluxNone = 0, kFluxInner = 1, kFluxLeft = 2, kFluxRight = 3 };
-// Up to this many bytes of a step's fields and tables (620k tetrahedra, two ions) the XCDs take one range each of every
-// kernel's blocks (near_block, dev.h).  Microseconds per explicit step without and with: 9.5k tetrahedra 40.0, 35.9; 60k 67.7,
+// Up to this many bytes of a step's fields and tables (620k tetrahedra, two ions) the XCDs take one range each of the
+// step's and the products' blocks (near_block, dev.h).  Microseconds per explicit step without and with: 9.5k tetrahedra 40.0, 35.9; 60k 67.7,
 // 59.3; 150k (125 MB) 126.7, 114.2; 484k (400 MB) 399.6, 395.7; 1.09M (910 MB) 888, 919; 7.8M 6230, 6454: data that passes through
 // the L2s and the MALL from HBM is read best in one sweep by all XCDs.
 constexpr size_t kXcdBytes = size_t(512) << 20;
