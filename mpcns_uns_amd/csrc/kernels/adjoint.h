@@ -22,10 +22,18 @@ struct AdjFields
     double *Jv, *Btb;                     // per cell, 3: adjoint of the current over the volume; of B_tot
     double *sE, *sPhi, *eF, *eC;
     double *Phib, *PhiAddb, *Baddb;
-    double *e_part, *c_part;              // per block: {dt, E_inf (3, summed over the steps)} of the edges, dt of the cells
-    double *f_part, *g_part;              // per block, summed over the steps: free stream (10) from the fluxes, the gradients
-    double *dtb;                          // 16: adjoint of the time step, then (W 10, B_tot 3) of the cell that sets it
+    // adjoint of the time step: per 256-face block, per cell, per 256-cell block; then (dtb, 14) the total and the
+    // derivatives of the step of the cell that sets it by its W (10) and B_tot (3)
+    double *dt_f, *dt_c, *dt_cp, *dtb;
     int32_t *dt_cell;                     // that cell (-1: none), and how many sweeps did not find it
-    double *sums;                         // 23: the sums of e_part's E_inf, f_part and g_part
+    // The free stream's and the inflow EMF's adjoints come from the few 256-entity blocks that touch the inflow: a block's
+    // slot or -1, the block of a slot, the rows (10 per entity) of a slot's entities, the blocks' sums
+    const int32_t *fs_face, *fs_cell, *inflow_edge, *block_face, *block_cell;
+    int32_t n_f, n_c, n_e;
+    double *fsf, *fsc, *f_part, *g_part, *e_part;
+    const int32_t *wall_slot, *wall_cell; // per cell: its number among the cells with a wall in the stencil, or -1; their list
+    int32_t n_wall;
+    double *mirror;                       // per wall cell: the parts of the first ion's velocities (3) in its gradients
+    double *sums;                         // 14: free stream (10), inflow EMF (3), the second of dt_cell
 };
 } // namespace mhdg
