@@ -39,6 +39,12 @@ struct Complex
     void build_up();
     void edge_nodes(int32_t e, int32_t &a, int32_t &b) const;
     void face_loop(int32_t f, int32_t *nodes, int &n) const; // node at which each loop edge is entered
+    void face_loop(int32_t f, std::vector<int32_t> &nodes) const
+    {
+        int n = 0;
+        nodes.resize(size_t(f2e.ptr[f + 1] - f2e.ptr[f]));
+        face_loop(f, nodes.data(), n);
+    }
 };
 
 // Combinatorial checks (reference Validate.cpp:18-69): number of violations of each invariant.

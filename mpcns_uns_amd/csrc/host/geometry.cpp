@@ -13,18 +13,16 @@ namespace mhdg
 namespace
 {
 // unique sorted node list of a cell (all its face loops)
-int cell_nodes(const Complex &cx, int32_t c, int32_t *out)
+void cell_nodes(const Complex &cx, int32_t c, std::vector<int32_t> &out, std::vector<int32_t> &loop)
 {
-    int n = 0;
-    int32_t loop[8];
-    int m;
+    out.clear();
     for (int64_t k = cx.c2f.ptr[c]; k < cx.c2f.ptr[c + 1]; ++k)
     {
-        cx.face_loop(cx.c2f.idx[k], loop, m);
-        for (int i = 0; i < m; ++i) out[n++] = loop[i];
+        cx.face_loop(cx.c2f.idx[k], loop);
+        out.insert(out.end(), loop.begin(), loop.end());
     }
-    std::sort(out, out + n);
-    return static_cast<int>(std::unique(out, out + n) - out);
+    std::sort(out.begin(), out.end());
+    out.erase(std::unique(out.begin(), out.end()), out.end());
 }
 
 // dual piece of the i-th loop edge of face f (c2f sign s) inside cell c with centre xc
@@ -66,9 +64,9 @@ Geometry compute_geometry(const Complex &cx, const double *xyz)
 #pragma omp parallel for schedule(static)
     for (int32_t f = 0; f < nf; ++f)
     {
-        int32_t loop[8];
-        int k;
-        cx.face_loop(f, loop, k);
+        thread_local std::vector<int32_t> loop;
+        cx.face_loop(f, loop);
+        const int k = static_cast<int>(loop.size());
         V3 p0;
         for (int i = 0; i < k; ++i) p0 += ld3(xyz, loop[i]);
         p0 *= 1.0 / static_cast<double>(k);
@@ -127,8 +125,9 @@ Geometry compute_geometry(const Complex &cx, const double *xyz)
 #pragma omp parallel for schedule(static)
     for (int32_t c = 0; c < nc; ++c)
     {
-        int32_t cn[64], loop[8];
-        const int nn = cell_nodes(cx, c, cn);
+        thread_local std::vector<int32_t> cn, loop;
+        cell_nodes(cx, c, cn, loop);
+        const int nn = static_cast<int>(cn.size());
         V3 xc0;
         for (int i = 0; i < nn; ++i) xc0 += ld3(xyz, cn[i]);
         xc0 *= 1.0 / static_cast<double>(nn);
@@ -138,8 +137,8 @@ Geometry compute_geometry(const Complex &cx, const double *xyz)
         {
             const int32_t f = cx.c2f.idx[kf];
             const int s = cx.c2f.sgn[kf];
-            int k;
-            cx.face_loop(f, loop, k);
+            cx.face_loop(f, loop);
+            const int k = static_cast<int>(loop.size());
             const V3 cf = ld3(g.face_center.data(), f);
             for (int i = 0; i < k; ++i)
             {
@@ -157,8 +156,8 @@ Geometry compute_geometry(const Complex &cx, const double *xyz)
         {
             const int32_t f = cx.c2f.idx[kf];
             const int s = cx.c2f.sgn[kf];
-            int k;
-            cx.face_loop(f, loop, k);
+            cx.face_loop(f, loop);
+            const int k = static_cast<int>(loop.size());
             const V3 cf = ld3(g.face_center.data(), f);
             for (int i = 0; i < k; ++i)
             {

@@ -140,3 +140,32 @@ def mixed_workload(hall, nx=6, ny=5, nz=4, jitter=0.1, seed=13, noise=0.01, **cf
     PhiAdd, Badd = mesh.background(workloads.B_IMF, workloads.DIPOLE_M, (0.0, 0.0, 0.0), 1e-3)
     UH, UNa, Phi = mesh.seeded_state(cfg, noise, seed, Badd)
     return dict(mesh=mesh, cfg=cfg, state=(UH, UNa, Phi), background=(PhiAdd, Badd), cells=cells, tags=tags, xyz=xyz)
+
+
+def polyhedron(n_lon=12, n_ring=3, centre=(2.5, 0.0, 0.0), radii=(0.4, 0.9)):
+    """Nodes, cells and tags: the triangulated sphere of n_ring rings and two poles as one cell, and a prism on each face."""
+    rng = np.random.default_rng(3)
+    th = np.pi * np.arange(1, n_ring + 1) / (n_ring + 1)
+    unit = [(0.0, 0.0, 1.0)]
+    for k, t in enumerate(th):
+        for j in range(n_lon):
+            p = 2 * np.pi * (j + 0.5 * k) / n_lon
+            unit.append((np.sin(t) * np.cos(p), np.sin(t) * np.sin(p), np.cos(t)))
+    unit.append((0.0, 0.0, -1.0))
+    unit = np.array(unit)
+    ring = lambda k, j: 1 + k * n_lon + j % n_lon
+    tri = [(0, ring(0, j), ring(0, j + 1)) for j in range(n_lon)]
+    for k in range(n_ring - 1):
+        for j in range(n_lon):
+            tri += [(ring(k, j), ring(k + 1, j), ring(k, j + 1)), (ring(k, j + 1), ring(k + 1, j), ring(k + 1, j + 1))]
+    last = len(unit) - 1
+    tri += [(ring(n_ring - 1, j), last, ring(n_ring - 1, j + 1)) for j in range(n_lon)]
+    n = len(unit)
+    r = radii[0] * (1 + 0.1 * rng.random(n)), radii[1] * (1 + 0.1 * rng.random(n))
+    xyz = np.concatenate([np.array(centre) + unit * r[0][:, None], np.array(centre) + unit * r[1][:, None]])
+    cells = [[list(t) for t in tri]]
+    for a, b, c in tri:
+        A, B, C = a + n, b + n, c + n
+        cells.append([[c, b, a], [A, B, C], [a, b, B, A], [b, c, C, B], [c, a, A, C]])
+    tags = [([v + n for v in t], 1 if k % 3 == 0 else 2) for k, t in enumerate(tri) if k % 3 < 2]
+    return xyz, cells, tags

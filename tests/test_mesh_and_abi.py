@@ -208,3 +208,16 @@ def test_converted_inputs_outlive_the_call():
     flux = np.random.default_rng(0).normal(size=m.n_faces)
     assert np.array_equal(m.cell_vector(flux.astype(np.float32)), m.cell_vector(flux.astype(np.float32).astype(np.float64)))
     assert np.array_equal(m.cell_vector(list(flux)), m.cell_vector(flux))
+
+
+def test_cells_of_many_faces():
+    """A cell of 72 triangles (216 loop nodes) inside 72 prisms: its volume is that of the divergence theorem."""
+    from meshes import polyhedron
+
+    from mpcns_uns_amd import Mesh
+
+    xyz, cells, _ = polyhedron()
+    mesh = Mesh.from_cells(xyz, cells)
+    assert (mesh.n_cells, mesh.n_faces, mesh.n_edges) == (73, 72 * 2 + 108, 108 * 2 + 38)
+    inner = sum(np.dot(xyz[a], np.cross(xyz[b], xyz[c])) for a, b, c in cells[0]) / 6
+    assert abs(mesh.array("cell_volume")[0] - inner) <= 1e-13
