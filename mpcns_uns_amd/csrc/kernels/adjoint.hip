@@ -1046,21 +1046,22 @@ struct StencilInverse
         return V3(a * r.x + b * r.y + c * r.z, b * r.x + d * r.y + e * r.z, c * r.x + e * r.y + f * r.z);
     }
 };
-// A primitive's gradient g, its limiter psi and what sets it: the entry (+ 64 by the relative limit, -1: none), the offset x
-// of its face with dl = g . x, and whose the extremes are (source)
+// A primitive's gradient g, its limiter psi and what sets it (kNoLimit: nothing): the room to an extreme or the relative
+// limit over dl = g . x, x the offset of its face; and whose the extremes are (source)
+enum : int32_t { kNoLimit, kRoom, kRelative };
 struct Limited
 {
     V3 g, x;
     double psi, dl;
-    int32_t act, hs, ls;
+    int32_t by, hs, ls;
     // the derivative of psi g along an input that moves g by gd, the extremes by hd and ld and the cell's value by wd
     __device__ __forceinline__ V3 column(const Params &P, const V3 &gd, double hd, double ld, double wd) const
     {
         double pd = 0.0;
-        if (act >= 0)
+        if (by != kNoLimit)
         {
             double dld = gd.x * x.x + gd.y * x.y + gd.z * x.z, num, den = dl;
-            if (act >= 64)
+            if (by == kRelative)
             {
                 num = P.rel_limit * wd;
                 if (dl < 0) { dld = -dld; den = -dl; }
@@ -1089,7 +1090,7 @@ template <int DEG> __device__ __forceinline__ Limited limited(const Params &P, c
     }
     L.g = inv(r);
     L.psi = 1.0;
-    L.act = -1;
+    L.by = kNoLimit;
     L.dl = 0.0;
     // psi = max(0, min(1, quotients)): the first smallest quotient below 1 counts, unless it is not above 0
 #pragma unroll
@@ -1097,7 +1098,7 @@ template <int DEG> __device__ __forceinline__ Limited limited(const Params &P, c
     {
         const V3 x = row.dx(i);
         const double dl = L.g.x * x.x + L.g.y * x.y + L.g.z * x.z, q = (dl > 0 ? hi - w : lo - w) / dl;
-        if (fabs(dl) > 1e-300 && q < L.psi) { L.psi = q; L.act = i; L.x = x; L.dl = dl; }
+        if (fabs(dl) > 1e-300 && q < L.psi) { L.psi = q; L.by = kRoom; L.x = x; L.dl = dl; }
     }
     if (P.rel_limit > 0 && (m == 0 || m == 4))
 #pragma unroll
@@ -1105,26 +1106,32 @@ template <int DEG> __device__ __forceinline__ Limited limited(const Params &P, c
         {
             const V3 x = row.dx(i);
             const double dl = L.g.x * x.x + L.g.y * x.y + L.g.z * x.z, q = P.rel_limit * w / fabs(dl);
-            if (fabs(dl) > 1e-300 && q < L.psi) { L.psi = q; L.act = i + 64; L.x = x; L.dl = dl; }
+            if (fabs(dl) > 1e-300 && q < L.psi) { L.psi = q; L.by = kRelative; L.x = x; L.dl = dl; }
         }
-    if (!(L.psi > 0.0)) { L.psi = 0.0; L.act = -1; }
+    if (!(L.psi > 0.0)) { L.psi = 0.0; L.by = kNoLimit; }
     return L;
 }
-// the entries whose state is the linear one (else it is the cell's own): a face state depends on the gradient there
-template <int DEG>
-__device__ __forceinline__ uint64_t linear_entries(const StencilRow<DEG> &row, const Limited &rho, const Limited &p)
+// Whether an entry's state is the linear one (else it is the cell's own): a face state depends on the gradient there.  A bit
+// per entry of a fixed row; walked rows, which may be longer than a word, form it again.
+template <int DEG> struct LinearEntries
 {
-    uint64_t linear = 0;
-    const V3 a(rho.psi * rho.g.x, rho.psi * rho.g.y, rho.psi * rho.g.z), b(p.psi * p.g.x, p.psi * p.g.y, p.psi * p.g.z);
+    V3 a, b; // the limited gradients of density and pressure
+    uint32_t bits = 0;
+    __device__ __forceinline__ LinearEntries(const StencilRow<DEG> &row, const Limited &rho, const Limited &p)
+        : a(rho.psi * rho.g.x, rho.psi * rho.g.y, rho.psi * rho.g.z), b(p.psi * p.g.x, p.psi * p.g.y, p.psi * p.g.z)
+    {
+        if constexpr (DEG > 0)
 #pragma unroll
-    for (int i = 0; i < row.count(); ++i)
+            for (int i = 0; i < DEG; ++i) bits |= uint32_t(positive(row, i)) << i;
+    }
+    __device__ __forceinline__ bool positive(const StencilRow<DEG> &row, int i) const
     {
         const V3 x = row.dx(i);
         const double rr = row.wc[0] + a.x * x.x + a.y * x.y + a.z * x.z, pp = row.wc[4] + b.x * x.x + b.y * x.y + b.z * x.z;
-        if (rr > 0 && pp > 0) linear |= uint64_t(1) << i;
+        return rr > 0 && pp > 0;
     }
-    return linear;
-}
+    __device__ __forceinline__ bool operator()(const StencilRow<DEG> &row, int i) const { return DEG > 0 ? bits >> i & 1 : positive(row, i); }
+};
 } // namespace
 
 // The first ion's velocities of a wall cell, which its mirror image couples: thread (wall cell, component j), the part of
@@ -1143,7 +1150,7 @@ template <int DEG> __global__ void __launch_bounds__(64, 2) k_adj_mirror(DevMesh
         for (int i = 0; i < DEG; ++i) st3(offsets, i, L3(d.fcen, pid(row.v[i])) - row.xc); // this thread's own
     const StencilInverse inv(d.sinv + 6 * size_t(c));
     auto bar = [&](int i) { return F.FS + 5 * (size_t(row.k0 + i) * kAdjNs); };
-    const uint64_t linear = linear_entries(row, limited(P, row, inv, 0), limited(P, row, inv, 4));
+    const LinearEntries<DEG> linear(row, limited(P, row, inv, 0), limited(P, row, inv, 4));
     double sum = 0.0;
 #pragma unroll
     for (int m = 1; m <= 3; ++m)
@@ -1155,7 +1162,7 @@ template <int DEG> __global__ void __launch_bounds__(64, 2) k_adj_mirror(DevMesh
 #pragma unroll
         for (int i = 0; i < row.count(); ++i)
         {
-            if (linear >> i & 1) gb += bar(i)[m] * row.dx(i);
+            if (linear(row, i)) gb += bar(i)[m] * row.dx(i);
             double nd = row.source(i) == kOwnCell ? wd : 0.0; // the entry's value along velocity j
             if (row.kind(i) == kWall)
             {
@@ -1236,14 +1243,14 @@ __global__ void __launch_bounds__(kGradThreads, 2) k_adj_gradients(DevMesh d, Pa
             const StencilRow<DEG> row(d, P, F, c, s, offsets);
             const StencilInverse inv(d.sinv + 6 * size_t(c));
             Limited L = limited(P, row, inv, 0);
-            const uint64_t linear = linear_entries(row, L, limited(P, row, inv, 4));
+            const LinearEntries<DEG> linear(row, L, limited(P, row, inv, 4));
             // I times the sum of w d dq along the cell's own primitive; a value that follows the cell's adds nothing
             bool nz = false, inflow = false; // some gradient has an adjoint; a face of the inflow
             V3 rc;
 #pragma unroll
             for (int i = 0; i < row.count(); ++i)
             {
-                for (int m = 0; m < 5; ++m) nz = nz || ((linear >> i & 1) && bar(i)[m] != 0.0);
+                for (int m = 0; m < 5; ++m) nz = nz || (linear(row, i) && bar(i)[m] != 0.0);
                 inflow = inflow || row.source(i) == kFree;
                 if (row.source(i) != kOwnCell) rc -= row.weighted(i);
             }
@@ -1259,7 +1266,7 @@ __global__ void __launch_bounds__(kGradThreads, 2) k_adj_gradients(DevMesh d, Pa
                 {
                     const double b = bar(i)[m];
                     sum += b;
-                    if (linear >> i & 1) gb += b * row.dx(i);
+                    if (linear(row, i)) gb += b * row.dx(i);
                 }
                 auto weigh = [&](const V3 &o) { return gb.x * o.x + gb.y * o.y + gb.z * o.z; };
                 sum = wb[m] + sum;
