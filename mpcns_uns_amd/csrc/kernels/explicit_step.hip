@@ -45,13 +45,17 @@ __global__ void __launch_bounds__(256) k_face_entries(DevMesh d, int2 *fent, int
     const int32_t f = gid();
     if (f >= d.nf) return;
     const int32_t l = d.fL[f], r = d.fR[f];
-    auto entry = [&](int32_t c) {
-        if (c < 0) return -1;
-        for (int32_t k = d.c2f_ptr[c]; k < d.c2f_ptr[c + 1]; ++k)
-            if (pid(d.c2f[k]) == f) return k;
-        return -1;
+    // of a cell that sees the face from both sides, the entry of that side
+    auto entry = [&](int32_t c, int32_t v) {
+        int32_t any = -1;
+        for (int32_t k = c < 0 ? 0 : d.c2f_ptr[c]; c >= 0 && k < d.c2f_ptr[c + 1]; ++k)
+        {
+            if (d.c2f[k] == v) return k;
+            if (pid(d.c2f[k]) == f && any < 0) any = k;
+        }
+        return any;
     };
-    fent[f] = make_int2(entry(l), entry(r));
+    fent[f] = make_int2(entry(l, f), entry(r, ~f));
     const bool any = (l >= 0 && d.mat[l] == 0) || (r >= 0 && d.mat[r] == 0);
     int8_t cls;
     if (d.kind[f] == kSkip || !any) cls = kFluxNone;
