@@ -113,6 +113,7 @@ struct mhdg_ctx
     mhdg::StepRun resident_run();
     void step_build();
     void launch_prepare(const mhdg::StepRun &x);
+    void launch_current(const mhdg::StepRun &x);
     // n_face face-EMF blocks and (dt_out) the CFL minimum with them
     void launch_states(const mhdg::StepRun &x, int32_t n_face, double *dt_out, double dt_max);
     // the explicit stage; the state is untouched when it throws.  Returns the time step, checked (kStageNone: 0, unchecked)

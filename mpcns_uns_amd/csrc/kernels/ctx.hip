@@ -1064,7 +1064,7 @@ int mhdg_prepare(mhdg_ctx *c)
 {
     MHDG_TRY(c, {
         c->launch_prepare(c->resident_run());
-        c->launch_states(c->resident_run(), 0, nullptr, 0);
+        c->launch_current(c->resident_run());
         c->check_launch("prepare");
         hip_check(hipStreamSynchronize(c->stream), "sync");
     })

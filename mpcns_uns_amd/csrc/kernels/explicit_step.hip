@@ -613,6 +613,40 @@ __device__ __forceinline__ void update_role(const DevMesh &d, const Params &P, c
 }
 } // namespace
 
+// cell_current (Current.cpp:9-31) alone, of the fields in the records, for a caller that wants the derived fields of a state
+// and takes no step (7.83M tetrahedra: 493 us; the states, which form it on the side for a step, 1729)
+template <int DEG> __global__ void __launch_bounds__(kRoleThreads) k_step_current(DevMesh d, StepFields F)
+{
+    constexpr int N = DEG > 0 ? DEG : 1;
+    const int32_t c = gid(d);
+    if (c >= d.nc) return;
+    int32_t k0, nk;
+    row_of<DEG>(d, c, k0, nk);
+    auto field = [&](int32_t q) { return L3(F.rec + size_t(F.rs) * size_t(q) + 5 * F.ns, 0); };
+    const V3 bc = field(c);
+    V3 sum;
+    auto add = [&](int32_t v, int32_t o, const V3 &bo) {
+        V3 bf = bc;
+        if (o >= 0) bf = 0.5 * (bc + bo);
+        sum += cross(psg(v) * L3(d.farea, pid(v)), bf);
+    };
+    if constexpr (DEG > 0)
+    {
+        int32_t v[N], o[N];
+        V3 bo[N];
+        row_ids<DEG>(d.c2f, k0, v);
+        row_ids<DEG>(d.c2n, k0, o);
+#pragma unroll
+        for (int i = 0; i < DEG; ++i) bo[i] = field(o[i] >= 0 ? o[i] : c);
+#pragma unroll
+        for (int i = 0; i < DEG; ++i) add(v[i], o[i], bo[i]);
+    }
+    else
+        for (int32_t k = k0; k < k0 + nk; ++k) add(d.c2f[k], d.c2n[k], field(d.c2n[k] >= 0 ? d.c2n[k] : c));
+    const double invV = 1.0 / d.cvol[c];
+    st3(F.J, c, V3(sum.x * invV, sum.y * invV, sum.z * invV));
+}
+
 template <int DEG, int NS>
 __global__ void __launch_bounds__(kStatesThreads, DEG == 4 && NS == 0 ? 4 : 3) k_step_states(DevMesh d, Params P, StepFields F, const double *Phi, const double *PhiAdd,
                                                                    int32_t n_cell, int32_t n_face, const double *dt_part, int32_t n_part,
@@ -736,6 +770,13 @@ void mhdg_ctx::launch_states(const StepRun &x, int32_t n_face, double *dt_out, d
         LAUNCH("states", (k_step_states<decltype(deg)::value, decltype(ns)::value>), dim3(n_cell + n_face + (dt_out ? 1 : 0)),
                dim3(kStatesThreads), 0, stream, d, P, x.F, static_cast<const double *>(x.Phi), static_cast<const double *>(PhiAdd), n_cell, n_face,
                static_cast<const double *>(x.dt_part), n_part, dt_max, dt_out, dt_box, ticket);
+    });
+}
+
+void mhdg_ctx::launch_current(const StepRun &x)
+{
+    by_shape(cdeg, P.ns, [&](auto deg, auto) {
+        LAUNCH("current", k_step_current<decltype(deg)::value>, dim3(blocks(nc, kRoleThreads)), dim3(kRoleThreads), 0, stream, d, x.F);
     });
 }
 
