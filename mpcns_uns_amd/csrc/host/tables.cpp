@@ -107,7 +107,9 @@ Tables build_tables(const mhdg_mesh_desc &d, const mhdg_config &cfg, int32_t lig
     {
         const int32_t v = t.e2f_ptr[e + 1] - t.e2f_ptr[e];
         t.max_valence = std::max(t.max_valence, v);
-        if (v > light_max) t.heavy.push_back(e);
+        if (v <= light_max) continue;
+        t.heavy.push_back(e);
+        t.max_heavy_cells = std::max(t.max_heavy_cells, t.ec_ptr[e + 1] - t.ec_ptr[e]);
     }
 
     auto A3 = [&](const double *p, long i) { return V3(p[3 * i], p[3 * i + 1], p[3 * i + 2]); };

@@ -20,7 +20,7 @@ struct Tables
     std::vector<int8_t> svalid;
     std::vector<double> recon, m_e, d2, taper;
     std::vector<int32_t> heavy; // edges whose valence exceeds the one-thread limit
-    int32_t max_valence = 0;
+    int32_t max_valence = 0, max_heavy_cells = 0; // most faces of an edge; most cells of one in `heavy`
 };
 
 // Throws std::runtime_error on inconsistent input.

@@ -26,6 +26,7 @@ struct mhdg_ctx
     mhdg::Params P{};
     mhdg::DevMesh d{};
     int32_t nc = 0, nf = 0, ne = 0, n_heavy = 0, max_valence = 0;
+    int32_t heavy_len = 0; // a row of the products' heavy blocks: the largest valence, or half the cells of a heavy edge
     size_t c2f_nnz = 0, ec_nnz = 0, e2f_nnz = 0;
     int32_t cdeg = 0, fdeg = 0; // uniform faces per cell / edges per face (0: mixed shapes)
     void *heavy = nullptr;

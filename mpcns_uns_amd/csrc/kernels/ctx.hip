@@ -193,9 +193,11 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     hip_check(hipStreamCreate(&stream), "hipStreamCreate");
     Tables t = build_tables(m, c, kLightMax);
     if (t.max_valence > kHeavyMax) throw std::runtime_error("edge valence exceeds the supported maximum");
+    if (t.max_heavy_cells > 2 * kHeavyMax) throw std::runtime_error("cells around an edge exceed the supported maximum");
     nc = t.nc; nf = t.nf; ne = t.ne;
     n_heavy = static_cast<int32_t>(t.heavy.size());
     max_valence = t.max_valence;
+    heavy_len = std::max(max_valence, (t.max_heavy_cells + 1) / 2);
     c2f_nnz = t.c2f.size();
     ec_nnz = t.ec_cell.size();
     e2f_nnz = t.e2f.size();
@@ -393,9 +395,9 @@ void mhdg_ctx::apply_op(const double *phi_in, const double *v, const double *inv
         launch_edge_emf(Ef_i, u_ideal, P.cuct, nullptr, ide, 0);
     }
     const double *idp = ideal_part ? ide : nullptr;
-    const size_t lds = n_heavy ? kApplyHeavyRows * size_t(max_valence) * sizeof(double) : 0;
+    const size_t lds = n_heavy ? kApplyHeavyRows * size_t(heavy_len) * sizeof(double) : 0;
     LAUNCH("edge_apply", k_edge_apply, dim3(n_heavy + nblk(ne)), dim3(256), lds, stream, d, int32_t(op_res), int32_t(op_hall), phi, gcell, idp,
-           imask, v, inv, dir, dt, mode, mask, b, out, static_cast<const int32_t *>(heavy), n_heavy, max_valence);
+           imask, v, inv, dir, dt, mode, mask, b, out, static_cast<const int32_t *>(heavy), n_heavy, heavy_len);
     check_launch("apply_op");
 }
 
@@ -420,10 +422,10 @@ void mhdg_ctx::rhs_residual(const double *Phi_n, const double *Eex, const double
         LAUNCH("hall_g", k_hall_g2_g<kCellLanes64>, dim3(nblk(lanes)), dim3(256), 0, stream, d, static_cast<const double *>(bcell),
                static_cast<const double *>(bcell2), alpha, B0, gcell, gcell2);
     }
-    const size_t lds = n_heavy ? kResidualHeavyRows * size_t(max_valence) * sizeof(double) : 0;
+    const size_t lds = n_heavy ? kResidualHeavyRows * size_t(heavy_len) * sizeof(double) : 0;
     LAUNCH("edge_apply", k_edge_rhs_residual, dim3(n_heavy + nblk(ne)), dim3(256), lds, stream, d, int32_t(op_res), int32_t(op_hall), Phi_n,
            static_cast<const double *>(gcell), static_cast<const double *>(phi_w), static_cast<const double *>(gcell2), Eex, x, dir, dt, bvec,
-           rvec, static_cast<const int32_t *>(heavy), n_heavy, max_valence);
+           rvec, static_cast<const int32_t *>(heavy), n_heavy, heavy_len);
     check_launch("rhs_residual");
 }
 

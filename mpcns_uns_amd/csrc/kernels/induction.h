@@ -13,7 +13,7 @@ template <int G> __global__ void k_bcell_g(DevMesh d, const double *phi, double 
 // NEAR: near_block's order (dev.h), on meshes with xcd_ranges.  An instantiation, not a test: forming the index from the
 // mesh's flag and the grid's size delays a short kernel's first loads (8M tetrahedra: this one 311 -> 330 us, FP32 149 -> 171).
 template <int G, bool NEAR> __global__ void k_hall_g_g(DevMesh d, const double *b, const double *alpha, const double *B0, double *g);
-// dynamic LDS of the edge kernels' heavy blocks, in doubles per unit of the largest valence
+// dynamic LDS of the edge kernels' heavy blocks, in doubles per unit of hv (mhdg_ctx::heavy_len)
 constexpr int kApplyHeavyRows = 3, kResidualHeavyRows = 6;
 __global__ void k_edge_apply(DevMesh d, int32_t resistive, int32_t hall, const double *phi, const double *g, const double *ide,
                              const int8_t *imask, const double *v, const double *invdiag, const int8_t *dir, double dt, int32_t mode,

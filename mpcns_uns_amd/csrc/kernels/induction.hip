@@ -253,8 +253,8 @@ __device__ __forceinline__ double ordered_sum(const double *x, int32_t n)
     for (; i < n; ++i) s += x[i];
     return s;
 }
-// One high-valence edge per block: terms in parallel into LDS (hv the largest valence of the mesh: hv face terms, then up
-// to 2 hv cell terms), each sum sequential in the reference's order (faces ascending, cells ascending) on a wave of its own.
+// One high-valence edge per block: terms in parallel into LDS (hv face terms, then up to 2 hv cell terms: hv is the largest
+// valence, or half the most cells of such an edge), each sum sequential in the reference's order (faces ascending, cells ascending) on a wave of its own.
 __device__ __forceinline__ void edge_apply_heavy(const DevMesh &d, int32_t resistive, int32_t hall, int32_t e, const double *phi, const double *g,
                                                  const double *ide, const int8_t *imask, const double *v, const double *invdiag,
                                                  const int8_t *dir, double dt, int32_t mode, int32_t mask, const double *bvec, double *out,

@@ -110,11 +110,11 @@ void mhdg_ctx::apply_G(const double *phi, double *out)
         LAUNCH("field_of_flux", k_field_of_flux, dim3(nbk(3 * int64_t(nc))), dim3(256), 0, stream, Badd, bcell, 3 * int64_t(nc), nt.B0);
         LAUNCH("hall_g", k_hall_g, dim3(nbk(nc)), dim3(256), 0, stream, d, bcell, alpha, nt.B0, gcell);
     }
-    const size_t lds = n_heavy ? kApplyHeavyRows * size_t(max_valence) * sizeof(double) : 0;
+    const size_t lds = n_heavy ? kApplyHeavyRows * size_t(heavy_len) * sizeof(double) : 0;
     LAUNCH("edge_apply", k_edge_apply, dim3(n_heavy + nbk(ne)), dim3(256), lds, stream, d, int32_t(op_res), int32_t(op_hall), phi, gcell,
            static_cast<const double *>(nullptr), static_cast<const int8_t *>(nullptr), static_cast<const double *>(nullptr),
            static_cast<const double *>(nullptr), static_cast<const int8_t *>(nullptr), 0.0, 0, 0, static_cast<const double *>(nullptr), out,
-           static_cast<const int32_t *>(heavy), n_heavy, max_valence);
+           static_cast<const int32_t *>(heavy), n_heavy, heavy_len);
     check_launch("apply_G");
 }
 
