@@ -369,9 +369,8 @@ template <class R> __global__ void __launch_bounds__(256) k_face(DevMesh d, Para
             const R a = mx(fabs(dot(uL, n)), fabs(dot(uR, n)));
             F = 0.5 * (fLx + fRx) - (0.5 * a) * (L3(Bind, r) - L3(Bind, l));
         }
-        else
+        else if (const int32_t c = l >= 0 ? l : r; c >= 0) // zero on a face without a cell
         {
-            const int32_t c = l >= 0 ? l : r;
             const V3T<R> u = L3(uplus, c);
             F = dot(u, n) * L3(Btot, c) - Bn_tot * u;
         }

@@ -512,9 +512,8 @@ __device__ __forceinline__ void face_emf_role(const DevMesh &d, const StepFields
         const double a = mx(fabs(dot(uL, n)), fabs(dot(uR, n)));
         E = 0.5 * (fl + fr) - (0.5 * a) * (iR - iL);
     }
-    else
+    else if (const int32_t c = l >= 0 ? l : r; c >= 0) // zero on a face without a cell
     {
-        const int32_t c = l >= 0 ? l : r;
         const V3 u = L3(F.uplus, c);
         E = dot(u, n) * L3(F.Btot, c) - Bn_tot * u;
     }
