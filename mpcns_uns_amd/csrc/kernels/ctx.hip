@@ -213,8 +213,7 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     const size_t E = ne, F = nf, C = nc;
     d.nc = nc; d.nf = nf; d.ne = ne;
     d.cdeg = cdeg; d.fdeg = fdeg;
-    // the bytes of a step's fields and tables, about
-    d.xcd_ranges = 8 * (size_t(step_row(P.ns)) * C + 5 * P.ns * (c2f_nnz + F + C) + 20 * F + 20 * C) <= kXcdBytes;
+    d.xcd_ranges = step_bytes(P.ns, C, F, c2f_nnz) <= kXcdBytes;
     d.c2f_ptr = upload(t.c2f_ptr); d.c2f = upload(t.c2f); d.cfs = upload(t.cfs);
     d.f2e_ptr = upload(t.f2e_ptr); d.f2e = upload(t.f2e);
     d.e2f_ptr = upload(t.e2f_ptr); d.e2f = upload(t.e2f);

@@ -33,12 +33,20 @@ struct StepRun
 // How far a stage goes: no update of the state, of its cells, of its cells and faces
 enum StageEnd { kStageNone, kStageCells, kStageState };
 enum : int8_t { kFluxNone = 0, kFluxInner = 1, kFluxLeft = 2, kFluxRight = 3 };
-// Up to this many bytes of a step's fields and tables (620k tetrahedra, two ions) the XCDs take one range each of the
-// step's and the products' blocks (near_block, dev.h).  Microseconds per explicit step without and with: 9.5k tetrahedra 40.0, 35.9; 60k 67.7,
-// 59.3; 150k (125 MB) 126.7, 114.2; 484k (400 MB) 399.6, 395.7; 1.09M (910 MB) 888, 919; 7.8M 6230, 6454: data that passes through
-// the L2s and the MALL from HBM is read best in one sweep by all XCDs.
-constexpr size_t kXcdBytes = size_t(512) << 20;
 inline int32_t step_row(int32_t ns) { return (5 * ns + 6 + 7) / 8 * 8; }
+// The bytes of a step's fields and tables, about: 1170 a tetrahedron with two ions, 3750 with ten
+inline size_t step_bytes(int32_t ns, size_t cells, size_t faces, size_t entries)
+{
+    return 8 * (size_t(step_row(ns)) * cells + 5 * size_t(ns) * (entries + faces + cells) + 20 * faces + 20 * cells);
+}
+// Up to this many of them (457k tetrahedra with two ions, 143k with ten) the XCDs take one range each of the step's and the
+// products' blocks (near_block, dev.h) and the products' first launch is flux_cell's.  Microseconds without and with the
+// order, forced either way.  Two ions, an explicit step: 9.5k tetrahedra 40.5, 36.8; 60k 67.8, 59.3; 150k 127, 114;
+// 290k 246, 239; 435k 362, 355; above the line 484k 401, 396; 683k 556, 562; 1.06M 850, 890; 7.8M 6230, 6454.  Ten ions, an
+// explicit step and a mixed Hall step (with flux_cell): 60k 164, 519 and 164, 492; 131k 371, 770 and 371, 743; above 150k 421, 918 and
+// 426, 905; 387k 1078, 1979 and 1090, 1969.  The line lies where the gain ends for every ion count: above it data passes
+// through the L2s and the MALL from HBM, which is read best in one sweep by all XCDs.
+constexpr size_t kXcdBytes = size_t(512) << 20;
 
 __global__ void k_face_geo(DevMesh d, double *geo);
 __global__ void k_face_entries(DevMesh d, int2 *fent, int8_t *fcls);

@@ -12,7 +12,7 @@
 // measurable (8M tetrahedra: 6181 us per step with the face EMFs in the states' launch, 6200 in one of their own).
 //
 // Measured, microseconds per explicit step, against one kernel per operation with gradients in memory (8 launches; one
-// MI355X): 9.5k tetrahedra 90 -> 36, 60k 113 -> 59, 484k 547 -> 396, 1.95M 1982 -> 1553, 7.83M 7723 -> 6235.  At 7.83M
+// MI355X): 9.5k tetrahedra 90 -> 36, 60k 113 -> 59, 484k 547 -> 400, 1.95M 1982 -> 1547, 7.83M 7723 -> 6196.  At 7.83M
 // prepare takes 623 us (994 before), states 2486 and fluxes 2596 (5660 for the gradients, fluxes, EMF candidates and
 // edge sums before), update 871 (1073).  prepare, the flux half of fluxes and update run at 5.0-5.5 TB/s of their bytes
 // (the streaming copy reaches 6.1); states is bound by its FP64 instructions and the loads' latency at three waves per

@@ -2,12 +2,13 @@
 // lanes per cell stage the cell's edge values in LDS, each lane forms the fluxes of its faces from them (a face's two
 // cells form it twice; one writes it for the edge kernel) and its part of the cell's field.
 //
-// It serves meshes whose tables stay in the caches (DevMesh::xcd_ranges), where a launch and its gap cost more than the
-// faces' fluxes do, and the tables (40 bytes a tetrahedron) are not read from HBM.
+// It serves meshes whose tables stay in the caches (DevMesh::xcd_ranges: up to 457k tetrahedra with two ions), where a launch
+// and its gap cost more than the faces' fluxes do, and the tables (40 bytes a tetrahedron) are not read from HBM.
 //
-// Hall steps, microseconds in FP64 / mixed precision: 9.5k tetrahedra 245 / 228 -> 217 / 199, 60k 396 / 346 -> 373 / 318, 286k
-// 956 / 792 -> 920 / 766, 484k 1715 / 1290 -> 1708 / 1292.  Above, the separate launches are as fast or faster (per product:
-// FP64 at 1.95M 94 us both; FP32 at 7.83M 191 us against 245), so the tables are built below that line only.
+// Hall steps, microseconds in FP64 / mixed precision, without and with it, forced either way: 9.5k tetrahedra 329 / 282 and
+// 298 / 263, 60k 445 / 375 and 422 / 357, 150k 653 / 589 and 641 / 577, 290k 1066 / 911 and 1028 / 897, 435k 1552 / 1269 and 1502 /
+// 1261; above the line 484k 1809 / 1422 and 1812 / 1411, 683k 2616 / 1919 and 2603 / 1934, 1.06M 4564 / 3272 and 4574 / 3354 (per
+// product, FP64 at 1.95M 94 us both; FP32 at 7.83M 191 us against 245), so the tables are built below it only.
 #include <stdexcept>
 #include <string>
 
