@@ -63,8 +63,6 @@ def kernel_bytes(mesh, name, precision_bytes=8, ns=2):
         # phi, star2, e2f, g (3C), ec lists + weights, edge vec, m_e, v, invdiag, dir, out
         "edge_apply": F * b + F * 8 + 4 * (E + 1) + 4 * nf2e + 3 * C * b + 4 * (E + 1) + 12 * nec + 24 * E + 8 * E
                       + 2 * E * b + 8 * E + E + E * b,
-        # one fused MGS step: w read + write, two basis vectors
-        "mgs": 4 * E * b,
         # the explicit stage (csrc/kernels/explicit_step.h): cell records of rs doubles, a state per ion at every (cell, face)
         # entry, a flux per ion and a 32-byte EMF row at every face
         "prepare": ns * 5 * C * 8 + rs * C * 8 + F * 8 + 3 * C * 8 * 4 + C * 8 * 2 + 4 * F * 8 + 4 * nc2f + C,
@@ -97,8 +95,7 @@ KERNEL_CLASSES = {
     "explicit": ("prepare", "dt_final", "states", "fluxes", "update", "faraday", "gyrate"),
     "operator": ("d1", "bcell", "flux_cell", "hall_g", "edge_apply", "d1_f32", "bcell_f32", "flux_cell_f32", "hall_g_f32",
                  "edge_apply_f32", "mg_apply_f32"),
-    "orthogonalisation": ("mgs", "finish", "dot", "multidot", "multidot_final", "multiaxpy", "scale", "multidot64", "multidot64_final",
-                          "multiaxpy64", "norm64"),
+    "orthogonalisation": ("dot", "multidot", "multiaxpy", "multidot64", "multiaxpy64", "mgs_dots", "mgs_axpy", "scale"),
     "multigrid": ("mg_first", "mg_smooth_f32", "mg_resid_f32", "mg_sweep", "mg_resid", "mg_restrict", "mg_prolong", "mg_dinv"),
 }
 

@@ -126,11 +126,13 @@ struct mhdg_ctx
     // coefficients (valid until the next kernel that writes the box) and h_{j+1,j}
     template <class T> const double *arnoldi_cgs(mhdg::Ortho<T> o, double dgks, double &hn)
     {
+        constexpr bool fp64 = sizeof(T) == 8;
+        const char *const dots = fp64 ? "multidot64" : "multidot", *const update = fp64 ? "multiaxpy64" : "multiaxpy";
         o.ticket = ++ticket;
-        prof_begin("multidot");
+        prof_begin(dots);
         mhdg::ortho_dots(o, false, stream);
         prof_end();
-        prof_begin("multiaxpy");
+        prof_begin(update);
         mhdg::ortho_update(o, mhdg::kCgs, dgks, stream);
         prof_end();
         check_launch("arnoldi");
@@ -142,10 +144,10 @@ struct mhdg_ctx
         }
         std::copy(h, h + o.nv, h_first);
         o.ticket = ++ticket;
-        prof_begin("multidot");
+        prof_begin(dots);
         mhdg::ortho_dots(o, false, stream);
         prof_end();
-        prof_begin("multiaxpy");
+        prof_begin(update);
         mhdg::ortho_update(o, mhdg::kPlain, 0.0, stream);
         mhdg::ortho_scale(o, stream);
         prof_end();

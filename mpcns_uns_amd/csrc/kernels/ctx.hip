@@ -209,7 +209,7 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
     };
     cdeg = uniform(t.c2f_ptr);
     fdeg = uniform(t.f2e_ptr);
-    if (c.ind_restart > 60) throw std::runtime_error("ind_restart above 60 is not supported");
+    if (c.ind_restart > kMaxRestart) throw std::runtime_error("ind_restart above 60 is not supported");
     const size_t E = ne, F = nf, C = nc;
     d.nc = nc; d.nf = nf; d.ne = ne;
     d.cdeg = cdeg; d.fdeg = fdeg;
@@ -315,7 +315,7 @@ void mhdg_ctx::build(const mhdg_mesh_desc &m, const mhdg_config &c)
 // ------------------------------------------------------------------------------------ pieces
 void mhdg_ctx::launch_edge_emf(const double *Efp, const double *u, double cuct, const double *Ein, double *Eout, int bc)
 {
-    const size_t lds = n_heavy ? 6 * size_t(max_valence) * sizeof(double) : 0;
+    const size_t lds = n_heavy ? kEmfHeavyRows * size_t(max_valence) * sizeof(double) : 0;
     LAUNCH("edge_emf", k_edge_emf<double>, dim3(n_heavy + nblk(ne)), dim3(256), lds, stream, d, P, Efp, u, cuct, kLightMax, Ein, Eout, bc,
            static_cast<const int32_t *>(heavy), n_heavy, max_valence);
     check_launch("edge emf");
@@ -455,10 +455,10 @@ int mhdg_ctx::solve64(const double *Phi_n, const double *Eex, const int8_t *dir,
             apply_op(nullptr, V[j], invdiag, dir, dt, 1, 1, nullptr, wvec);
             Ortho<double> o = ortho64(j);
             o.ticket = ++ticket;
-            prof_begin("multidot64");
+            prof_begin("mgs_dots");
             ortho_dots(o, true, stream);
             prof_end();
-            prof_begin("multiaxpy64");
+            prof_begin("mgs_axpy");
             ortho_update(o, kMgs, 0.0, stream);
             prof_end();
             prof_begin("scale");

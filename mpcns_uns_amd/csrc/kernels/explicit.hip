@@ -496,7 +496,7 @@ template <class R> __global__ void __launch_bounds__(256) k_cell_update(DevMesh 
 // add_ideal_emf edge loop (Common/induction/IdealEMF.cpp:59-128).  The first n_heavy blocks take one high-valence edge
 // each (they last longest: 30 to 70 us alone behind this kernel before), the others one edge per thread with valence at
 // most `vmax`.  E_out[e] = E_in[e] + E_ideal (E_in nullable = 0); apply_bc additionally applies the boundary EMF of
-// Solver::rhs.  Dynamic LDS: six rows of hv values when there are heavy edges.
+// Solver::rhs.  Dynamic LDS: kEmfHeavyRows rows of hv values when there are heavy edges.
 template <class R> __global__ void __launch_bounds__(256) k_edge_emf(DevMesh d, Params P, const R *Ef, const R *u_cell, double cuct,
                                                   int32_t vmax, const R *E_in, R *E_out, int32_t apply_bc, const int32_t *heavy,
                                                   int32_t n_heavy, int32_t hv)

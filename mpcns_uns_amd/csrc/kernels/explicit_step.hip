@@ -803,7 +803,7 @@ double mhdg_ctx::explicit_stage(const StepRun &x, double dt_max, StageEnd end)
     ++ticket;
     launch_states(x, blocks(nf, kStatesThreads), split ? nullptr : x.dt_dev, dt_max);
     const int n_edge = blocks(ne, kRoleThreads), n_flux = blocks(nf, kRoleThreads / P.ns);
-    const size_t lds = sizeof(double) * std::max<size_t>(5 * kRoleThreads, n_heavy ? 6 * size_t(max_valence) : 0);
+    const size_t lds = sizeof(double) * std::max<size_t>(5 * kRoleThreads, n_heavy ? kEmfHeavyRows * size_t(max_valence) : 0);
     auto kflux = P.ns == 2 ? k_step_fluxes<2> : k_step_fluxes<0>;
     LAUNCH("fluxes", kflux, dim3(n_heavy + n_edge + n_flux), dim3(kRoleThreads), lds, stream, d, P, x.F, x.E, static_cast<const int32_t *>(heavy),
            n_heavy, max_valence, n_edge);

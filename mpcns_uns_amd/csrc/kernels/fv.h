@@ -234,7 +234,7 @@ template <class R> __device__ __forceinline__ V3T<R> emf_of(const R *Ef, int32_t
 }
 
 // One high-valence edge per block (pole axes of a lat-lon net): per-face terms in parallel, every sum sequential in the
-// reference's order.  sh holds eight rows of hv values (hv the largest valence of the mesh).
+// reference's order.  sh holds kEmfHeavyRows rows of hv values (hv the largest valence of the mesh).
 template <class R>
 __device__ __forceinline__ void edge_emf_heavy(const DevMesh &d, const Params &P, const R *Ef, const R *u_cell, double cuct, int32_t e,
                                                const R *E_in, R *E_out, int32_t apply_bc, R *sh, int32_t hv)

@@ -19,7 +19,8 @@ __device__ __forceinline__ int32_t xcd_block(uint32_t nb)
     if (b >= 8 * per) return int32_t(b);
     return int32_t((b % 8) * per + b / 8);
 }
-// LDS rows of a heavy edge: half the valence for the 16-byte Dual
+constexpr int kEmfHeavyRows = 6; // LDS rows of a heavy edge in k_edge_emf and the step's fluxes (edge_emf_heavy), a value per face
+// Their length: half the valence for the 16-byte Dual
 template <class R> constexpr int32_t kHeavyShared() { return sizeof(R) == sizeof(double) ? kHeavyMax : kHeavyMax / 2; }
 
 // explicit.hip: templates on the real type R (double: the step; Dual: its tangent-linear)

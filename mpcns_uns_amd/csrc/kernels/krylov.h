@@ -14,13 +14,14 @@ namespace mhdg
 constexpr int kDotChunk = 16;       // basis vectors per dot-product pass
 constexpr int kOrthoBlocks = 1024;  // largest grid of the vector kernels (512 and 2048 measured no better)
 constexpr int kOrthoThreads = 256;
-// Up to this many blocks of a dot-product pass the update's blocks sum the partials themselves (34 KB of them at most,
-// from the L2) and the launch that sums them, 4 us and its gap on a step of 40 us, goes; with 1024 blocks of partials
+// Up to this many blocks of a dot-product pass the update's blocks sum the partials themselves (1 KB a column from the L2: 17
+// columns for 16 vectors, 121 with the Gram columns of 60) and the launch that sums them, 4 us and its gap on a step of 40 us, goes; with 1024 blocks of partials
 // that would read 280 MB.
 constexpr int kFoldBlocks = 128;
-constexpr int kMaxBasis = 62;       // slots 62 and 63 of a column hold the re-projection flag and <w, w>
+constexpr int kMaxRestart = 60;     // vectors of a cycle: their coefficients, the norm, then slots 62 (re-projection) and 63 (<w, w>)
 // Columns of partial sums: <V_i, w> at i, <w, w> at kColWW, <V_i, V_j> at kColGram + i
 constexpr int kColWW = 63, kColGram = 64, kCols = 128;
+static_assert(kMaxRestart + 1 < 62 && kMaxRestart <= kCols - kColGram, "the coefficients and the norm end before slot 62");
 
 // What a kernel hands to the host (pinned host memory): written, then the ticket.
 struct HostBox

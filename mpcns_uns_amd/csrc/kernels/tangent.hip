@@ -253,7 +253,7 @@ void mhdg_ctx::explicit_tangent(int n_steps, double dt_max, const Params &Pt)
         LAUNCH("cell_update_t", k_cell_update<Dual>, dim3(nb), dim3(256), 0, stream, d, Pt, 2, 0, static_cast<const Dual *>(tw.FA), none,
                Ws, static_cast<const Dual *>(tw.Btot),
                static_cast<const Dual *>(tw.J), static_cast<const Dual *>(tw.dt_dev), 0.0, 1, 1, Us, noneW);
-        LAUNCH("edge_emf_t", k_edge_emf<Dual>, dim3(n_heavy + nbk(ne)), dim3(256), n_heavy ? 6 * size_t(max_valence) * sizeof(Dual) : 0, stream,
+        LAUNCH("edge_emf_t", k_edge_emf<Dual>, dim3(n_heavy + nbk(ne)), dim3(256), n_heavy ? kEmfHeavyRows * size_t(max_valence) * sizeof(Dual) : 0, stream,
                d, Pt, static_cast<const Dual *>(tw.Ef), static_cast<const Dual *>(tw.uplus), Pt.cuct, kLightMax,
                static_cast<const Dual *>(nullptr), tw.E, 1, static_cast<const int32_t *>(heavy), n_heavy, max_valence);
         LAUNCH("faraday_t", k_faraday<Dual>, dim3(nbk(nf)), dim3(256), 0, stream, d, static_cast<const Dual *>(tw.E),

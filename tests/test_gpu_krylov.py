@@ -42,7 +42,14 @@ def test_solves_agree_with_the_oracle(net, scale):
     for precision in (0, 3, 1):
         # each solve from a cold start: the warm start of the one before is dropped with the state
         dev.set_state(*w["state"])
+        dev.profile(None)
+        dev.profile(True)
         got, it, res = dev.ind_solve(w["state"][2], E, dirichlet, dt, precision)
+        dev.profile(False)
+        passes = dev.profile_report()[{0: "mgs_dots", 3: "multidot64", 1: "multidot"}[precision]][0]
+        if scale == 200.0 and net != "box":
+            assert it > 16  # one pass takes 16 vectors, a cycle has up to 40
+        assert passes > it if precision == 3 and scale == 1e-4 else passes >= it  # a second projection is a pass of its own
         # both stop at a residual of 1e-12 |b|, A = I + dt F d1 with dt |F d1| of order `scale`
         assert res <= 1e-12 and maxrel(got, ref) < 1e-10, precision
         if precision == 0:
