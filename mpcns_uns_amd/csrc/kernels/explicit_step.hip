@@ -12,9 +12,9 @@
 // measurable (8M tetrahedra: 6181 us per step with the face EMFs in the states' launch, 6200 in one of their own).
 //
 // Measured, microseconds per explicit step, against one kernel per operation with gradients in memory (8 launches; one
-// MI355X): 9.5k tetrahedra 90 -> 36, 60k 113 -> 59, 484k 547 -> 400, 1.95M 1982 -> 1547, 7.83M 7723 -> 6196.  At 7.83M
-// prepare takes 623 us (994 before), states 2486 and fluxes 2596 (5660 for the gradients, fluxes, EMF candidates and
-// edge sums before), update 871 (1073).  prepare, the flux half of fluxes and update run at 5.0-5.5 TB/s of their bytes
+// MI355X): 9.5k tetrahedra 90 -> 36, 60k 113 -> 58, 484k 547 -> 400, 1.95M 1982 -> 1547, 7.83M 7723 -> 6196.  At 7.83M
+// prepare takes 617 us (994 before), states 2331 and fluxes 2403 (5660 for the gradients, fluxes, EMF candidates and
+// edge sums before), update 846 (1073).  prepare, the flux half of fluxes and update run at 5.0-5.5 TB/s of their bytes
 // (the streaming copy reaches 6.1); states is bound by its FP64 instructions and the loads' latency at three waves per
 // SIMD, the edge half of fluxes by the L1's outstanding requests.  The roles' blocks follow one another: taking them in
 // turn, one or eight each, let the two working sets evict each other (484k: fluxes 153 -> 213 us, states 154 -> 206).
@@ -74,7 +74,8 @@ __global__ void __launch_bounds__(256) k_face_entries(DevMesh d, int2 *fent, int
     }
     fcls[f] = cls;
 }
-// columns [first, first + n) of the cell records as a dense n-per-cell array
+// columns [first, first + n) of the cell records as a dense n-per-cell array, for a getter: one launch ahead of the copy to
+// the host (B_ind of 4k hexahedra 17 us without it, 30 with; of 484k tetrahedra 798 and 804)
 __global__ void __launch_bounds__(256) k_rec_get(const double *rec, int32_t rs, int32_t first, int32_t n, int32_t nc, double *out)
 {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
